@@ -172,7 +172,9 @@ void fft3_refine_adj_c2r(const FftTables& T, const float2* X1, const float2* FP,
                          float* out, hipStream_t s);
 
 int refine_dot_blocks(int N);
-void launch_vol_mean(const float* vols, int count, int N, float* mean, hipStream_t s);
+// mean of each of `count` volumes; `part` holds vol_mean_blocks(N) doubles per volume
+int vol_mean_blocks(int N);
+void launch_vol_mean(const float* vols, int count, int N, double* part, float* mean, hipStream_t s);
 void launch_reslice_ref(const float* ref, const RefineGeom* geom, int E, int N, float* out, hipStream_t s);
 void launch_refine_dot(const float2* X1, const float2* FP, const float* filter, const float* wbin, const RefineGeom* geom,
                        int E, int N, double* part, double* sc, hipStream_t s);

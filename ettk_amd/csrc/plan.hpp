@@ -173,7 +173,7 @@ struct ettk_plan {
     const float* r_fp_parts = nullptr;  // r_fp holds the spectra of particles [r_fp_p0, r_fp_p1) of this array,
     int r_fp_p0 = 0, r_fp_p1 = 0;       // enqueued ahead of the refinement that uses them (refine_spectra_ahead)
     ettk::DevBuf<float> r_mean, r_mpart;
-    ettk::DevBuf<double> r_pdot, r_sc, r_mom;
+    ettk::DevBuf<double> r_pdot, r_sc, r_mom, r_vsum;
     ettk::DevBuf<ettk::RefineGeom> r_geom;
 };
 

@@ -52,7 +52,8 @@ static void particle_spectra(ettk_plan* P, const float* d_parts, int p0, int p1)
     hipStream_t s = P->stream;
     P->r_fp.ensure((size_t)cnt * nh);
     P->r_mean.ensure(cnt);
-    launch_vol_mean(d_parts + (size_t)p0 * n3, cnt, N, P->r_mean.p, s);
+    P->r_vsum.ensure((size_t)cnt * vol_mean_blocks(N));
+    launch_vol_mean(d_parts + (size_t)p0 * n3, cnt, N, P->r_vsum.p, P->r_mean.p, s);
     const int CH = 64;
     for (int c0 = 0; c0 < cnt; c0 += CH) {
         int c = std::min(CH, cnt - c0);
