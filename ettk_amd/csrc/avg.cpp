@@ -8,7 +8,8 @@ namespace ettk {
 EvalGeom make_geom_public(const ettk_plan* P, const ettk_particle& d, const Mat4& t, int particle);
 void launch_avg_acc(const float2* F, const float* w, int E, long nh, double* re, double* im, double* acc, hipStream_t s);
 void launch_avg_final(const double* re, const double* im, const double* acc, int N, float2* F, hipStream_t s);
-void launch_avg_normalise(const float* A, int N, float* out, hipStream_t s);
+int avg_normalise_partials();
+void launch_avg_normalise(const float* A, int N, double* part, float* out, hipStream_t s);
 void launch_var_acc(const float* R, const float* mean, const float* w, int E, double wsum, const float* avg, int N,
                     double* var, hipStream_t s);
 void launch_var_out(const double* var, int N, float* out, hipStream_t s);
@@ -246,7 +247,8 @@ int ettk_avg_finalize(ettk_plan* P, float* d_out) {
         ensure_ccc_workspace(P, 1);
         launch_avg_final(acc_buf(P, 0).p, acc_buf(P, 1).p, acc_buf(P, 2).p, N, P->S1.p, s);
         fft3_c2r(P->ctx->fft, P->S1.p, P->S1.p, P->R1.p, N, 1, s);
-        launch_avg_normalise(P->R1.p, N, d_out, s);
+        P->avg_part.ensure(avg_normalise_partials());
+        launch_avg_normalise(P->R1.p, N, P->avg_part.p, d_out, s);
         ETTK_HIP(hipStreamSynchronize(s));
     } catch (const Error& e) {
         set_error(e.msg);

@@ -154,7 +154,7 @@ struct ettk_plan {
     // S^2 / SO(3) state (so3.hip)
     ettk::So3State* so3 = nullptr;
     // averaging accumulators
-    ettk::DevBuf<double> avg_re, avg_im, avg_acc;
+    ettk::DevBuf<double> avg_re, avg_im, avg_acc, avg_part;
     // continuous refinement (refine.cpp): reference minus its mean (x fastest), its wedge normals, particle
     // spectra and per-evaluation workspace
     ettk::DevBuf<float> ref_x;

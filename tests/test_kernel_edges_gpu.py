@@ -31,3 +31,31 @@ def test_particle_mean_blocks(torch_gpu, ctx, N):
         assert np.abs(s1 - s0).max() < 5e-5
     finally:
         plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [16, 48, 96])
+def test_average_transposed_tiles(torch_gpu, ctx, N):
+    """The average's output tiles: half a 32-wide tile at 16, one and a half at 48, three at 96.  One particle averaged at
+    the identity against the FP64 oracle, whose interpolator moves a sample by the same 2^-17 voxel: the spectrum is
+    divided by the amplitude it was multiplied by, in FP64, so FP32 transforms (2^-24 times their log2(N^3) <= 20
+    levels, forward and back, 3e-6 at most) set the difference, and a factor of 8 is left."""
+    from ettk_amd.abi import Particle, particle_array
+    from ettk_amd.lib import Plan
+    from oracle_lib import OraclePlan, oracle, vp
+
+    g = np.random.default_rng(N)
+    v = g.standard_normal((1, N, N, N)).astype(np.float32)
+    p = default_params(N, 8, mask_radius=N / 2 - 3, square_mask=2)
+    plan, orc = Plan(ctx, p), OraclePlan(p)
+    try:
+        out = torch_gpu.full((N, N, N), 7.0, dtype=torch_gpu.float32, device="cuda")
+        torch_gpu.cuda.synchronize()
+        plan.average(to_dev(torch_gpu, v), [Particle()], [1.0], [np.eye(4)], out)
+        want, one, eye = np.zeros((N, N, N)), np.ones(1, np.float32), np.eye(4).reshape(1, 16)
+        oracle().orc_average(orc.h, 1, vp(v), particle_array([Particle()]), vp(one), vp(eye), vp(want))
+        err = np.abs(out.cpu().numpy() - want).max()
+        print(f"[edges] average N={N} err {err:.2e}", flush=True)
+        assert err < 2.4e-5
+    finally:
+        plan.close()
