@@ -14,6 +14,7 @@
 #include "kernels.hpp"
 
 #include <hip/hip_ext.h>
+#include "tricubic.hpp"
 #include "wedge.hpp"
 
 #include <algorithm>
@@ -41,14 +42,6 @@ __device__ __forceinline__ float block_sum(float v, float* sh) {
 }
 
 // ------------------------------------------------------------------ reslice
-__device__ __forceinline__ void keys_w(float f, float* w) {  // vtkTricubicInterpWeights
-    float fm1 = f - 1.f, fd2 = f * 0.5f, ft3 = f * 3.f;
-    w[0] = -fd2 * fm1 * fm1;
-    w[1] = ((ft3 - 2.f) * fd2 - 1.f) * fm1;
-    w[2] = -((ft3 - 4.f) * f - 1.f) * fd2;
-    w[3] = f * fd2 * fm1;
-}
-
 // Validity of a sample is decided in FP32 unless it lies within 1e-3 of the border, where the FP64 map decides
 // (the reference places samples in FP64: a sample that FP32 rounding moves across the border would otherwise
 // enter or leave the valid set and change the mean the volume is centred on).
@@ -63,22 +56,14 @@ __device__ __forceinline__ bool inside_fp64(const double* md, int i, int j, int 
     return x >= lo && x <= hx && y >= lo && y <= hy && z >= lo && z <= hz;
 }
 
-// One workgroup reslices an 8x8x8 tile of the output.  The input voxels its 64-tap stencils can touch lie in
-// the bounding box of the tile's transformed corners: at most floor(7 sqrt 3) + 1 + 4 = 17 voxels per axis for
-// a rigid map.  That box (its actual extent, about 14 voxels per axis for a random rotation), with the volume's
-// border replicated where it reaches outside (the taps clamp to the border), is staged in LDS at fixed strides,
-// so every tap is a plain LDS read and the 4 taps of a row are consecutive words.  A non-rigid map whose box does
-// not fit reads the clamped taps from global memory instead.
-// Each wavefront interpolates a 4x4x4 block of the tile: the taps of its voxels then cover a compact region
-// of the box and, with the row and plane strides 17 and 300, fall on fewer common LDS banks than those of an
-// 8x8 plane.  A 17^3 box at these strides (20 KB) lets 8 workgroups share a CU's 160 KB of LDS.
+// One workgroup reslices an 8x8x8 tile of the output from the LDS-staged box of the particle (tricubic.hpp).
 // Measured on 256 evaluations at 64^3 (one launch): 654 us, against 775 us for an 18^3 box at strides 19/343,
 // 8x8 planes per wavefront and two reductions; outputs bit-identical.
-static constexpr int kTile = 8, kBox = 17, kSY = 17, kSZ = 300;
 // kUse names the caller in kernel traces (0: CCC evaluations, 1: S^2 projection); the code is the same
 template <int kUse>
 __global__ void __launch_bounds__(kThreads) k_reslice(const float* __restrict__ parts, const EvalGeom* __restrict__ geom,
                                                        int N, float* __restrict__ out, float* __restrict__ partials) {
+    static_assert(kThreads == kTriThreads, "the staging's thread map");
     __shared__ float2 sh[kThreads / 64];
     __shared__ float box[kBox * kSZ];
     int e, tb;
@@ -89,48 +74,18 @@ __global__ void __launch_bounds__(kThreads) k_reslice(const float* __restrict__ 
     const int nt = N / kTile;
     const int ti = tb / (nt * nt), tj = (tb / nt) % nt, tk = tb % nt;
     const int i0 = ti * kTile, j0 = tj * kTile, k0 = tk * kTile;
-    const float tol = 7.62939453125e-06f;
-    // staged box [lo, hi] per input axis (x, y, z); it may reach outside the volume
     int lo[3], hi[3];
-    bool fits = true;
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        float c0 = g.m[a] * i0 + g.m[3 + a] * j0 + g.m[6 + a] * k0 + g.m[9 + a];
-        float ext = (kTile - 1) * (fabsf(g.m[a]) + fabsf(g.m[3 + a]) + fabsf(g.m[6 + a]));
-        float mn = c0 + (kTile - 1) * (fminf(g.m[a], 0.f) + fminf(g.m[3 + a], 0.f) + fminf(g.m[6 + a], 0.f));
-        lo[a] = (int)floorf(mn + tol) - 1;
-        hi[a] = (int)floorf(mn + ext + tol) + 2;
-        if (!(hi[a] - lo[a] + 1 <= kBox) || !(fabsf(mn) < 1e6f)) fits = false;
-    }
-    if (fits) {
-        // 2-D thread map over (y, x) of the box, loop over z; coordinates clamped to the volume
-        constexpr int kRows = kThreads / kBox;
-        const int t = threadIdx.x;
-        const int wx = hi[0] - lo[0] + 1, wy = hi[1] - lo[1] + 1, wz = hi[2] - lo[2] + 1;
-        const int x = t % kBox, y0 = t / kBox;
-        if (t < kBox * kRows && x < wx) {
-            const int gx = min(max(lo[0] + x, 0), N - 1);
-            for (int y = y0; y < wy; y += kRows) {
-                const int gy = min(max(lo[1] + y, 0), N - 1);
-                const float* src = vol + (size_t)gy * N + gx;
-#pragma unroll 6
-                for (int z = 0; z < wz; z++) {
-                    const int gz = min(max(lo[2] + z, 0), N - 1);
-                    box[z * kSZ + y * kSY + x] = src[(size_t)gz * N * N];
-                }
-            }
-        }
-    }
+    const bool fits = tile_box(g.m, i0, j0, k0, lo, hi);
+    if (fits) stage_tile_box(vol, N, N, N, lo, hi, box);
     __syncthreads();
     float s = 0.f, c = 0.f;
     const float lob = -0.5f, hib = (float)N - 0.5f;
     for (int t = threadIdx.x; t < kTile * kTile * kTile; t += blockDim.x) {
-        // t >> 6 numbers the tile's eight 4x4x4 blocks (two passes of four wavefronts), l = t & 63 the voxel
-        // within its block
-        const int sb = t >> 6, l = t & 63;
-        const int i = i0 + 4 * (sb >> 2) + (l >> 4);
-        const int j = j0 + 4 * ((sb >> 1) & 1) + ((l >> 2) & 3);
-        const int k = k0 + 4 * (sb & 1) + (l & 3);
+        int i, j, k;
+        tile_voxel(t, i, j, k);
+        i += i0;
+        j += j0;
+        k += k0;
         float px = g.m[0] * i + g.m[3] * j + g.m[6] * k + g.m[9];
         float py = g.m[1] * i + g.m[4] * j + g.m[7] * k + g.m[10];
         float pz = g.m[2] * i + g.m[5] * j + g.m[8] * k + g.m[11];
@@ -139,53 +94,7 @@ __global__ void __launch_bounds__(kThreads) k_reslice(const float* __restrict__ 
         if (near_border(px, lob, hib) || near_border(py, lob, hib) || near_border(pz, lob, hib))
             in = inside_fp64(g.md, i, j, k, -0.5, N - 0.5, N - 0.5, N - 0.5);
         if (in) {
-            float xx = px + tol, yy = py + tol, zz = pz + tol;
-            int ix = (int)floorf(xx), iy = (int)floorf(yy), iz = (int)floorf(zz);
-            if (fits) {
-                // the box was sized from the tile's corners; a sample within rounding of a voxel boundary can
-                // floor one voxel outside it: take the neighbouring cubic piece at f just outside [0, 1) instead
-                // (the Keys kernel is C1, the value agrees to O(f^2) of a few ulps)
-                ix = min(max(ix, lo[0] + 1), hi[0] - 2);
-                iy = min(max(iy, lo[1] + 1), hi[1] - 2);
-                iz = min(max(iz, lo[2] + 1), hi[2] - 2);
-            }
-            float wx[4], wy[4], wz[4];
-            keys_w(xx - ix, wx);
-            keys_w(yy - iy, wy);
-            keys_w(zz - iz, wz);
-            float acc = 0.f;
-            if (fits) {
-                const float* b0 = box + (iz - 1 - lo[2]) * kSZ + (iy - 1 - lo[1]) * kSY + (ix - 1 - lo[0]);
-#pragma unroll
-                for (int a = 0; a < 4; a++) {
-                    float ay = 0.f;
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                        const float* row = b0 + a * kSZ + b * kSY;
-                        ay += wy[b] * (wx[0] * row[0] + wx[1] * row[1] + wx[2] * row[2] + wx[3] * row[3]);
-                    }
-                    acc += wz[a] * ay;
-                }
-            } else {
-                int cx[4], cy[4], cz[4];
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    cx[q] = min(max(ix - 1 + q, 0), N - 1);
-                    cy[q] = min(max(iy - 1 + q, 0), N - 1);
-                    cz[q] = min(max(iz - 1 + q, 0), N - 1);
-                }
-#pragma unroll
-                for (int a = 0; a < 4; a++) {
-                    float ay = 0.f;
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                        const float* row = vol + ((size_t)cz[a] * N + cy[b]) * N;
-                        ay += wy[b] * (wx[0] * row[cx[0]] + wx[1] * row[cx[1]] + wx[2] * row[cx[2]] + wx[3] * row[cx[3]]);
-                    }
-                    acc += wz[a] * ay;
-                }
-            }
-            v = acc;
+            v = fits ? sample_box(box, lo, hi, px, py, pz) : sample_global(vol, N, N, N, px, py, pz);
             s += v;
             c += 1.f;
         }

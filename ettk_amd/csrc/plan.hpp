@@ -5,6 +5,7 @@
 #include <cstring>
 #include <functional>
 #include <memory>
+#include <mutex>
 
 #include "kernels.hpp"
 
@@ -90,6 +91,11 @@ struct CccGraph {
     int gen = -1;
     hipGraphExec_t exec = nullptr;
 };
+// geometry of one extracted box (extract.hip)
+struct ExtractGeom {
+    float m[12];    // input index = m[0..2] x + m[3..5] y + m[6..8] z + m[9..11]  (rows x, y, z)
+    double md[12];  // the same map in FP64: decides validity for samples within FP32 rounding of the border
+};
 struct Timing {
     double ccc_ms = 0, total_ms = 0;
     long long n_ccc = 0;
@@ -104,6 +110,11 @@ struct ettk_ctx {
     ettk::FftTables fft;
     void* scratch = nullptr;  // device address of this device's fixed CCC scratch region (noalloc.hip)
     struct ettk_plan_cache* plans = nullptr;  // plans kept for ettk_align_buckets (tune.cpp)
+    // ettk_extract_batch: geometry, per-tile sums and means, kept between calls (allocations and frees wait for the
+    // device)
+    std::mutex extract_mu;
+    ettk::DevBuf<ettk::ExtractGeom> extract_geom;
+    ettk::DevBuf<float> extract_part, extract_mean;
 };
 
 struct ettk_plan {

@@ -59,3 +59,36 @@ def test_average_transposed_tiles(torch_gpu, ctx, N):
         assert err < 2.4e-5
     finally:
         plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,scale", [(1, 1.0), (7, 1.0), (8, 1.0), (17, 1.0), (33, 1.0), (20, 1.7)])
+def test_extract_tiles(torch_gpu, ctx, N, scale):
+    """Extraction by 8^3 tiles: boxes smaller than a tile, exactly one, one voxel more than two or four, and a map that
+    magnifies 1.7 times, whose input box exceeds the staged one.  Positions in FP32 (coordinates below 128: 7.6e-6 per
+    operation) move a sample by about 1e-5 voxels, times a gradient of at most 1 / 1.5 of the maximum per voxel of a
+    volume smoothed by 1.5 voxels, along three axes: 2e-5 of the maximum."""
+    from scipy import ndimage
+
+    from ettk_amd.abi import Particle
+    from ettk_amd.synth import random_rotation
+    from oracle_lib import extract
+
+    g = np.random.default_rng(N)
+    tomo = ndimage.gaussian_filter(g.standard_normal((64, 80, 96)), 1.5).astype(np.float32)
+    n = 9
+    pos = np.stack([g.uniform(0, 95, n), g.uniform(0, 79, n), g.uniform(0, 63, n)], 1)
+    descs = []
+    for _ in range(n):
+        t = np.eye(4)
+        t[:3, :3] = random_rotation(g) * scale
+        descs.append(Particle(matrix=t, normal=tuple(g.uniform(-40, 40, 3)), cut_offset=float(g.uniform(-1, 1))))
+    out = torch_gpu.full((n, N, N, N), 9.0, dtype=torch_gpu.float32, device="cuda")
+    torch_gpu.cuda.synchronize()
+    ctx.extract(to_dev(torch_gpu, tomo), pos, descs, N, out)
+    got, want = out.cpu().numpy(), extract(tomo, pos, descs, N)
+    both = (got != 0) & (want != 0)
+    print(f"[edges] extract N={N} x{scale}: {both.sum()} valid voxels", flush=True)
+    assert np.count_nonzero((got != 0) != (want != 0)) <= 0.0005 * n * N ** 3
+    if both.any():
+        assert np.abs(got - want)[both].max() <= 2e-5 * np.abs(tomo).max()
