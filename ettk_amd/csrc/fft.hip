@@ -7,6 +7,7 @@
 //   r2c: pass k (pairs of real rows packed as one complex row, split after the transform), pass j, pass i
 //   c2r: pass i, pass j (complex, backward), then pass k (pairs of half rows -> two real rows)
 #include "kernels.hpp"
+#include "regfft.hpp"
 #include "wedge.hpp"
 
 #include <cfloat>
@@ -36,17 +37,6 @@ void fft_tables_init(FftTables& T, hipStream_t s) {
     ETTK_HIP(hipStreamSynchronize(s));
 }
 
-// ------------------------------------------------------------------ compile-time radix plans
-template <int L> struct Radices;
-template <> struct Radices<16>  { static constexpr int n = 2; static constexpr int r[4] = {4, 4, 1, 1}; };
-template <> struct Radices<32>  { static constexpr int n = 3; static constexpr int r[4] = {4, 4, 2, 1}; };
-template <> struct Radices<48>  { static constexpr int n = 3; static constexpr int r[4] = {4, 4, 3, 1}; };
-template <> struct Radices<64>  { static constexpr int n = 3; static constexpr int r[4] = {4, 4, 4, 1}; };
-template <> struct Radices<96>  { static constexpr int n = 4; static constexpr int r[4] = {4, 4, 3, 2}; };
-template <> struct Radices<128> { static constexpr int n = 4; static constexpr int r[4] = {4, 4, 4, 2}; };
-template <> struct Radices<192> { static constexpr int n = 4; static constexpr int r[4] = {4, 4, 4, 3}; };
-template <> struct Radices<256> { static constexpr int n = 4; static constexpr int r[4] = {4, 4, 4, 4}; };
-
 template <int L> struct Shape {
     static constexpr int TPP = L / 4;                       // threads per pencil
     static constexpr int P = (1024 / L) > 0 ? 1024 / L : 1; // pencils per workgroup
@@ -54,36 +44,6 @@ template <int L> struct Shape {
     static constexpr int LD = L + 1;                        // padded LDS row
     static_assert(THREADS >= L, "one twiddle per thread");
 };
-
-__device__ __forceinline__ float2 mul_i(float2 z, bool inv) {  // forward: -i z, inverse: +i z
-    return inv ? make_float2(-z.y, z.x) : make_float2(z.y, -z.x);
-}
-
-template <int R>
-__device__ __forceinline__ void butterfly(float2* x, bool inv) {
-    if constexpr (R == 2) {
-        float2 a = x[0], b = x[1];
-        x[0] = cadd(a, b);
-        x[1] = csub(a, b);
-    } else if constexpr (R == 3) {
-        const float s = inv ? 0.86602540378443864676f : -0.86602540378443864676f;
-        float2 t1 = cadd(x[1], x[2]);
-        float2 t2 = make_float2(x[0].x - 0.5f * t1.x, x[0].y - 0.5f * t1.y);
-        float2 d = csub(x[1], x[2]);
-        float2 id = make_float2(-s * d.y, s * d.x);  // i*s*d
-        x[0] = cadd(x[0], t1);
-        x[1] = cadd(t2, id);
-        x[2] = csub(t2, id);
-    } else if constexpr (R == 4) {
-        float2 a = cadd(x[0], x[2]), b = csub(x[0], x[2]);
-        float2 c = cadd(x[1], x[3]), d = csub(x[1], x[3]);
-        float2 md = mul_i(d, inv);  // forward: -i d
-        x[0] = cadd(a, c);
-        x[2] = csub(a, c);
-        x[1] = cadd(b, md);
-        x[3] = csub(b, md);
-    }
-}
 
 template <int L, int R>
 __device__ __forceinline__ void stockham_stage(float2* pen, int lane, int Ns, const float2* tw, bool inv) {
@@ -146,31 +106,6 @@ __device__ __forceinline__ void lds_fft(float2* pen, int lane, const float2* tw,
 // 64 = 8 x 8 Cooley-Tukey: each of 8 threads holds x[t + 8m] (m = 0..7), runs an 8-point DFT in registers,
 // applies W64^(t k1), and the 8 x 8 block is transposed through the pencil's own LDS row; an 8-point DFT per
 // thread finishes X[k1 + 8 k2].  One LDS exchange instead of three radix-4 stages.
-__device__ __forceinline__ float2 mul_w8(float2 z, int n, bool inv) {  // z * exp(-+2 pi i n / 8), n = 1..3
-    const float r = 0.70710678118654752440f;
-    switch (n) {
-        case 1: return inv ? make_float2(r * (z.x - z.y), r * (z.x + z.y)) : make_float2(r * (z.x + z.y), r * (z.y - z.x));
-        case 2: return mul_i(z, inv);
-        default: return inv ? make_float2(-r * (z.x + z.y), r * (z.x - z.y)) : make_float2(r * (z.y - z.x), -r * (z.x + z.y));
-    }
-}
-// in place, natural order in and out: a[k] = sum_n a[n] exp(-+2 pi i n k / 8)
-__device__ __forceinline__ void dft8(float2* a, bool inv) {
-    float2 b0 = cadd(a[0], a[4]), b4 = csub(a[0], a[4]);
-    float2 b1 = cadd(a[1], a[5]), b5 = mul_w8(csub(a[1], a[5]), 1, inv);
-    float2 b2 = cadd(a[2], a[6]), b6 = mul_i(csub(a[2], a[6]), inv);
-    float2 b3 = cadd(a[3], a[7]), b7 = mul_w8(csub(a[3], a[7]), 3, inv);
-    float2 c0 = cadd(b0, b2), c2 = csub(b0, b2), c1 = cadd(b1, b3), c3 = mul_i(csub(b1, b3), inv);
-    float2 c4 = cadd(b4, b6), c6 = csub(b4, b6), c5 = cadd(b5, b7), c7 = mul_i(csub(b5, b7), inv);
-    a[0] = cadd(c0, c1);
-    a[4] = csub(c0, c1);
-    a[2] = cadd(c2, c3);
-    a[6] = csub(c2, c3);
-    a[1] = cadd(c4, c5);
-    a[5] = csub(c4, c5);
-    a[3] = cadd(c6, c7);
-    a[7] = csub(c6, c7);
-}
 // the twiddles a thread of a length-64 pencil applies, w[k] = exp(-2 pi i lane k / 64), held in registers
 // for all the pencil transforms of a kernel (length 64 only; other lengths read the LDS table)
 template <int L> struct TwCache {
@@ -361,6 +296,29 @@ __global__ void __launch_bounds__(StridedShape<L>::THREADS) k_fft_strided(Stride
         for (int u = 0; u < NL; u++) a.out[base + (long)(l0 + u * STEP) * a.es] = lds[qm * S::LD + l0 + u * STEP];
 }
 
+// Pencils in registers (regfft.hpp): loads and stores in rows of P consecutive pencils, one LDS exchange.  Bound by HBM.
+template <int L, bool INV>
+__global__ void __launch_bounds__(ColShape<L>::THREADS) k_fft_col(StridedArgs a, const float2* __restrict__ twg) {
+    using S = ColShape<L>;
+    __shared__ float2 ex[L * S::P];
+    __shared__ float2 tw[L];
+    // consecutive pencil groups on one XCD: a group's rows share cache lines with the neighbouring groups' where the
+    // rows are not aligned to them
+    const long pen = (long)xcd_tile(blockIdx.x, gridDim.x) * S::P + threadIdx.x % S::P;
+    const int t = threadIdx.x / S::P;
+    const bool valid = pen < a.npencils;  // an invalid pencil transforms pencil 0 and stores nothing
+    const long base = valid ? (pen / a.inner) * a.outer_stride + (pen % a.inner) : 0;
+    float2 x[S::E];
+#pragma unroll
+    for (int j = 0; j < S::E; j++) x[j] = a.in[base + (long)(t + j * S::T) * a.es];
+    for (int q = threadIdx.x; q < L; q += S::THREADS) tw[q] = twg[q];
+    __syncthreads();
+    col_fft<L, INV>(x, t, ex + threadIdx.x % S::P, tw);
+    if (valid)
+#pragma unroll
+        for (int j = 0; j < S::E; j++) a.out[base + (long)(t + j * S::T) * a.es] = x[j];
+}
+
 // ------------------------------------------------------------------ CCC spectra: one pass along i (L <= 64)
 // deterministic sum over the NT threads of a workgroup (NT need not be a multiple of 64), valid in thread 0
 template <int NT>
@@ -390,92 +348,80 @@ __device__ __forceinline__ float block_sum_nt(float v, float* sred) {
 //   per-block partials of sum hw |X1|^2, sum fw, sum hw |X2|^2 (hw = 2 off the last half plane)
 // The element-wise arithmetic is that of k_spec_filter2 (nbfFourierFilter::executeHalf, FFilt.h:587-606, and
 // normalizeFourierHalf, CorrMetric.h:498-530); the transforms are those of the separate i passes.
+// Each thread keeps its E elements of a pencil in registers through the three transforms (regfft.hpp).
 template <int L>
-__global__ void __launch_bounds__(StridedShape<L>::THREADS) k_ccc_ipass(CccIpassArgs a, const float2* __restrict__ twg) {
-    using S = StridedShape<L>;
-    constexpr int H = L / 2 + 1, LH = L * H, STEP = S::THREADS / S::P, NL = L / STEP;
-    static_assert(L % STEP == 0, "pencil elements per thread");
-    __shared__ float2 lds[S::P * S::LD];
+__global__ void __launch_bounds__(ColShape<L>::THREADS) k_ccc_ipass(CccIpassArgs a, const float2* __restrict__ twg) {
+    using S = ColShape<L>;
+    constexpr int H = L / 2 + 1, LH = L * H, NE = S::E;
+    __shared__ float2 ex[L * S::P];
     __shared__ float2 tw[L];
-    __shared__ float sred[S::THREADS / 64 + S::THREADS % 64 + 1];
+    __shared__ float sred[S::THREADS / 64 + 1];
     const int e = blockIdx.y;
-    const float2 twv = twg[threadIdx.x % L];
-    const int qm = threadIdx.x % S::P, l0 = threadIdx.x / S::P;
-    const int p = blockIdx.x * S::P + qm;  // pencil (j, k) = (p / H, p % H) of evaluation e
+    const int t = threadIdx.x / S::P;
+    const int p = blockIdx.x * S::P + threadIdx.x % S::P;  // pencil (j, k) = (p / H, p % H) of evaluation e
     const bool valid = p < LH;
     const int pc = valid ? p : 0, pj = pc / H, pk = pc % H;
     const size_t vol = (size_t)e * L * LH;
-    float2* __restrict__ pen = &lds[qm * S::LD];
-    {
-        float2 v[NL];
+    float2* __restrict__ xp = ex + threadIdx.x % S::P;
+    float2 x[NE];
 #pragma unroll
-        for (int u = 0; u < NL; u++) v[u] = ld_stream(&a.S2[vol + (size_t)(l0 + u * STEP) * LH + pc]);
-#pragma unroll
-        for (int u = 0; u < NL; u++) pen[l0 + u * STEP] = valid ? v[u] : make_float2(0.f, 0.f);
-    }
-    if (threadIdx.x < L) tw[threadIdx.x] = twv;
+    for (int u = 0; u < NE; u++) x[u] = ld_stream(&a.S2[vol + (size_t)(t + u * S::T) * LH + pc]);
+    for (int q = threadIdx.x; q < L; q += S::THREADS) tw[q] = twg[q];
     __syncthreads();
-    const int q = threadIdx.x / S::TPP, lane = threadIdx.x % S::TPP;
-    const TwCache<L> twc = tw_cache<L>(tw, lane);
-    pencil_fft<L>(&lds[q * S::LD], lane, tw, twc, false);
-    // filter weights of this thread's elements (i = l0 + u STEP of pencil p), the particle side in place
+    col_fft<L, false>(x, t, xp, tw);
+    // filter weights of this thread's elements (i = t + u T of pencil p), the particle side in place
     const EvalGeom& g = a.geom[e];
     const int dc_i = L / 2, dc_j = L / 2, dc_k = H - 1;
     const float hw = pk < H - 1 ? 2.f : 1.f;
-    float fw[NL], flt[NL], w1[NL];
-#pragma unroll
-    for (int u = 0; u < NL; u++) {
-        const size_t h = (size_t)(l0 + u * STEP) * LH + pc;
-        flt[u] = a.filter[h];
-        w1[u] = a.W1 ? a.W1[h] : 1.f;
-    }
+    float fw[NE], w1[NE];
     float s2 = 0.f, swf = 0.f;
 #pragma unroll
-    for (int u = 0; u < NL; u++) {
-        const int i = l0 + u * STEP;
-        float w = w1[u];
-        if (!g.full) w *= wedge_smooth(g.v1, g.v2, i, pj, pk, L, H);
-        fw[u] = flt[u] * w;
-        const bool dc = i == dc_i && pj == dc_j && pk == dc_k;
-        float2 z = pen[i];
+    for (int u = 0; u < NE; u++) {
+        const size_t h = (size_t)(t + u * S::T) * LH + pc;
+        fw[u] = a.filter[h];
+        w1[u] = a.W1 ? a.W1[h] : 1.f;
+    }
+#pragma unroll
+    for (int u = 0; u < NE; u++) {
+        const int i = t + u * S::T;
+        fw[u] *= g.full ? w1[u] : w1[u] * wedge_smooth(g.v1, g.v2, i, pj, pk, L, H);
+        float2 z = x[u];
         if (a.mcf) {
             const float m2 = z.x * z.x + z.y * z.y;
             const float C = sqrtf(sqrtf(m2));
             if (C > 0.f) z = make_float2(z.x / C, z.y / C);
         }
         if (a.apply) z = cscale(z, fw[u]);
-        if (dc) z = make_float2(0.f, 0.f);
+        if (i == dc_i && pj == dc_j && pk == dc_k) z = make_float2(0.f, 0.f);
         if (valid) {
             st_stream(&a.S2[vol + (size_t)i * LH + pc], z);
             s2 += hw * (z.x * z.x + z.y * z.y);
             swf += fw[u];
         }
-        pen[i] = z;
+        x[u] = z;
     }
-    __syncthreads();
-    pencil_fft<L>(&lds[q * S::LD], lane, tw, twc, true);
+    col_fft<L, true>(x, t, xp, tw);
     // reference side: its spectrum loads are issued before the particle side's inverse transform is stored
-    float2 f1[NL];
+    float2 f1[NE];
 #pragma unroll
-    for (int u = 0; u < NL; u++) f1[u] = a.F1mcf[(size_t)(l0 + u * STEP) * LH + pc];
+    for (int u = 0; u < NE; u++) f1[u] = a.F1mcf[(size_t)(t + u * S::T) * LH + pc];
     if (valid)
 #pragma unroll
-        for (int u = 0; u < NL; u++) st_stream(&a.S3[vol + (size_t)(l0 + u * STEP) * LH + pc], pen[l0 + u * STEP]);
+        for (int u = 0; u < NE; u++) st_stream(&a.S3[vol + (size_t)(t + u * S::T) * LH + pc], x[u]);
     float s1 = 0.f;
 #pragma unroll
-    for (int u = 0; u < NL; u++) {
-        const int i = l0 + u * STEP;
+    for (int u = 0; u < NE; u++) {
+        const int i = t + u * S::T;
         float2 z = f1[u];
         if (a.apply) z = cscale(z, fw[u]);
         if (i == dc_i && pj == dc_j && pk == dc_k) z = make_float2(0.f, 0.f);
         if (valid) s1 += hw * (z.x * z.x + z.y * z.y);
-        pen[i] = z;
+        x[u] = z;
     }
-    __syncthreads();
-    pencil_fft<L>(&lds[q * S::LD], lane, tw, twc, true);
+    col_fft<L, true>(x, t, xp, tw);
     if (valid)
 #pragma unroll
-        for (int u = 0; u < NL; u++) st_stream(&a.S1[vol + (size_t)(l0 + u * STEP) * LH + pc], pen[l0 + u * STEP]);
+        for (int u = 0; u < NE; u++) st_stream(&a.S1[vol + (size_t)(t + u * S::T) * LH + pc], x[u]);
     const float t1 = block_sum_nt<S::THREADS>(s1, sred);
     const float tf = block_sum_nt<S::THREADS>(swf, sred);
     const float t2 = block_sum_nt<S::THREADS>(s2, sred);
@@ -1045,6 +991,19 @@ static const char* prof_name(int which) {
 }
 
 template <int L>
+static void launch_strided(const StridedArgs& a, const float2* tw, hipStream_t s) {
+    if constexpr (L <= 64) {
+        using S = StridedShape<L>;
+        k_fft_strided<L><<<(unsigned)((a.npencils + S::P - 1) / S::P), S::THREADS, 0, s>>>(a, tw);
+    } else {
+        using S = ColShape<L>;
+        const unsigned nb = (unsigned)((a.npencils + S::P - 1) / S::P);
+        if (a.inv) k_fft_col<L, true><<<nb, S::THREADS, 0, s>>>(a, tw);
+        else k_fft_col<L, false><<<nb, S::THREADS, 0, s>>>(a, tw);
+    }
+}
+
+template <int L>
 static void launch_r2c(const FftTables& T, const R2CArgs& a, float2* scratch, hipStream_t s) {
     using S = Shape<L>;
     constexpr int H = L / 2 + 1;
@@ -1067,14 +1026,14 @@ static void launch_r2c(const FftTables& T, const R2CArgs& a, float2* scratch, hi
         StridedArgs sj{a.out, a.out, (long)a.batch * L * H, (long)H, (long)L * H, (long)H, 0};
         {
             ProfScope ps(T.prof, prof_name<L>(1), 2 * vol_c, s);
-            k_fft_strided<L><<<(unsigned)((sj.npencils + StridedShape<L>::P - 1) / StridedShape<L>::P), StridedShape<L>::THREADS, 0, s>>>(sj, tw);
+            launch_strided<L>(sj, tw, s);
         }
     }
     // pass i: pencils over (b, j, k), element stride L*H
     StridedArgs si{a.out, a.out, (long)a.batch * L * H, (long)L * H, (long)L * L * H, (long)L * H, 0};
     {
         ProfScope ps(T.prof, prof_name<L>(1), 2 * vol_c, s);
-        k_fft_strided<L><<<(unsigned)((si.npencils + StridedShape<L>::P - 1) / StridedShape<L>::P), StridedShape<L>::THREADS, 0, s>>>(si, tw);
+        launch_strided<L>(si, tw, s);
     }
     (void)scratch;
 }
@@ -1088,7 +1047,7 @@ static void launch_c2r(const FftTables& T, const float2* in, float2* tmp, float*
     StridedArgs si{in, tmp, (long)batch * L * H, (long)L * H, (long)L * L * H, (long)L * H, 1};
     {
         ProfScope ps(T.prof, prof_name<L>(1), 2 * vol_c, s);
-        k_fft_strided<L><<<(unsigned)((si.npencils + StridedShape<L>::P - 1) / StridedShape<L>::P), StridedShape<L>::THREADS, 0, s>>>(si, tw);
+        launch_strided<L>(si, tw, s);
     }
     if constexpr (L <= 64) {
         ProfScope ps(T.prof, plane_name<L>(1), vol_c + vol_r, s);
@@ -1097,7 +1056,7 @@ static void launch_c2r(const FftTables& T, const float2* in, float2* tmp, float*
         StridedArgs sj{tmp, tmp, (long)batch * L * H, (long)H, (long)L * H, (long)H, 1};
         {
             ProfScope ps(T.prof, prof_name<L>(1), 2 * vol_c, s);
-            k_fft_strided<L><<<(unsigned)((sj.npencils + StridedShape<L>::P - 1) / StridedShape<L>::P), StridedShape<L>::THREADS, 0, s>>>(sj, tw);
+            launch_strided<L>(sj, tw, s);
         }
         long npairs = (long)batch * L * L / 2;
         {
@@ -1116,7 +1075,7 @@ static void launch_c2r_op_r2c(const FftTables& T, const float2* in, float2* io, 
     StridedArgs si{in, io, (long)batch * L * H, (long)L * H, (long)L * L * H, (long)L * H, 1};
     if (in) {
         ProfScope ps(T.prof, prof_name<L>(1), 2 * vol_c, s);
-        k_fft_strided<L><<<(unsigned)((si.npencils + StridedShape<L>::P - 1) / StridedShape<L>::P), StridedShape<L>::THREADS, 0, s>>>(si, tw);
+        launch_strided<L>(si, tw, s);
     }
     {
         static const std::string name = "k_c2r_r2c_plane<" + std::to_string(L) + ">";
@@ -1126,7 +1085,7 @@ static void launch_c2r_op_r2c(const FftTables& T, const float2* in, float2* io, 
     StridedArgs sf{io, io, (long)batch * L * H, (long)L * H, (long)L * L * H, (long)L * H, 0};
     if (fwd_i) {
         ProfScope ps(T.prof, prof_name<L>(1), 2 * vol_c, s);
-        k_fft_strided<L><<<(unsigned)((sf.npencils + StridedShape<L>::P - 1) / StridedShape<L>::P), StridedShape<L>::THREADS, 0, s>>>(sf, tw);
+        launch_strided<L>(sf, tw, s);
     }
 }
 
@@ -1157,7 +1116,7 @@ void launch_combine_fftA(const FftTables& T, const float2* F1m, const float2* F2
 
 template <int L>
 static int ccc_ipass_blocks_t() {
-    return (L * (L / 2 + 1) + StridedShape<L>::P - 1) / StridedShape<L>::P;
+    return (L * (L / 2 + 1) + ColShape<L>::P - 1) / ColShape<L>::P;
 }
 int fft3_ccc_ipass_blocks(int n) {
     switch (n) {
@@ -1176,7 +1135,7 @@ static void launch_ccc_ipass(const FftTables& T, const CccIpassArgs& a, int batc
     const double vol_c = (double)batch * L * L * H * sizeof(float2);
     static const std::string name = "k_ccc_ipass<" + std::to_string(L) + ">";
     ProfScope ps(T.prof, name.c_str(), 4 * vol_c, s);  // S2 read and written, S3 and S1 written
-    k_ccc_ipass<L><<<dim3((unsigned)ccc_ipass_blocks_t<L>(), (unsigned)batch), StridedShape<L>::THREADS, 0, s>>>(a, tw);
+    k_ccc_ipass<L><<<dim3((unsigned)ccc_ipass_blocks_t<L>(), (unsigned)batch), ColShape<L>::THREADS, 0, s>>>(a, tw);
 }
 void fft3_ccc_ipass(const FftTables& T, const CccIpassArgs& a, int n, int batch, hipStream_t s) {
     switch (n) {
@@ -1329,11 +1288,15 @@ __global__ void __launch_bounds__(StridedShape<L>::THREADS) k_refine_ipass_adj(
 }
 
 template <int L>
+static int refine_ipass_blocks_t() {
+    return (L * (L / 2 + 1) + StridedShape<L>::P - 1) / StridedShape<L>::P;
+}
+template <int L>
 static void launch_refine_dot_t(const FftTables& T, float2* X1, const float2* FP, const float* filter,
                                 const float* wbin, const RefineGeom* geom, int batch, double* part, hipStream_t s) {
     const float2* tw = T.tw.p + T.offset[fft_len_index(L)];
     ProfScope ps(T.prof, "k_refine_ipass_dot", 3.0 * batch * L * L * (L / 2 + 1) * sizeof(float2), s);
-    k_refine_ipass_dot<L><<<dim3((unsigned)ccc_ipass_blocks_t<L>(), (unsigned)batch), StridedShape<L>::THREADS, 0, s>>>(
+    k_refine_ipass_dot<L><<<dim3((unsigned)refine_ipass_blocks_t<L>(), (unsigned)batch), StridedShape<L>::THREADS, 0, s>>>(
         X1, FP, filter, wbin, geom, part, tw);
 }
 template <int L>
@@ -1344,7 +1307,7 @@ static void launch_refine_adj_c2r_t(const FftTables& T, const float2* X1, const 
     const float2* tw = T.tw.p + T.offset[fft_len_index(L)];
     {
         ProfScope ps(T.prof, "k_refine_ipass_adj", 3.0 * batch * L * L * H * sizeof(float2), s);
-        k_refine_ipass_adj<L><<<dim3((unsigned)ccc_ipass_blocks_t<L>(), (unsigned)batch), StridedShape<L>::THREADS, 0,
+        k_refine_ipass_adj<L><<<dim3((unsigned)refine_ipass_blocks_t<L>(), (unsigned)batch), StridedShape<L>::THREADS, 0,
                                 s>>>(X1, FP, filter, wbin, geom, sc, tmp, tw);
     }
     ETTK_HIP(hipGetLastError());
@@ -1352,7 +1315,15 @@ static void launch_refine_adj_c2r_t(const FftTables& T, const float2* X1, const 
     ProfScope ps(T.prof, plane_name<L>(1), vol_c + vol_r, s);
     k_c2r_plane<L><<<(unsigned)((long)batch * L), Plane<L>::THREADS, 0, s>>>(tmp, out, tw);
 }
-int fft3_refine_ipass_blocks(int n) { return fft3_ccc_ipass_blocks(n); }
+int fft3_refine_ipass_blocks(int n) {
+    switch (n) {
+        case 16: return refine_ipass_blocks_t<16>();
+        case 32: return refine_ipass_blocks_t<32>();
+        case 48: return refine_ipass_blocks_t<48>();
+        case 64: return refine_ipass_blocks_t<64>();
+        default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_refine_ipass: unsupported size " + std::to_string(n)};
+    }
+}
 void fft3_refine_dot(const FftTables& T, float2* X1, const float2* FP, const float* filter, const float* wbin,
                      const RefineGeom* geom, int n, int batch, double* part, hipStream_t s) {
     switch (n) {
