@@ -3,9 +3,7 @@
 // Device side of nbfFourierImageMetric::executeFourierNewHalf (inc/em/nbfFourierImageMetric.h:1078-1323)
 // for a batch of (particle, transform) evaluations:
 //   reslice  -> nbfWedgedSubImage3D::getImage (inc/em/nbfWedgedSubImage3D.h:603-828), VTK tricubic
-//   spec     -> nbfFourierFilter::executeHalf (nbfFourierFilter.h:587-606) with the smoothed analytic wedge
-//               of nbfWedge3D::getImageHalf (nbfWedge3D.h:313-360) generated on the fly, and the Hermitian
-//               weighted sums of normalizeFourierHalf (nbfCorrelationImageMetric.h:498-530)
+//   (the spectral weighting and the transforms around it are in fft.hip)
 //   combine  -> the quadratic expression of FIM.h:1202-1203
 //   dftA/BC  -> the zero-padded (2N)^3 c2r of FIM.h:1209-1214 evaluated only on the search window
 //               (FIM.h:1222-1247) as three separable partial DFTs, followed by the spherical mask and the
@@ -174,67 +172,6 @@ void launch_wedge_ref(const WedgeRef& w, int N, float* W, hipStream_t s) {
     ETTK_HIP(hipGetLastError());
 }
 
-// ------------------------------------------------------------------ spectral filter
-// both sides of one evaluation in one pass, the smoothed wedge computed once per element:
-//   X1 = F1 * filter * W1 W2(e)            (reference side, F1 shared by all evaluations; n1 and sum(W filter))
-//   X2 = mcf(F2[e]) * filter * W1 W2(e)    (particle side, in place; n2)
-// (nbfFourierFilter::executeHalf, FFilt.h:587-606, and the Hermitian weighted sums of normalizeFourierHalf,
-// CorrMetric.h:498-530)
-__global__ void __launch_bounds__(kThreads) k_spec_filter2(const float2* __restrict__ F1, float2* __restrict__ X1,
-                                                            float2* __restrict__ X2, const float* __restrict__ filter,
-                                                            const float* __restrict__ W1, const EvalGeom* __restrict__ geom,
-                                                            int N, int mcf, int apply, float* __restrict__ p_n1,
-                                                            float* __restrict__ p_wf, float* __restrict__ p_n2) {
-    __shared__ float sh[8];
-    const int e = blockIdx.y;
-    const int H = N / 2 + 1;
-    const long nh = (long)N * N * H;
-    const EvalGeom& g = geom[e];
-    const long chunk = (nh + gridDim.x - 1) / gridDim.x;
-    const long h0 = blockIdx.x * chunk, h1 = min(nh, h0 + chunk);
-    const long dc = ((long)(N / 2) * N + N / 2) * H + (H - 1);
-    float s1 = 0.f, swf = 0.f, s2 = 0.f;
-    for (long h = h0 + threadIdx.x; h < h1; h += blockDim.x) {
-        int i, j, k;
-        split3((unsigned)h, (unsigned)N, (unsigned)H, i, j, k);
-        float w = W1 ? W1[h] : 1.f;
-        if (!g.full) w *= wedge_smooth(g.v1, g.v2, i, j, k, N, H);
-        const float fw = filter[h] * w;
-        const float hw = k < H - 1 ? 2.f : 1.f;
-        float2 a = F1[h];
-        if (apply) a = cscale(a, fw);
-        if (h == dc) a = make_float2(0.f, 0.f);
-        X1[(size_t)e * nh + h] = a;
-        s1 += hw * (a.x * a.x + a.y * a.y);
-        swf += fw;
-        float2 z = X2[(size_t)e * nh + h];
-        if (mcf) {
-            float m2 = z.x * z.x + z.y * z.y;
-            float C = sqrtf(sqrtf(m2));
-            if (C > 0.f) z = make_float2(z.x / C, z.y / C);
-        }
-        if (apply) z = cscale(z, fw);
-        if (h == dc) z = make_float2(0.f, 0.f);
-        X2[(size_t)e * nh + h] = z;
-        s2 += hw * (z.x * z.x + z.y * z.y);
-    }
-    const float t1 = block_sum(s1, sh);
-    const float tw = block_sum(swf, sh);
-    const float t2 = block_sum(s2, sh);
-    if (threadIdx.x == 0) {
-        p_n1[(size_t)e * gridDim.x + blockIdx.x] = t1;
-        p_wf[(size_t)e * gridDim.x + blockIdx.x] = tw;
-        p_n2[(size_t)e * gridDim.x + blockIdx.x] = t2;
-    }
-}
-void launch_spec_filter2(const float2* F1, float2* X1, float2* X2, const float* filter, const float* W1,
-                         const EvalGeom* geom, int n_eval, int N, int mcf, int apply, float* p_n1, float* p_wf,
-                         float* p_n2, int nb, hipStream_t s) {
-    dim3 grid(nb, n_eval);
-    k_spec_filter2<<<grid, kThreads, 0, s>>>(F1, X1, X2, filter, W1, geom, N, mcf, apply, p_n1, p_wf, p_n2);
-    ETTK_HIP(hipGetLastError());
-}
-
 // ------------------------------------------------------------------ wedge overlap
 // nbfCorrelationImageMetric::getWedgeOverlap (CorrMetric.h:533-566): sum(W1 W2(t) filter) over the half grid,
 // W2 the particle's smoothed wedge at the evaluation's transform (all ones when geom.full).  Per-block FP64
@@ -274,29 +211,6 @@ void launch_wedge_overlap(const float* W1, const float* filter, const EvalGeom* 
     const int nb = 64;
     k_wedge_overlap<<<dim3(nb, E), kThreads, 0, s>>>(W1, filter, geom, N, part);
     k_sum_partials<<<(E + 127) / 128, 128, 0, s>>>(part, nb, E, out);
-    ETTK_HIP(hipGetLastError());
-}
-
-// ------------------------------------------------------------------ reference-side real-space mask
-__global__ void __launch_bounds__(kThreads) k_mask_ref(float* __restrict__ R, const float* __restrict__ m1, int N,
-                                                        float* __restrict__ partials) {
-    __shared__ float sh[8];
-    const int e = blockIdx.y;
-    const long n3 = (long)N * N * N;
-    const long chunk = (n3 + gridDim.x - 1) / gridDim.x;
-    const long o0 = blockIdx.x * chunk, o1 = min(n3, o0 + chunk);
-    float s = 0.f;
-    for (long o = o0 + threadIdx.x; o < o1; o += blockDim.x) {
-        float r = R[(size_t)e * n3 + o], m = m1[o];
-        s += r * r * m;
-        R[(size_t)e * n3 + o] = r * m;
-    }
-    float t = block_sum(s, sh);
-    if (threadIdx.x == 0) partials[(size_t)e * gridDim.x + blockIdx.x] = t;
-}
-void launch_mask_ref(float* R, const float* m1, int n_eval, int N, float* partials, int nb, hipStream_t s) {
-    dim3 grid(nb, n_eval);
-    k_mask_ref<<<grid, kThreads, 0, s>>>(R, m1, N, partials);
     ETTK_HIP(hipGetLastError());
 }
 

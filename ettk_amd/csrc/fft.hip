@@ -160,15 +160,59 @@ __device__ __forceinline__ void fft64_reg(float2* pen, int lane, const TwCache<6
     __syncthreads();
 }
 
+// The same for 96 = 12 x 8 and 128 = 16 x 8: an (L/8)-point DFT per thread, the exchange, then L/8 8-point DFTs over the
+// 8 threads (two per thread; at 96 half of the threads' second one is idle).  The pencil's storage spans 9 L/8 entries.
+template <int L, bool INV>
+__device__ __forceinline__ void fft_reg8(float2* pen, int lane, const float2* tw) {
+    constexpr int N1 = L / 8, NR = (N1 + 7) / 8;
+    float2 x[N1];
+#pragma unroll
+    for (int m = 0; m < N1; m++) x[m] = pen[lane + 8 * m];
+    Dft<N1, INV>::run(x);
+#pragma unroll
+    for (int k = 1; k < N1; k++) {
+        float2 w = tw[lane * k];
+        if (INV) w.y = -w.y;
+        x[k] = cmul(x[k], w);
+    }
+    wave_lds_order();
+#pragma unroll
+    for (int k = 0; k < N1; k++) pen[k * 9 + lane] = x[k];
+    wave_lds_order();
+    float2 y[NR][8];
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        const int k1 = lane + 8 * r;
+        if (k1 < N1) {
+#pragma unroll
+            for (int b = 0; b < 8; b++) y[r][b] = pen[k1 * 9 + b];
+            Dft<8, INV>::run(y[r]);
+        }
+    }
+    wave_lds_order();
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        const int k1 = lane + 8 * r;
+        if (k1 < N1)
+#pragma unroll
+            for (int k = 0; k < 8; k++) pen[k1 + N1 * k] = y[r][k];
+    }
+    __syncthreads();
+}
+
 // threads per pencil of the pencil FFT used by the fused and strided passes, and the LDS stride of a pencil
 template <int L> struct PenT {
-    static constexpr int TPP = (L == 64) ? 8 : Shape<L>::TPP;
-    static constexpr int LD = (L == 64) ? 73 : L + 1;
+    static constexpr bool kReg = L == 64 || L == 96 || L == 128;
+    static constexpr int TPP = kReg ? 8 : Shape<L>::TPP;
+    static constexpr int LD = kReg ? 9 * (L / 8) + 1 : L + 1;
 };
 template <int L>
 __device__ __forceinline__ void pencil_fft(float2* pen, int lane, const float2* tw, const TwCache<L>& tc, bool inv) {
     if constexpr (L == 64) fft64_reg(pen, lane, tc, inv);
-    else lds_fft<L>(pen, lane, tw, inv);
+    else if constexpr (PenT<L>::kReg) {
+        if (inv) fft_reg8<L, true>(pen, lane, tw);
+        else fft_reg8<L, false>(pen, lane, tw);
+    } else lds_fft<L>(pen, lane, tw, inv);
 }
 
 // ------------------------------------------------------------------ r2c, pass along k (real rows)
@@ -319,7 +363,7 @@ __global__ void __launch_bounds__(ColShape<L>::THREADS) k_fft_col(StridedArgs a,
         for (int j = 0; j < S::E; j++) a.out[base + (long)(t + j * S::T) * a.es] = x[j];
 }
 
-// ------------------------------------------------------------------ CCC spectra: one pass along i (L <= 64)
+// ------------------------------------------------------------------ CCC spectra: one pass along i (L <= 128)
 // deterministic sum over the NT threads of a workgroup (NT need not be a multiple of 64), valid in thread 0
 template <int NT>
 __device__ __forceinline__ float block_sum_nt(float v, float* sred) {
@@ -346,8 +390,8 @@ __device__ __forceinline__ float block_sum_nt(float v, float* sred) {
 //   X2 = mcf(F2) * fw, DC term zeroed -> S2 (the combine's F2), and its inverse i-transform -> S3
 //   X1 = F1mcf * fw, DC term zeroed -> inverse i-transform -> S1
 //   per-block partials of sum hw |X1|^2, sum fw, sum hw |X2|^2 (hw = 2 off the last half plane)
-// The element-wise arithmetic is that of k_spec_filter2 (nbfFourierFilter::executeHalf, FFilt.h:587-606, and
-// normalizeFourierHalf, CorrMetric.h:498-530); the transforms are those of the separate i passes.
+// The element-wise arithmetic is that of nbfFourierFilter::executeHalf (FFilt.h:587-606) and normalizeFourierHalf
+// (CorrMetric.h:498-530).
 // Each thread keeps its E elements of a pencil in registers through the three transforms (regfft.hpp).
 template <int L>
 __global__ void __launch_bounds__(ColShape<L>::THREADS) k_ccc_ipass(CccIpassArgs a, const float2* __restrict__ twg) {
@@ -477,7 +521,7 @@ __global__ void __launch_bounds__(Shape<L>::THREADS) k_c2r_rows(const float2* __
     }
 }
 
-// ------------------------------------------------------------------ fused plane passes (L <= 64)
+// ------------------------------------------------------------------ fused plane passes (L <= 128)
 // One workgroup per (batch, i) plane of L x L reals: the k pass (pairs of real rows packed as complex rows) and
 // the j pass run back to back in LDS, so an r2c moves each element through HBM twice (plane pass + i pass)
 // instead of three times.  H pencil groups of TPP threads; the spare group of the k pass works on a dummy row.
@@ -672,7 +716,7 @@ __global__ void __launch_bounds__(Plane<L>::THREADS) k_c2r_plane(const float2* _
     }
 }
 
-// ------------------------------------------------------------------ fused c2r -> pointwise op -> r2c (L <= 64)
+// ------------------------------------------------------------------ fused c2r -> pointwise op -> r2c (L <= 128)
 // Between the inverse and the forward transform of one volume, a (b, i) plane is complete in LDS after the c2r
 // plane passes: the pointwise operation and the r2c plane passes run there, so the real volume never goes
 // through HBM.  `io` holds the half spectrum after the inverse i pass and receives the forward j/k passes.
@@ -1012,7 +1056,7 @@ static void launch_r2c(const FftTables& T, const R2CArgs& a, float2* scratch, hi
     const double vol_c = (double)a.batch * L * L * H * sizeof(float2);  // one pass over the half spectrum
     const double vol_r = a.pro == PRO_PAD_MASKED ? (double)a.batch * a.ns * a.ns * a.ns * sizeof(float)
                                                  : (double)a.batch * L * L * L * sizeof(float);
-    if constexpr (L <= 64) {
+    if constexpr (L <= 128) {
         // passes k and j fused per (b, i) plane
         ProfScope ps(T.prof, plane_name<L>(0), vol_r + vol_c, s);
         k_r2c_plane<L><<<(unsigned)((long)a.batch * L), Plane<L>::THREADS, 0, s>>>(a, tw);
@@ -1049,7 +1093,7 @@ static void launch_c2r(const FftTables& T, const float2* in, float2* tmp, float*
         ProfScope ps(T.prof, prof_name<L>(1), 2 * vol_c, s);
         launch_strided<L>(si, tw, s);
     }
-    if constexpr (L <= 64) {
+    if constexpr (L <= 128) {
         ProfScope ps(T.prof, plane_name<L>(1), vol_c + vol_r, s);
         k_c2r_plane<L><<<(unsigned)((long)batch * L), Plane<L>::THREADS, 0, s>>>(tmp, out, tw);
     } else {
@@ -1089,8 +1133,6 @@ static void launch_c2r_op_r2c(const FftTables& T, const float2* in, float2* io, 
     }
 }
 
-bool fft3_fused_supported(int n) { return n == 16 || n == 32 || n == 48 || n == 64; }
-
 bool ccc_combine_fft_supported(const CccSizes& z) { return z.N == 64; }
 void launch_dftBC_fft(const FftTables& T, const float2* G1, const float2* tabK, const CccSizes& z, int n_eval,
                       float* best_val, int* best_idx, hipStream_t s) {
@@ -1124,6 +1166,8 @@ int fft3_ccc_ipass_blocks(int n) {
         case 32: return ccc_ipass_blocks_t<32>();
         case 48: return ccc_ipass_blocks_t<48>();
         case 64: return ccc_ipass_blocks_t<64>();
+        case 96: return ccc_ipass_blocks_t<96>();
+        case 128: return ccc_ipass_blocks_t<128>();
         default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_ccc_ipass: unsupported size " + std::to_string(n)};
     }
 }
@@ -1143,6 +1187,8 @@ void fft3_ccc_ipass(const FftTables& T, const CccIpassArgs& a, int n, int batch,
         case 32: launch_ccc_ipass<32>(T, a, batch, s); break;
         case 48: launch_ccc_ipass<48>(T, a, batch, s); break;
         case 64: launch_ccc_ipass<64>(T, a, batch, s); break;
+        case 96: launch_ccc_ipass<96>(T, a, batch, s); break;
+        case 128: launch_ccc_ipass<128>(T, a, batch, s); break;
         default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_ccc_ipass: unsupported size " + std::to_string(n)};
     }
     ETTK_HIP(hipGetLastError());
@@ -1321,6 +1367,8 @@ int fft3_refine_ipass_blocks(int n) {
         case 32: return refine_ipass_blocks_t<32>();
         case 48: return refine_ipass_blocks_t<48>();
         case 64: return refine_ipass_blocks_t<64>();
+        case 96: return refine_ipass_blocks_t<96>();
+        case 128: return refine_ipass_blocks_t<128>();
         default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_refine_ipass: unsupported size " + std::to_string(n)};
     }
 }
@@ -1331,6 +1379,8 @@ void fft3_refine_dot(const FftTables& T, float2* X1, const float2* FP, const flo
         case 32: launch_refine_dot_t<32>(T, X1, FP, filter, wbin, geom, batch, part, s); break;
         case 48: launch_refine_dot_t<48>(T, X1, FP, filter, wbin, geom, batch, part, s); break;
         case 64: launch_refine_dot_t<64>(T, X1, FP, filter, wbin, geom, batch, part, s); break;
+        case 96: launch_refine_dot_t<96>(T, X1, FP, filter, wbin, geom, batch, part, s); break;
+        case 128: launch_refine_dot_t<128>(T, X1, FP, filter, wbin, geom, batch, part, s); break;
         default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_refine_dot: unsupported size " + std::to_string(n)};
     }
     ETTK_HIP(hipGetLastError());
@@ -1343,6 +1393,8 @@ void fft3_refine_adj_c2r(const FftTables& T, const float2* X1, const float2* FP,
         case 32: launch_refine_adj_c2r_t<32>(T, X1, FP, filter, wbin, geom, sc, batch, tmp, out, s); break;
         case 48: launch_refine_adj_c2r_t<48>(T, X1, FP, filter, wbin, geom, sc, batch, tmp, out, s); break;
         case 64: launch_refine_adj_c2r_t<64>(T, X1, FP, filter, wbin, geom, sc, batch, tmp, out, s); break;
+        case 96: launch_refine_adj_c2r_t<96>(T, X1, FP, filter, wbin, geom, sc, batch, tmp, out, s); break;
+        case 128: launch_refine_adj_c2r_t<128>(T, X1, FP, filter, wbin, geom, sc, batch, tmp, out, s); break;
         default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_refine_adj_c2r: unsupported size " + std::to_string(n)};
     }
     ETTK_HIP(hipGetLastError());
@@ -1355,6 +1407,8 @@ void fft3_r2c_planes(const FftTables& T, const R2CArgs& a, hipStream_t s) {
         case 32: launch_r2c_planes<32>(T, a, s); break;
         case 48: launch_r2c_planes<48>(T, a, s); break;
         case 64: launch_r2c_planes<64>(T, a, s); break;
+        case 96: launch_r2c_planes<96>(T, a, s); break;
+        case 128: launch_r2c_planes<128>(T, a, s); break;
         default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_r2c_planes: unsupported size " + std::to_string(a.n)};
     }
     ETTK_HIP(hipGetLastError());
@@ -1367,6 +1421,8 @@ void fft3_op_r2c_after_ipass(const FftTables& T, float2* io, int n, int batch, i
         case 32: launch_c2r_op_r2c<32>(T, nullptr, io, batch, op, aux, partials, s, forward_i); break;
         case 48: launch_c2r_op_r2c<48>(T, nullptr, io, batch, op, aux, partials, s, forward_i); break;
         case 64: launch_c2r_op_r2c<64>(T, nullptr, io, batch, op, aux, partials, s, forward_i); break;
+        case 96: launch_c2r_op_r2c<96>(T, nullptr, io, batch, op, aux, partials, s, forward_i); break;
+        case 128: launch_c2r_op_r2c<128>(T, nullptr, io, batch, op, aux, partials, s, forward_i); break;
         default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_op_r2c_after_ipass: unsupported size " + std::to_string(n)};
     }
     ETTK_HIP(hipGetLastError());
@@ -1380,6 +1436,8 @@ void fft3_c2r_op_r2c(const FftTables& T, const float2* in, float2* io, int n, in
         case 32: launch_c2r_op_r2c<32>(T, in, io, batch, op, aux, partials, s); break;
         case 48: launch_c2r_op_r2c<48>(T, in, io, batch, op, aux, partials, s); break;
         case 64: launch_c2r_op_r2c<64>(T, in, io, batch, op, aux, partials, s); break;
+        case 96: launch_c2r_op_r2c<96>(T, in, io, batch, op, aux, partials, s); break;
+        case 128: launch_c2r_op_r2c<128>(T, in, io, batch, op, aux, partials, s); break;
         default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_c2r_op_r2c: unsupported size " + std::to_string(n)};
     }
     ETTK_HIP(hipGetLastError());

@@ -275,8 +275,6 @@ static void plan_constants(ettk_plan* P) {
     P->dummy_filter = !(bp || p.bfactor != 0.0f);
     P->sum_filter = 0;
     for (float v : f) P->sum_filter += v;
-    P->nb_real = (int)((n3 + 1023) / 1024);
-    P->nb_spec = (int)((nh + 1023) / 1024);
     P->nb_res = reslice_blocks(N);
     P->h_m1 = m1;
     P->m1.upload(m1.data(), n3, s);
@@ -289,10 +287,8 @@ static void plan_constants(ettk_plan* P) {
     search_window(P);
 }
 
-// spectral partials per evaluation: per k_spec_filter2 block, or per k_ccc_ipass block (fused transforms)
-static size_t spectral_partials(const ettk_plan* P) {
-    return (size_t)std::max(P->nb_spec, fft3_fused_supported(P->N) ? fft3_ccc_ipass_blocks(P->N) : 0);
-}
+// spectral partials per evaluation: one per k_ccc_ipass block
+static size_t spectral_partials(const ettk_plan* P) { return (size_t)fft3_ccc_ipass_blocks(P->N); }
 
 // one region holding a CccWork for E evaluations: every piece starts on a 256-byte boundary
 template <class F>
@@ -305,7 +301,7 @@ static void ccc_work_pieces(const ettk_plan* P, int E, F&& piece) {
     piece(3, nb_sp * E * sizeof(float));                                // p_n1
     piece(4, nb_sp * E * sizeof(float));                                // p_n2
     piece(5, nb_sp * E * sizeof(float));                                // p_wf
-    piece(6, (size_t)std::max(P->nb_real, N) * E * sizeof(float));      // p_k1
+    piece(6, (size_t)N * E * sizeof(float));                            // p_k1: one per plane
     piece(7, (size_t)E * sizeof(float));                                // stats
     piece(8, (size_t)4 * E * sizeof(float));                            // scalars
     piece(9, (size_t)P->z.E * E * sizeof(float));                       // bval
@@ -365,7 +361,7 @@ void ensure_ccc_workspace(ettk_plan* P, int cap) {
     P->p_n1.ensure(nb_sp * cap);
     P->p_n2.ensure(nb_sp * cap);
     P->p_wf.ensure(nb_sp * cap);
-    P->p_k1.ensure((size_t)std::max(P->nb_real, N) * cap);  // mask partials: per block, or per plane (fused)
+    P->p_k1.ensure((size_t)N * cap);  // mask partials, one per plane
     P->stats.ensure(cap);
     P->scalars.ensure((size_t)4 * cap);
     P->bval.ensure((size_t)P->z.E * cap);
@@ -544,48 +540,26 @@ void ccc_enqueue_chunk(ettk_plan* P, const CccWork& W, const float* d_parts, con
     }
     launch_reslice_mean(W.p_res, P->nb_res, E, W.stats, s);
     R2CArgs a2{W.R2, W.S2, N, E, PRO_RESLICED, P->maskfft.p, W.stats};
-    const bool fused = fft3_fused_supported(N);
-    int nb_sp = P->nb_spec;
-    if (fused) {
-        // F2 = r2c((reslice - mean) maskfft shift) up to its i pass; then on pencils along i: the i pass, both
-        // spectra weighted by filter x W1 W2 (X1 = F1mcf, the reference with MCF applied once; X2 = mcf(F2)),
-        // X2 kept for the combine, and both inverse i passes of the transforms below
-        fft3_r2c_planes(P->ctx->fft, a2, s);
-        CccIpassArgs ia{W.S2, W.S3, W.S1, P->F1mcf.p, P->filter.p, W1, geo, P->p.mcf, apply, W.p_n1, W.p_wf, W.p_n2};
-        fft3_ccc_ipass(P->ctx->fft, ia, N, E, s);
-        nb_sp = fft3_ccc_ipass_blocks(N);
-        // reference side: c2r -> r1 m1 (with the k1_m partials) -> r2c = F1m, one partial per (evaluation, plane)
-        // (at 64 the forward i passes of both run inside the combine kernel)
-        const bool fwd = !ccc_combine_fft_supported(P->z);
-        fft3_op_r2c_after_ipass(P->ctx->fft, W.S1, N, E, PLANE_OP_MASK, P->m1.p, W.p_k1, fwd, s);
-        // particle side: Q = r2c(c2r(X2)^2 shift)
-        fft3_op_r2c_after_ipass(P->ctx->fft, W.S3, N, E, PLANE_OP_SQUARE_SHIFT, nullptr, nullptr, fwd, s);
-    } else {
-        fft3_r2c(P->ctx->fft, a2, nullptr, s);
-        // both spectra weighted by filter x W1 W2 in one pass: X1 = F1mcf (reference, MCF applied once), X2 = mcf(F2)
-        {
-            ProfScope ps(kp, "k_spec_filter", 4 * Hb, s);
-            launch_spec_filter2(P->F1mcf.p, W.S1, W.S2, P->filter.p, W1, geo, E, N, P->p.mcf, apply, W.p_n1, W.p_wf,
-                                W.p_n2, P->nb_spec, s);
-        }
-        fft3_c2r(P->ctx->fft, W.S1, W.S1, W.R1, N, E, s);
-        {
-            ProfScope ps(kp, "k_mask_ref", 2 * Rb, s);
-            launch_mask_ref(W.R1, P->m1.p, E, N, W.p_k1, P->nb_real, s);
-        }
-        R2CArgs a1{W.R1, W.S1, N, E, PRO_NONE, nullptr, nullptr};
-        fft3_r2c(P->ctx->fft, a1, nullptr, s);
-        fft3_c2r(P->ctx->fft, W.S2, W.S3, W.R2, N, E, s);
-        R2CArgs a3{W.R2, W.S3, N, E, PRO_SQUARE_SHIFT, nullptr, nullptr};
-        fft3_r2c(P->ctx->fft, a3, nullptr, s);
-    }
+    // F2 = r2c((reslice - mean) maskfft shift) up to its i pass; then on pencils along i: the i pass, both
+    // spectra weighted by filter x W1 W2 (X1 = F1mcf, the reference with MCF applied once; X2 = mcf(F2)),
+    // X2 kept for the combine, and both inverse i passes of the transforms below
+    fft3_r2c_planes(P->ctx->fft, a2, s);
+    CccIpassArgs ia{W.S2, W.S3, W.S1, P->F1mcf.p, P->filter.p, W1, geo, P->p.mcf, apply, W.p_n1, W.p_wf, W.p_n2};
+    fft3_ccc_ipass(P->ctx->fft, ia, N, E, s);
+    const int nb_sp = fft3_ccc_ipass_blocks(N);
+    // reference side: c2r -> r1 m1 (with the k1_m partials) -> r2c = F1m, one partial per (evaluation, plane)
+    // (at 64 the forward i passes of both run inside the combine kernel)
+    const bool fwd = !ccc_combine_fft_supported(P->z);
+    fft3_op_r2c_after_ipass(P->ctx->fft, W.S1, N, E, PLANE_OP_MASK, P->m1.p, W.p_k1, fwd, s);
+    // particle side: Q = r2c(c2r(X2)^2 shift)
+    fft3_op_r2c_after_ipass(P->ctx->fft, W.S3, N, E, PLANE_OP_SQUARE_SHIFT, nullptr, nullptr, fwd, s);
     // combine, upsampled correlation on the search window, peak
-    launch_ccc_scalars(W.p_n1, W.p_n2, W.p_k1, W.p_wf, nb_sp, fused ? N : P->nb_real, E, N, W.scalars, s);
+    launch_ccc_scalars(W.p_n1, W.p_n2, W.p_k1, W.p_wf, nb_sp, N, E, N, W.scalars, s);
     const bool cfft = ccc_combine_fft_supported(P->z);
     {
         ProfScope ps(kp, cfft ? "k_combine_fftA" : "k_combine_dftA", 3 * Hb + Gb, s);
         if (cfft)
-            launch_combine_fftA(P->ctx->fft, W.S1, W.S2, W.S3, P->Mfft.p, W.scalars, P->z, E, W.G1, fused, s);
+            launch_combine_fftA(P->ctx->fft, W.S1, W.S2, W.S3, P->Mfft.p, W.scalars, P->z, E, W.G1, true, s);
         else
             launch_combine_dftA(W.S1, W.S2, W.S3, P->Mfft.p, W.scalars, P->tabA.p, P->z, E, W.G1, s);
     }
@@ -744,7 +718,7 @@ int ettk_fft3(ettk_ctx* ctx, int n, int batch, int kind, const void* in, void* o
     ETTK_REQUIRE(ctx && in && out && batch > 0, ETTK_ERR_ARG, "ettk_fft3: bad argument");
     ETTK_REQUIRE(fft_len_index(n) >= 0, ETTK_ERR_UNSUPPORTED, "ettk_fft3: unsupported size " + std::to_string(n));
     ETTK_REQUIRE(kind >= ETTK_FFT_R2C && kind <= ETTK_FFT_SQUARE, ETTK_ERR_ARG, "ettk_fft3: unknown kind");
-    ETTK_REQUIRE(kind < ETTK_FFT_MASK || fft3_fused_supported(n), ETTK_ERR_UNSUPPORTED,
+    ETTK_REQUIRE(kind < ETTK_FFT_MASK || n <= 64, ETTK_ERR_UNSUPPORTED,
                  "ettk_fft3: the fused transforms need n <= 64");
     ETTK_REQUIRE(kind != ETTK_FFT_MASK || aux, ETTK_ERR_ARG, "ettk_fft3: ETTK_FFT_MASK needs the mask");
     ETTK_HIP(hipSetDevice(ctx->device));

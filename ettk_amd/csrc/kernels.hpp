@@ -47,7 +47,7 @@ struct EvalGeom {
 };
 
 // The CCC steps between the particle's r2c plane passes and the fused plane kernels, on pencils along i
-// (n <= 64, fft3_fused_supported): S2 holds the plane-pass output of the resliced particles and receives the
+// (n <= 128): S2 holds the plane-pass output of the resliced particles and receives the
 // filtered particle spectra X2; S3 receives X2 and S1 the filtered reference spectrum X1, both inverse-transformed
 // along i (the inputs of fft3_op_r2c_after_ipass).  Partials: fft3_ccc_ipass_blocks(n) per evaluation.
 struct CccIpassArgs {
@@ -65,7 +65,7 @@ struct CccIpassArgs {
 };
 int fft3_ccc_ipass_blocks(int n);
 void fft3_ccc_ipass(const FftTables& T, const CccIpassArgs& a, int n, int batch, hipStream_t s);
-// the k/j plane passes of an r2c only (n <= 64): the i pass is left to fft3_ccc_ipass
+// the k/j plane passes of an r2c only (n <= 128): the i pass is left to fft3_ccc_ipass
 void fft3_r2c_planes(const FftTables& T, const R2CArgs& a, hipStream_t s);
 // fft3_c2r_op_r2c whose inverse i pass has already run (io holds the i-inverse-transformed spectra); without
 // `forward_i` its forward i pass is left to launch_combine_fftA
@@ -104,13 +104,6 @@ void launch_reslice_projection(const float* parts, const EvalGeom* geom, int n, 
                                int nb, hipStream_t s);
 // mean of the valid voxels per evaluation, from the reslice partials (nb per eval): stats[e] = mean
 void launch_reslice_mean(const float* partials, int nb, int n_eval, float* stats, hipStream_t s);
-// spectral weighting of both CCC sides: X1 = F1 filter W1 W2(e) (F1 shared), X2 = mcf(X2) filter W1 W2(e) in
-// place (mcf: F / |F|^.5), DC = 0; per-block partials of the Hermitian weighted |X1|^2, sum(W filter), |X2|^2
-void launch_spec_filter2(const float2* F1, float2* X1, float2* X2, const float* filter, const float* W1,
-                         const EvalGeom* geom, int n_eval, int N, int mcf, int apply, float* p_n1, float* p_wf,
-                         float* p_n2, int nb, hipStream_t s);
-// r1 *= m1, partial sums of r1^2 m1
-void launch_mask_ref(float* R, const float* m1, int n_eval, int N, float* partials, int nb, hipStream_t s);
 // per-evaluation scalars: norm1, norm2, k1_m, sum(W filter)
 void launch_ccc_scalars(const float* p_n1, const float* p_n2, const float* p_k1, const float* p_wf, int nb_spec,
                         int nb_real, int n_eval, int N, float* scalars, hipStream_t s);
@@ -159,11 +152,11 @@ __device__ __forceinline__ float refine_hweight(const float* __restrict__ filter
 }
 int refine_moment_blocks(int N);
 void launch_refine_scalars(const double* part, int nb, int E, double* sc, hipStream_t s);
-// the refinement's transforms with the score and adjoint steps in their i passes (box sizes 16, 32, 48, 64):
-//   fft3_refine_dot: forward i pass of X1 in place (after fft3_r2c_planes) with the FP64 score partials of
-//     launch_refine_dot, fft3_refine_ipass_blocks(n) per evaluation;
-//   fft3_refine_adj_c2r: the adjoint spectrum of launch_refine_adj formed on load, its inverse i pass into
-//     `tmp`, then the c2r plane passes into `out` (X1 unchanged)
+// the refinement's transforms with the score and adjoint steps in their i passes (box sizes up to 128):
+//   fft3_refine_dot: forward i pass of X1 in place (after fft3_r2c_planes) with the FP64 score partials
+//     <H X1, H X2>, |H X1|^2, |H X2|^2 (Hermitian weights), fft3_refine_ipass_blocks(n) per evaluation;
+//   fft3_refine_adj_c2r: the adjoint spectrum H (H X2 / (n1 n2) - S H X1 / n1^2) formed on load, its inverse i
+//     pass into `tmp`, then the c2r plane passes into `out` (X1 unchanged)
 int fft3_refine_ipass_blocks(int n);
 void fft3_refine_dot(const FftTables& T, float2* X1, const float2* FP, const float* filter, const float* wbin,
                      const RefineGeom* geom, int n, int batch, double* part, hipStream_t s);
@@ -171,15 +164,10 @@ void fft3_refine_adj_c2r(const FftTables& T, const float2* X1, const float2* FP,
                          const float* wbin, const RefineGeom* geom, const double* sc, int n, int batch, float2* tmp,
                          float* out, hipStream_t s);
 
-int refine_dot_blocks(int N);
 // mean of each of `count` volumes; `part` holds vol_mean_blocks(N) doubles per volume
 int vol_mean_blocks(int N);
 void launch_vol_mean(const float* vols, int count, int N, double* part, float* mean, hipStream_t s);
 void launch_reslice_ref(const float* ref, const RefineGeom* geom, int E, int N, float* out, hipStream_t s);
-void launch_refine_dot(const float2* X1, const float2* FP, const float* filter, const float* wbin, const RefineGeom* geom,
-                       int E, int N, double* part, double* sc, hipStream_t s);
-void launch_refine_adj(float2* X1, const float2* FP, const float* filter, const float* wbin, const RefineGeom* geom,
-                       int E, int N, const double* sc, hipStream_t s);
 void launch_refine_moments(const float* ref, const RefineGeom* geom, const float* G, const float* maskfft, int E, int N,
                            float* mpart, double* mom, hipStream_t s);
 void launch_wedge_ref(const WedgeRef& w, int N, float* W, hipStream_t s);

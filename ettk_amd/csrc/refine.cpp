@@ -69,8 +69,8 @@ static std::vector<RefineChunk*> refine_prepare(ettk_plan* P, int n) {
     const int N = P->N;
     ensure_ccc_workspace(P, std::min(n, 128));
     const int cap = std::min(P->cap, 128);
-    const int nbd = refine_dot_blocks(N), nbm = refine_moment_blocks(N);
-    P->r_pdot.ensure((size_t)3 * std::max(nbd, fft3_fused_supported(N) ? fft3_refine_ipass_blocks(N) : 0) * cap);
+    const int nbm = refine_moment_blocks(N);
+    P->r_pdot.ensure((size_t)3 * fft3_refine_ipass_blocks(N) * cap);
     P->r_mpart.ensure((size_t)12 * nbm * cap);
     P->r_sc.ensure((size_t)4 * n);
     P->r_mom.ensure((size_t)12 * n);
@@ -148,40 +148,25 @@ static void refine_geometry(const ettk_plan* P, const ettk_particle* descs, cons
 // upload of the chunk's geometry, its kernels and the download of its scores and moments; returns at once.  The
 // particle spectra of the referenced particles must be in P->r_fp.
 static void refine_enqueue(ettk_plan* P, RefineChunk& c) {
-    const int N = P->N, H = P->H;
-    const long nh = (long)N * N * H;
+    const int N = P->N;
     hipStream_t s = P->stream;
     KernelProf* kp = P->ctx->fft.prof;
     const int E = c.E, e0 = c.e0;
     RefineGeom* geo = P->r_geom.p + e0;
     upload_before(P, geo, c.hg.p, (size_t)E * sizeof(RefineGeom));
-    const double Rb = (double)E * N * N * N * sizeof(float), Hb = (double)E * nh * sizeof(float2);
+    const double Rb = (double)E * N * N * N * sizeof(float);
     {
         ProfScope ps(kp, "k_reslice_ref", Rb, s);
         launch_reslice_ref(P->ref_x.p, geo, E, N, P->R2.p, s);
     }
     R2CArgs a{P->R2.p, P->S2.p, N, E, PRO_MASK_SHIFT, P->maskfft.p, nullptr};
     double* sc = P->r_sc.p + (size_t)4 * e0;
-    if (fft3_fused_supported(N)) {
-        // the score terms in the epilogue of the forward i pass, the adjoint spectrum in the prologue of the
-        // inverse one: X1 is read once by each instead of once more by separate score and adjoint passes
-        fft3_r2c_planes(P->ctx->fft, a, s);
-        fft3_refine_dot(P->ctx->fft, P->S2.p, P->r_fp.p, P->filter.p, P->ref_wbin.p, geo, N, E, P->r_pdot.p, s);
-        launch_refine_scalars(P->r_pdot.p, fft3_refine_ipass_blocks(N), E, sc, s);
-        fft3_refine_adj_c2r(P->ctx->fft, P->S2.p, P->r_fp.p, P->filter.p, P->ref_wbin.p, geo, sc, N, E, P->S3.p, P->R1.p,
-                            s);
-    } else {
-        fft3_r2c(P->ctx->fft, a, nullptr, s);
-        {
-            ProfScope ps(kp, "k_refine_dot", 2 * Hb, s);
-            launch_refine_dot(P->S2.p, P->r_fp.p, P->filter.p, P->ref_wbin.p, geo, E, N, P->r_pdot.p, sc, s);
-        }
-        {
-            ProfScope ps(kp, "k_refine_adj", 3 * Hb, s);
-            launch_refine_adj(P->S2.p, P->r_fp.p, P->filter.p, P->ref_wbin.p, geo, E, N, sc, s);
-        }
-        fft3_c2r(P->ctx->fft, P->S2.p, P->S3.p, P->R1.p, N, E, s);
-    }
+    // the score terms in the epilogue of the forward i pass, the adjoint spectrum in the prologue of the inverse one:
+    // X1 is read once by each instead of once more by separate score and adjoint passes
+    fft3_r2c_planes(P->ctx->fft, a, s);
+    fft3_refine_dot(P->ctx->fft, P->S2.p, P->r_fp.p, P->filter.p, P->ref_wbin.p, geo, N, E, P->r_pdot.p, s);
+    launch_refine_scalars(P->r_pdot.p, fft3_refine_ipass_blocks(N), E, sc, s);
+    fft3_refine_adj_c2r(P->ctx->fft, P->S2.p, P->r_fp.p, P->filter.p, P->ref_wbin.p, geo, sc, N, E, P->S3.p, P->R1.p, s);
     double* mom = P->r_mom.p + (size_t)12 * e0;
     {
         ProfScope ps(kp, "k_refine_moments", Rb, s);

@@ -216,45 +216,6 @@ __global__ void __launch_bounds__(kT) k_reslice_ref(const float* __restrict__ re
     }
 }
 
-// per-block FP64 partials of <H X1, H X2>, |H X1|^2, |H X2|^2 (Hermitian weights): X1 = S1[e], X2 = FP[spec]
-__global__ void __launch_bounds__(kT) k_refine_dot(const float2* __restrict__ X1, const float2* __restrict__ FP,
-                                                    const float* __restrict__ filter, const float* __restrict__ wbin,
-                                                    const RefineGeom* __restrict__ geom, int N,
-                                                    double* __restrict__ part) {
-    __shared__ double sh[3][kT / 64];
-    const int e = blockIdx.y, H = N / 2 + 1;
-    const long nh = (long)N * N * H;
-    const RefineGeom g = geom[e];
-    const float2* x1p = X1 + (size_t)e * nh;
-    const float2* x2p = FP + (size_t)g.spec * nh;
-    double sd = 0.0, s1 = 0.0, s2 = 0.0;
-    for (long h = (long)blockIdx.x * kT + threadIdx.x; h < nh; h += (long)gridDim.x * kT) {
-        int a, b, c;
-        split3((unsigned)h, (unsigned)N, (unsigned)H, a, b, c);
-        const float w = refine_hweight(filter, wbin, g, h, a, b, c, N, H);
-        const float2 u = x1p[h], v = x2p[h];
-        const double ww = (c == 0 || c == H - 1) ? (double)w * w : 2.0 * (double)w * w;
-        sd += ww * ((double)u.x * v.x + (double)u.y * v.y);
-        s1 += ww * ((double)u.x * u.x + (double)u.y * u.y);
-        s2 += ww * ((double)v.x * v.x + (double)v.y * v.y);
-    }
-    sd = dsum64(sd);
-    s1 = dsum64(s1);
-    s2 = dsum64(s2);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        sh[0][w] = sd;
-        sh[1][w] = s1;
-        sh[2][w] = s2;
-    }
-    __syncthreads();
-    if (threadIdx.x < 3) {
-        double t = 0.0;
-        for (int i = 0; i < kT / 64; i++) t += sh[threadIdx.x][i];
-        part[((size_t)e * gridDim.x + blockIdx.x) * 3 + threadIdx.x] = t;
-    }
-}
-
 // sc[e] = {S, n1, n2} in FP64
 __global__ void __launch_bounds__(64) k_refine_scalars(const double* __restrict__ part, int nb, int n_eval,
                                                        double* __restrict__ sc) {
@@ -275,29 +236,6 @@ __global__ void __launch_bounds__(64) k_refine_scalars(const double* __restrict_
     sc[e * 4 + 0] = (n1 > 0 && n2 > 0) ? d / (n1 * n2) : 0.0;
     sc[e * 4 + 1] = n1;
     sc[e * 4 + 2] = n2;
-}
-
-// adjoint spectrum in place: X1 <- H (H X2 / (n1 n2) - S H X1 / n1^2)
-__global__ void __launch_bounds__(kT) k_refine_adj(float2* __restrict__ X1, const float2* __restrict__ FP,
-                                                    const float* __restrict__ filter, const float* __restrict__ wbin,
-                                                    const RefineGeom* __restrict__ geom, int N,
-                                                    const double* __restrict__ sc) {
-    const int e = blockIdx.y, H = N / 2 + 1;
-    const long nh = (long)N * N * H;
-    const RefineGeom g = geom[e];
-    const double S = sc[e * 4], n1 = sc[e * 4 + 1], n2 = sc[e * 4 + 2];
-    const float ca = (n1 > 0 && n2 > 0) ? (float)(1.0 / (n1 * n2)) : 0.f;
-    const float cb = n1 > 0 ? (float)(S / (n1 * n1)) : 0.f;
-    float2* x1p = X1 + (size_t)e * nh;
-    const float2* x2p = FP + (size_t)g.spec * nh;
-    for (long h = (long)blockIdx.x * kT + threadIdx.x; h < nh; h += (long)gridDim.x * kT) {
-        int a, b, c;
-        split3((unsigned)h, (unsigned)N, (unsigned)H, a, b, c);
-        const float w = refine_hweight(filter, wbin, g, h, a, b, c, N, H);
-        const float2 u = x1p[h], v = x2p[h];
-        const float w2 = w * w;
-        x1p[h] = make_float2(w2 * (ca * v.x - cb * u.x), w2 * (ca * v.y - cb * u.y));
-    }
 }
 
 // twelve moments per evaluation: per-workgroup partial sums of gamma(p) dI1/dq_a w_b(p) over kMT consecutive
@@ -380,11 +318,6 @@ int refine_moment_blocks(int N) {
     const int nt = N / kRT;
     return (nt * nt * nt + kMT - 1) / kMT;
 }
-int refine_dot_blocks(int N) {
-    const long nh = (long)N * N * (N / 2 + 1);
-    return (int)std::min<long>(64, (nh + 4 * kT - 1) / (4 * kT));
-}
-
 int vol_mean_blocks(int N) { return (int)(((long)N * N * N + kMeanV - 1) / kMeanV); }
 void launch_vol_mean(const float* vols, int count, int N, double* part, float* mean, hipStream_t s) {
     ETTK_REQUIRE(N % 4 == 0, ETTK_ERR_ARG, "launch_vol_mean: box size must be a multiple of 4");
@@ -404,24 +337,8 @@ void launch_reslice_ref(const float* ref, const RefineGeom* geom, int E, int N, 
     k_reslice_ref<<<dim3(nt * nt * nt, E), kT, 0, s>>>(ref, geom, N, out);
     ETTK_HIP(hipGetLastError());
 }
-void launch_refine_dot(const float2* X1, const float2* FP, const float* filter, const float* wbin, const RefineGeom* geom,
-                       int E, int N,
-                       double* part, double* sc, hipStream_t s) {
-    const int nb = refine_dot_blocks(N);
-    k_refine_dot<<<dim3(nb, E), kT, 0, s>>>(X1, FP, filter, wbin, geom, N, part);
-    k_refine_scalars<<<E, 64, 0, s>>>(part, nb, E, sc);
-    ETTK_HIP(hipGetLastError());
-}
 void launch_refine_scalars(const double* part, int nb, int E, double* sc, hipStream_t s) {
     k_refine_scalars<<<E, 64, 0, s>>>(part, nb, E, sc);
-    ETTK_HIP(hipGetLastError());
-}
-void launch_refine_adj(float2* X1, const float2* FP, const float* filter, const float* wbin, const RefineGeom* geom,
-                       int E, int N,
-                       const double* sc, hipStream_t s) {
-    const long nh = (long)N * N * (N / 2 + 1);
-    const int nb = (int)std::min<long>(512, (nh + 4 * kT - 1) / (4 * kT));
-    k_refine_adj<<<dim3(nb, E), kT, 0, s>>>(X1, FP, filter, wbin, geom, N, sc);
     ETTK_HIP(hipGetLastError());
 }
 void launch_refine_moments(const float* ref, const RefineGeom* geom, const float* G, const float* maskfft, int E, int N,
