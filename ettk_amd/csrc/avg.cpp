@@ -125,9 +125,9 @@ int ettk_avg_accumulate(ettk_plan* P, const float* d_particles, int n, const ett
             }
             ETTK_HIP(hipMemcpyAsync(P->geom.p, g.data(), E * sizeof(EvalGeom), hipMemcpyHostToDevice, s));
             ETTK_HIP(hipMemcpyAsync(dw.p, w.data(), E * sizeof(float), hipMemcpyHostToDevice, s));
-            launch_reslice(d_particles, P->geom.p, E, N, P->R2.p, P->p_res.p, P->nb_res, s);
+            launch_reslice(d_particles, P->geom.p, E, N, P->R.p, P->p_res.p, P->nb_res, s);
             launch_reslice_mean(P->p_res.p, P->nb_res, E, P->stats.p, s);
-            R2CArgs a{P->R2.p, P->S2.p, N, E, PRO_RESLICED, nullptr, P->stats.p};
+            R2CArgs a{P->R.p, P->S2.p, N, E, PRO_RESLICED, nullptr, P->stats.p};
             fft3_r2c(P->ctx->fft, a, nullptr, s);
             launch_avg_acc(P->S2.p, dw.p, E, nh, acc_buf(P, 0).p, acc_buf(P, 1).p, acc_buf(P, 2).p, s);
             ETTK_HIP(hipStreamSynchronize(s));
@@ -181,9 +181,9 @@ int ettk_avg_variance(ettk_plan* P, const float* d_particles, int n, const ettk_
             }
             ETTK_HIP(hipMemcpyAsync(P->geom.p, g.data(), E * sizeof(EvalGeom), hipMemcpyHostToDevice, s));
             ETTK_HIP(hipMemcpyAsync(dw.p, w.data(), E * sizeof(float), hipMemcpyHostToDevice, s));
-            launch_reslice(d_particles, P->geom.p, E, N, P->R2.p, P->p_res.p, P->nb_res, s);
+            launch_reslice(d_particles, P->geom.p, E, N, P->R.p, P->p_res.p, P->nb_res, s);
             launch_reslice_mean(P->p_res.p, P->nb_res, E, P->stats.p, s);
-            launch_var_acc(P->R2.p, P->stats.p, dw.p, E, wsum, d_average, N, var.p, s);
+            launch_var_acc(P->R.p, P->stats.p, dw.p, E, wsum, d_average, N, var.p, s);
             ETTK_HIP(hipStreamSynchronize(s));
         }
         launch_var_out(var.p, N, d_out, s);
@@ -246,9 +246,9 @@ int ettk_avg_finalize(ettk_plan* P, float* d_out) {
         hipStream_t s = P->stream;
         ensure_ccc_workspace(P, 1);
         launch_avg_final(acc_buf(P, 0).p, acc_buf(P, 1).p, acc_buf(P, 2).p, N, P->S1.p, s);
-        fft3_c2r(P->ctx->fft, P->S1.p, P->S1.p, P->R1.p, N, 1, s);
+        fft3_c2r(P->ctx->fft, P->S1.p, P->S1.p, P->R.p, N, 1, s);
         P->avg_part.ensure(avg_normalise_partials());
-        launch_avg_normalise(P->R1.p, N, P->avg_part.p, d_out, s);
+        launch_avg_normalise(P->R.p, N, P->avg_part.p, d_out, s);
         ETTK_HIP(hipStreamSynchronize(s));
     } catch (const Error& e) {
         set_error(e.msg);

@@ -214,209 +214,6 @@ void launch_wedge_overlap(const float* W1, const float* filter, const EvalGeom* 
     ETTK_HIP(hipGetLastError());
 }
 
-// ------------------------------------------------------------------ per-evaluation scalars
-__global__ void __launch_bounds__(64) k_ccc_scalars(const float* p_n1, const float* p_n2, const float* p_k1,
-                                                    const float* p_wf, int nb, int nbr, int n_eval, int N, float* scalars) {
-    const int e = blockIdx.x, l = threadIdx.x;
-    double s1 = 0, s2 = 0, k1 = 0, wf = 0;
-    for (int b = l; b < nb; b += 64) {
-        s1 += p_n1[(size_t)e * nb + b];
-        s2 += p_n2[(size_t)e * nb + b];
-        if (p_wf) wf += p_wf[(size_t)e * nb + b];
-    }
-    for (int b = l; b < nbr; b += 64) k1 += p_k1[(size_t)e * nbr + b];
-    s1 = wave_dsum(s1);
-    s2 = wave_dsum(s2);
-    k1 = wave_dsum(k1);
-    wf = wave_dsum(wf);
-    if (l != 0) return;
-    double n3 = (double)N * N * N;
-    float n1 = (float)sqrt(s1 / n3), n2 = (float)sqrt(s2 / n3);
-    scalars[e * 4 + 0] = n1;
-    scalars[e * 4 + 1] = n2;
-    scalars[e * 4 + 2] = (float)(k1 / ((double)n1 * (double)n1));  // k1_m of the normalised reference
-    scalars[e * 4 + 3] = (float)wf;
-}
-void launch_ccc_scalars(const float* p_n1, const float* p_n2, const float* p_k1, const float* p_wf, int nb,
-                        int nbr, int n_eval, int N, float* scalars, hipStream_t s) {
-    k_ccc_scalars<<<n_eval, 64, 0, s>>>(p_n1, p_n2, p_k1, p_wf, nb, nbr, n_eval, N, scalars);
-    ETTK_HIP(hipGetLastError());
-}
-
-// acc + a b as four chained FMAs (the partial DFTs' inner product)
-__device__ __forceinline__ float2 cmac(float2 acc, float2 a, float2 b) {
-    acc.x = fmaf(a.x, b.x, acc.x);
-    acc.x = fmaf(-a.y, b.y, acc.x);
-    acc.y = fmaf(a.x, b.y, acc.y);
-    acc.y = fmaf(a.y, b.x, acc.y);
-    return acc;
-}
-
-// ------------------------------------------------------------------ combine + first partial DFT (along i)
-__global__ void __launch_bounds__(kThreads) k_combine_dftA(const float2* __restrict__ F1m, const float2* __restrict__ F2,
-                                                            const float2* __restrict__ Q, const float2* __restrict__ Mfft,
-                                                            const float* __restrict__ scalars,
-                                                            const float2* __restrict__ tabA, CccSizes z,
-                                                            float2* __restrict__ G1) {
-    extern __shared__ float2 lds[];
-    const int N = z.N, H = z.H, E = z.E;
-    float2* C = lds;             // [i][k]
-    float2* A = lds + N * H;     // [x][i]
-    const int j = blockIdx.x, e = blockIdx.y;
-    const long nh = (long)N * N * H;
-    const float n1 = scalars[e * 4 + 0], n2 = scalars[e * 4 + 1];
-    const float n3 = (float)N * N * N;
-    const float a = 2.f * n3 / (n1 * n2);
-    const float b = 1.f / (n2 * n2);
-    struct Quad {
-        float2 f1, f2, q, m;
-    };
-    const float2* __restrict__ f1p = F1m + (size_t)e * nh;
-    const float2* __restrict__ f2p = F2 + (size_t)e * nh;
-    const float2* __restrict__ qp = Q + (size_t)e * nh;
-    block_copy_rt<5>(
-        N * H,
-        [&](int t) {
-            const long h = ((long)(t / H) * N + j) * H + t % H;
-            return Quad{f1p[h], f2p[h], qp[h], Mfft[h]};
-        },
-        [&](int t, const Quad& v) {
-            const int i = t / H, k = t % H;
-            float2 c = csub(cscale(cmulc(v.f1, v.f2), a), cscale(cmulc(v.m, v.q), b));
-            if ((i + j + k) & 1) c = make_float2(-c.x, -c.y);
-            C[t] = c;
-        });
-    block_copy_rt<9>(E * N, [&](int t) { return tabA[t]; }, [&](int t, float2 v) { A[t] = v; });
-    __syncthreads();
-    for (int t = threadIdx.x; t < E * H; t += blockDim.x) {
-        int x = t / H, k = t % H;
-        float2 acc = make_float2(0.f, 0.f);
-        for (int i = 0; i < N; i++) acc = cmac(acc, A[x * N + i], C[i * H + k]);
-        G1[(((size_t)e * E + x) * N + j) * H + k] = acc;
-    }
-}
-void launch_combine_dftA(const float2* F1m, const float2* F2, const float2* Q, const float2* Mfft,
-                         const float* scalars, const float2* tabA, const CccSizes& z, int n_eval, float2* G1,
-                         hipStream_t s) {
-    dim3 grid(z.N, n_eval);
-    size_t shm = (size_t)(z.N * z.H + z.E * z.N) * sizeof(float2);
-    ensure_dynamic_lds((const void*)k_combine_dftA, shm);
-    k_combine_dftA<<<grid, kThreads, shm, s>>>(F1m, F2, Q, Mfft, scalars, tabA, z, G1);
-    ETTK_HIP(hipGetLastError());
-}
-
-// ------------------------------------------------------------------ second and third partial DFTs + argmax
-__global__ void __launch_bounds__(kThreads) k_dftBC_argmax(const float2* __restrict__ G1, const float2* __restrict__ tabA,
-                                                            const float2* __restrict__ tabK, CccSizes z,
-                                                            float* __restrict__ best_val, int* __restrict__ best_idx) {
-    extern __shared__ float2 lds[];
-    const int N = z.N, H = z.H, E = z.E;
-    float2* g1 = lds;                 // [j][k]
-    float2* A = g1 + N * H;           // [y][j]
-    float2* g2 = A + E * N;           // [y][k]
-    float2* K = g2 + E * H;           // [zz][k]
-    __shared__ float sv[kThreads];
-    __shared__ int si[kThreads];
-    const int x = blockIdx.x, e = blockIdx.y;
-    const float2* src = G1 + ((size_t)e * E + x) * N * H;
-    block_copy_rt<9>(N * H, [&](int t) { return src[t]; }, [&](int t, float2 v) { g1[t] = v; });
-    block_copy_rt<9>(E * N, [&](int t) { return tabA[t]; }, [&](int t, float2 v) { A[t] = v; });
-    block_copy_rt<5>(E * H, [&](int t) { return tabK[t]; }, [&](int t, float2 v) { K[t] = v; });
-    __syncthreads();
-    for (int t = threadIdx.x; t < E * H; t += blockDim.x) {
-        int y = t / H, k = t % H;
-        float2 acc = make_float2(0.f, 0.f);
-        for (int j = 0; j < N; j++) acc = cmac(acc, A[y * N + j], g1[j * H + k]);
-        g2[t] = acc;
-    }
-    __syncthreads();
-    const float scale = 8.f / ((float)(2 * N) * (float)(2 * N) * (float)(2 * N));
-    float bv = -FLT_MAX;
-    int bi = 0x7fffffff;
-    const int dx = z.ub2 - x;
-    for (int t = threadIdx.x; t < E * E; t += blockDim.x) {
-        int y = t / E, zz = t % E;
-        int dy = z.ub2 - y, dz = z.ub2 - zz;
-        float rad = (float)(dx * dx + dy * dy + dz * dz);
-        if (!(rad < z.restr2)) continue;
-        float acc = 0.f;
-        for (int k = 0; k < H; k++) {
-            const float2 p = g2[y * H + k], q = K[zz * H + k];
-            acc = fmaf(p.x, q.x, acc);
-            acc = fmaf(-p.y, q.y, acc);
-        }
-        acc *= scale;
-        if (acc > bv || (acc == bv && t < bi)) { bv = acc; bi = t; }
-    }
-    sv[threadIdx.x] = bv;
-    si[threadIdx.x] = bi;
-    __syncthreads();
-    for (int st = blockDim.x / 2; st > 0; st >>= 1) {
-        if (threadIdx.x < st) {
-            float v2 = sv[threadIdx.x + st];
-            int i2 = si[threadIdx.x + st];
-            if (v2 > sv[threadIdx.x] || (v2 == sv[threadIdx.x] && i2 < si[threadIdx.x])) {
-                sv[threadIdx.x] = v2;
-                si[threadIdx.x] = i2;
-            }
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        best_val[(size_t)e * E + x] = sv[0];
-        best_idx[(size_t)e * E + x] = si[0];
-    }
-}
-void launch_dftBC_argmax(const float2* G1, const float2* tabA, const float2* tabK, const CccSizes& z, int n_eval,
-                         float* best_val, int* best_idx, hipStream_t s) {
-    dim3 grid(z.E, n_eval);
-    size_t shm = (size_t)(z.N * z.H + z.E * z.N + 2 * z.E * z.H) * sizeof(float2);
-    ensure_dynamic_lds((const void*)k_dftBC_argmax, shm);
-    k_dftBC_argmax<<<grid, kThreads, shm, s>>>(G1, tabA, tabK, z, best_val, best_idx);
-    ETTK_HIP(hipGetLastError());
-}
-
-// ------------------------------------------------------------------ final reduction per evaluation
-__global__ void k_peak_final(const float* __restrict__ best_val, const int* __restrict__ best_idx,
-                             const float* __restrict__ scalars, float sum_filter, int overlap, CccSizes z, int n_eval,
-                             float* __restrict__ out) {
-    int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n_eval) return;
-    const int E = z.E;
-    float bv = -FLT_MAX;
-    int bx = -1, byz = 0;
-    for (int x = 0; x < E; x++) {
-        float v = best_val[(size_t)e * E + x];
-        int id = best_idx[(size_t)e * E + x];
-        if (id == 0x7fffffff) continue;
-        if (bx < 0 || v > bv) { bv = v; bx = x; byz = id; }
-    }
-    float px = 0.f, py = 0.f, pz = 0.f;
-    double maxT = -(double)FLT_MAX;
-    if (bx >= 0) {
-        px = (float)bx;
-        py = (float)(byz / E);
-        pz = (float)(byz % E);
-        maxT = bv;
-    }
-    const float k1m = scalars[e * 4 + 2], wf = scalars[e * 4 + 3];
-    double peak = fmax(0.0, (double)k1m - maxT);
-    if (overlap) peak = peak / (double)wf * (double)sum_filter;
-    float cp = (float)peak;
-    double big = (double)(2 * z.N) * (2 * z.N) * (2 * z.N);
-    cp = (float)((double)cp / big / big);
-    float c = (E - 1) / 2.0f;
-    out[e * 4 + 0] = cp;
-    out[e * 4 + 1] = (px - c) / 2.0f;
-    out[e * 4 + 2] = (py - c) / 2.0f;
-    out[e * 4 + 3] = (pz - c) / 2.0f;
-}
-void launch_peak_final(const float* best_val, const int* best_idx, const float* scalars, float sum_filter,
-                       int overlap, const CccSizes& z, int n_eval, float* out, hipStream_t s) {
-    k_peak_final<<<(n_eval + 127) / 128, 128, 0, s>>>(best_val, best_idx, scalars, sum_filter, overlap, z, n_eval, out);
-    ETTK_HIP(hipGetLastError());
-}
-
 template <class T>
 __global__ void k_fill_zero(T* __restrict__ p, size_t n) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = T(0);

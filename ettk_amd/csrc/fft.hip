@@ -722,11 +722,17 @@ __global__ void __launch_bounds__(Plane<L>::THREADS) k_c2r_plane(const float2* _
 // through HBM.  `io` holds the half spectrum after the inverse i pass and receives the forward j/k passes.
 //   PLANE_OP_MASK:          r <- r m (m = aux, N^3), partials[plane] = sum r^2 m over the plane
 //   PLANE_OP_SQUARE_SHIFT:  r <- r^2 (-1)^(i+j+k)
+// One launch runs one or two batches of `planes` planes, each with its operation: the CCC's two sides together fill the
+// chip where one evaluation's N planes would not.
+struct PlaneOps {
+    float2 *io0, *io1;
+    int op0, op1;
+    unsigned planes;
+    const float* mask;  // PLANE_OP_MASK
+    float* partials;    // PLANE_OP_MASK
+};
 template <int L>
-__global__ void __launch_bounds__(Plane<L>::THREADS) k_c2r_r2c_plane(float2* __restrict__ io, int op,
-                                                                       const float* __restrict__ aux,
-                                                                       float* __restrict__ partials,
-                                                                       const float2* __restrict__ twg) {
+__global__ void __launch_bounds__(Plane<L>::THREADS) k_c2r_r2c_plane(PlaneOps a, const float2* __restrict__ twg) {
     using PL = Plane<L>;
     constexpr int H = PL::H, LD = PL::LD, T = PL::THREADS;
     constexpr int NZ = ((L / 2) * L + T - 1) / T;
@@ -735,10 +741,14 @@ __global__ void __launch_bounds__(Plane<L>::THREADS) k_c2r_r2c_plane(float2* __r
     __shared__ float2 buf[H * LD];
     __shared__ float2 tw[L];
     __shared__ float sred[NFW + REM + 1];
-    const long plane = blockIdx.x;
+    const bool second = blockIdx.x >= a.planes;
+    const long plane = second ? blockIdx.x - a.planes : blockIdx.x;
+    const int op = second ? a.op1 : a.op0;
+    const float* __restrict__ aux = a.mask;
+    float* __restrict__ partials = a.partials;
     const int pi = (int)(plane % L);
     const float2 twv = twg[threadIdx.x % L];  // stored after the staging loads are in flight
-    float2* ip = io + plane * L * H;
+    float2* ip = (second ? a.io1 : a.io0) + plane * L * H;
     block_copy<T, L * H>([&](int t) { return ip[t]; }, [&](int t, float2 v) { buf[(t % H) * LD + t / H] = v; });
     if (threadIdx.x < L) tw[threadIdx.x] = twv;
     __syncthreads();
@@ -831,193 +841,289 @@ __global__ void __launch_bounds__(Plane<L>::THREADS) k_c2r_r2c_plane(float2* __r
     for (int t = threadIdx.x; t < L * H; t += blockDim.x) ip[t] = r2c_half_at<L>(buf, t / H, t % H);
 }
 
-// ------------------------------------------------------------------ combine + first DFT axis by FFT (N = 64)
-// The first axis of the zero-padded 2N-point inverse transform on the search window (k_combine_dftA's table
-// A[x][i] = (-1)^f e^{+i pi f u / N}, f = i - N/2, u = I0 + x - N) as two length-N FFTs per pencil: with
-// u = 2m + b, G(u) = sum_f [(-1)^f C(f) e^{+2 pi i f b / 2N}] e^{+2 pi i f m / N}, a backward N-point transform of
-// the twiddled pencil (f periodic mod N) for each parity b, read at m mod N.  One workgroup per (j, evaluation):
-// 2H pencils (k, b) of 8 threads, each a length-64 register FFT.
-// FWD: F1m and Q arrive before their forward i transform (the fused plane kernels' outputs); the workgroup runs
-// those transforms on its 2H pencils first.
-static constexpr int kCfP = 2 * 33, kCfT = kCfP * 8;
-template <bool FWD>
-__global__ void __launch_bounds__(kCfT) k_combine_fftA(const float2* __restrict__ F1m, const float2* __restrict__ F2,
-                                                       const float2* __restrict__ Q, const float2* __restrict__ Mfft,
-                                                       const float* __restrict__ scalars, CccSizes z,
-                                                       float2* __restrict__ G1, const float2* __restrict__ tw64,
-                                                       const float2* __restrict__ tw128) {
-    constexpr int L = 64, H = L / 2 + 1, LD = PenT<64>::LD, NE = (L * H + kCfT - 1) / kCfT;
-    static_assert(L * H == NE * kCfT, "four elements per thread");
-    __shared__ float2 pens[kCfP * LD];
+// ------------------------------------------------------------------ combine + first DFT axis by FFT
+// norms of both sides of evaluation e from the i pass's partials, in the lanes of one wavefront (FP64, a fixed order)
+__device__ __forceinline__ double wave_xsum(double v) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+__device__ __forceinline__ float ccc_norm(const float* __restrict__ part, int nb, int e, double n3) {
+    double s = 0;
+    for (int b = threadIdx.x & 63; b < nb; b += 64) s += part[(size_t)e * nb + b];
+    return (float)sqrt(wave_xsum(s) / n3);
+}
+
+// e^{+2 pi i (i - L/2) / 2L} for i = 0 .. L-1 from the forward twiddles of length 2L
+template <int L>
+__device__ __forceinline__ float2 half_step(const float2* __restrict__ tw2, int i) {
+    return cconj(tw2[(i - L / 2 + 2 * L) % (2 * L)]);
+}
+// Window index (from u = I0 - L) of element n of the parity-par transform: n stands for m = n or n - L, u = 2m + par
+template <int L>
+__device__ __forceinline__ int window_at(int n, int par, int I0) {
+    return 2 * (n < L / 2 ? n : n - L) + par - (I0 - L);
+}
+
+// The first axis of the zero-padded 2L-point inverse transform on the search window, A[x][i] = (-1)^f e^{+i pi f u / L},
+// f = i - L/2, u = I0 + x - L, as two length-L FFTs per pencil: with u = 2m + b,
+// G(u) = sum_f [(-1)^f C(f) e^{+2 pi i f b / 2L}] e^{+2 pi i f m / L}, a backward L-point transform of the twiddled
+// pencil (f periodic mod L) for each parity b, read at m mod L.  F1m and Q arrive before their forward i transform
+// (the fused plane kernels' outputs), which runs here first.  A workgroup holds P pencils (j, k) of one evaluation in
+// registers through all four transforms (regfft.hpp); rows of P neighbouring pencils of every array are whole cache
+// lines.  Bound by HBM (3H read, the window's rows written): 240 evaluations at 64^3 take 148 us (6.1 TB/s), where a
+// workgroup per (j, evaluation) with its 66 pencils staged in LDS took 305; 36 at 128^3 take 219 us, where the table
+// product (an LDS-resident plane and table: one workgroup of 4 waves per CU) took 861.
+template <int L>
+__global__ void __launch_bounds__(ColShape<L>::THREADS) k_ccc_combine(const float2* __restrict__ F1m, const float2* __restrict__ F2,
+                                                                  const float2* __restrict__ Q, const float2* __restrict__ Mfft,
+                                                                  const float* __restrict__ p_n1, const float* __restrict__ p_n2,
+                                                                  int nb, CccSizes z, float2* __restrict__ G1,
+                                                                  const float2* __restrict__ twg, const float2* __restrict__ tw2) {
+    using S = ColShape<L>;
+    constexpr int H = L / 2 + 1, LH = L * H, NE = S::E, T = S::T, HS = L / 2 / T;  // HS: half the pencil in slots
+    __shared__ float2 ex[L * S::P];
     __shared__ float2 tw[L];
-    __shared__ float2 wb[L];  // e^{+2 pi i (i - L/2) / 2L} for i = 0 .. L-1
-    // the j planes of one evaluation on one XCD: a plane's rows of 33 complex values are not aligned to cache
-    // lines, and the lines they share with the neighbouring planes are then fetched into one L2 only
-    int j, e;
-    xcd_eval_tile(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, e, j);
-    const int E = z.E;
-    const long nh = (long)L * L * H;
-    if (threadIdx.x < L) {
-        tw[threadIdx.x] = tw64[threadIdx.x];
-        wb[threadIdx.x] = cconj(tw128[(threadIdx.x - L / 2 + 2 * L) % (2 * L)]);
-    }
-    const float n1 = scalars[e * 4 + 0], n2 = scalars[e * 4 + 1];
-    const float n3 = (float)L * L * L;
-    const float a = 2.f * n3 / (n1 * n2);
-    const float b = 1.f / (n2 * n2);
-    const float2* __restrict__ f1p = F1m + (size_t)e * nh;
-    const float2* __restrict__ f2p = F2 + (size_t)e * nh;
-    const float2* __restrict__ qp = Q + (size_t)e * nh;
-    const int q = threadIdx.x >> 3, lane = threadIdx.x & 7;
-    // this thread's elements t = threadIdx.x + u kCfT of the (i, k) plane
-    float2 c0[NE], c1[NE];
-    if constexpr (FWD) {
-        {
-            float2 vf1[NE], vq[NE];
-#pragma unroll
-            for (int u = 0; u < NE; u++) {
-                const int t = threadIdx.x + u * kCfT;
-                const long h = ((long)(t / H) * L + j) * H + t % H;
-                vf1[u] = ld_stream(&f1p[h]);
-                vq[u] = ld_stream(&qp[h]);
-            }
-#pragma unroll
-            for (int u = 0; u < NE; u++) {
-                const int t = threadIdx.x + u * kCfT, i = t / H, k = t % H;
-                pens[k * LD + i] = vf1[u];
-                pens[(H + k) * LD + i] = vq[u];
-            }
-        }
-        __syncthreads();
-        fft64_reg(&pens[q * LD], lane, tw_cache<64>(tw, lane), false);  // F1m and Q along i
-        float2 vf2[NE], vm[NE];  // loaded after the transforms: fewer registers held across them
-#pragma unroll
-        for (int u = 0; u < NE; u++) {
-            const int t = threadIdx.x + u * kCfT;
-            const long h = ((long)(t / H) * L + j) * H + t % H;
-            vf2[u] = ld_stream(&f2p[h]);
-            vm[u] = Mfft[h];
-        }
-#pragma unroll
-        for (int u = 0; u < NE; u++) {
-            const int t = threadIdx.x + u * kCfT, i = t / H, k = t % H;
-            float2 c = csub(cscale(cmulc(pens[k * LD + i], vf2[u]), a), cscale(cmulc(vm[u], pens[(H + k) * LD + i]), b));
-            if ((i + j + k) & 1) c = make_float2(-c.x, -c.y);
-            if ((i - L / 2) & 1) c = make_float2(-c.x, -c.y);  // (-1)^f of the table
-            c0[u] = c;
-            c1[u] = cmul(c, wb[i]);
-        }
-        __syncthreads();
-    } else {
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < NE; u++) {
-            const int t = threadIdx.x + u * kCfT;
-            const long h = ((long)(t / H) * L + j) * H + t % H;
-            const float2 f1 = ld_stream(&f1p[h]), f2 = ld_stream(&f2p[h]), qv = ld_stream(&qp[h]), m = Mfft[h];
-            const int i = t / H, k = t % H;
-            float2 c = csub(cscale(cmulc(f1, f2), a), cscale(cmulc(m, qv), b));
-            if ((i + j + k) & 1) c = make_float2(-c.x, -c.y);
-            if ((i - L / 2) & 1) c = make_float2(-c.x, -c.y);
-            c0[u] = c;
-            c1[u] = cmul(c, wb[i]);
-        }
-    }
+    __shared__ float2 wb[L];
+    __shared__ float sn[2];
+    const int e = blockIdx.y, t = threadIdx.x / S::P;
+    const int p = blockIdx.x * S::P + threadIdx.x % S::P;  // pencil (j, k) = (p / H, p % H)
+    const bool valid = p < LH;
+    const int pc = valid ? p : 0;
+    const size_t vol = (size_t)e * L * LH + pc;
+    float2* __restrict__ xp = ex + threadIdx.x % S::P;
+    float2 f1[NE], q[NE];
 #pragma unroll
     for (int u = 0; u < NE; u++) {
-        const int t = threadIdx.x + u * kCfT, i = t / H, k = t % H;
-        const int n = (i + L / 2) & (L - 1);  // f mod L
-        pens[k * LD + n] = c0[u];
-        pens[(H + k) * LD + n] = c1[u];
+        const size_t h = vol + (size_t)(t + u * T) * LH;
+        f1[u] = ld_stream(&F1m[h]);
+        q[u] = ld_stream(&Q[h]);
+    }
+    for (int i = threadIdx.x; i < L; i += S::THREADS) {
+        tw[i] = twg[i];
+        wb[i] = half_step<L>(tw2, i);
+    }
+    if (threadIdx.x < 128) {
+        const float n = ccc_norm(threadIdx.x < 64 ? p_n1 : p_n2, nb, e, (double)L * L * L);
+        if ((threadIdx.x & 63) == 0) sn[threadIdx.x >> 6] = n;
     }
     __syncthreads();
-    fft64_reg(&pens[q * LD], lane, tw_cache<64>(tw, lane), true);
-    const int u0 = z.I0 - L;
-    for (int t = threadIdx.x; t < E * H; t += kCfT) {
-        const int x = t / H, k = t % H, u = u0 + x, par = u & 1, m = ((u - par) / 2) & (L - 1);
-        G1[(((size_t)e * E + x) * L + j) * H + k] = pens[(par * H + k) * LD + m];
+    col_fft<L, false>(f1, t, xp, tw);
+    col_fft<L, false>(q, t, xp, tw);
+    // C = (-M conj(Q)/n2^2 + 2 F1m/n1 conj(F2 N^3/n2)) (-1)^(i+j+k), times (-1)^f: i cancels
+    const float n1 = sn[0], n2 = sn[1];
+    const float sg = ((pc / H + pc % H + L / 2) & 1) ? -1.f : 1.f;
+    const float a = sg * (2.f * (float)(L * L * L) / (n1 * n2)), b = sg / (n2 * n2);
+#pragma unroll
+    for (int u = 0; u < NE; u++) {
+        const size_t i = t + u * T;
+        const float2 f2 = ld_stream(&F2[vol + i * LH]), m = Mfft[i * LH + pc];
+        f1[u] = csub(cscale(cmulc(f1[u], f2), a), cscale(cmulc(m, q[u]), b));
+        q[u] = cmul(f1[u], wb[i]);
+    }
+    // element f mod L = i + L/2 mod L: a rotation of the slots by HS
+#pragma unroll
+    for (int par = 0; par < 2; par++) {
+        float2 x[NE];
+#pragma unroll
+        for (int u = 0; u < NE; u++) x[(u + HS) % NE] = par ? q[u] : f1[u];
+        col_fft<L, true>(x, t, xp, tw);
+        if (valid)
+#pragma unroll
+            for (int u = 0; u < NE; u++) {
+                const int xi = window_at<L>(t + u * T, par, z.I0);
+                if (xi >= 0 && xi < z.E) G1[((size_t)e * z.E + xi) * LH + p] = x[u];
+            }
     }
 }
 
-// The second axis the same way (k_dftBC_argmax's A along j), then the third axis on the crop, the spherical mask
-// and the first maximum as k_dftBC_argmax computes them.  One workgroup per (x, evaluation).
-__global__ void __launch_bounds__(kCfT) k_dftBC_fft(const float2* __restrict__ G1, const float2* __restrict__ tabK,
-                                                    CccSizes z, float* __restrict__ best_val, int* __restrict__ best_idx,
-                                                    const float2* __restrict__ tw64, const float2* __restrict__ tw128) {
-    constexpr int L = 64, H = L / 2 + 1, LD = PenT<64>::LD;
-    extern __shared__ float2 K[];  // [zz][k], E x H
-    __shared__ float2 pens[kCfP * LD];
+// The second axis the same way on the pencils along j of one (x, evaluation), in rounds of P columns k; then the third
+// axis on the crop, T = sum_k Re(G2(y, k) K(z, k)) as 3 x 3 register tiles of (y, z), the spherical mask and the first
+// maximum (value descending, then index ascending).  The tiles read 6 values for 9 outputs from LDS instead of 18: 93 us
+// for 240 evaluations at 64^3 against 171, 71 us for 36 at 128^3 against 219 with the second axis as a table product.
+template <int L> struct BcShape {
+    static constexpr int H = L / 2 + 1;
+    static constexpr int ROUNDS = L == 128 ? 2 : 1;  // at 128 all columns' exchange (67 KB) would leave one workgroup per CU
+    static constexpr int P = (H + ROUNDS - 1) / ROUNDS;
+    static constexpr int T = ColShape<L>::T;
+    static constexpr int THREADS = (P * T + 63) / 64 * 64;
+};
+template <int L>
+__global__ void __launch_bounds__(BcShape<L>::THREADS) k_ccc_dftBC(const float2* __restrict__ G1, const float2* __restrict__ tabK,
+                                                               CccSizes z, float* __restrict__ best_val, int* __restrict__ best_idx,
+                                                               const float2* __restrict__ twg, const float2* __restrict__ tw2) {
+    using B = BcShape<L>;
+    constexpr int H = B::H, P = B::P, T = B::T, NE = L / T, HS = L / 2 / T, NT = B::THREADS;
+    extern __shared__ float2 dyn[];  // G2 [y][k], then K [zz][k], each E x H
+    __shared__ float2 ex[L * P];
     __shared__ float2 tw[L];
     __shared__ float2 wb[L];
-    __shared__ float sv[kCfT];
-    __shared__ int si[kCfT];
-    const int x = blockIdx.x, e = blockIdx.y, E = z.E;
-    if (threadIdx.x < L) {
-        tw[threadIdx.x] = tw64[threadIdx.x];
-        wb[threadIdx.x] = cconj(tw128[(threadIdx.x - L / 2 + 2 * L) % (2 * L)]);
+    __shared__ float sv[NT / 64];
+    __shared__ int si[NT / 64];
+    const int xi = blockIdx.x, e = blockIdx.y, E = z.E;
+    float2 *g2 = dyn, *K = dyn + (size_t)E * H;
+    const int t = threadIdx.x / P, c = threadIdx.x % P;
+    const float2* __restrict__ src = G1 + ((size_t)e * E + xi) * L * H;  // [j][k]
+#pragma unroll
+    for (int r = 0; r < B::ROUNDS; r++) {
+        const int k = r * P + c;
+        const bool live = t < T && k < H;
+        float2 v[NE];
+#pragma unroll
+        for (int u = 0; u < NE; u++) v[u] = live ? src[(t + u * T) * H + k] : make_float2(0.f, 0.f);
+        if (r == 0) {
+            for (int i = threadIdx.x; i < L; i += NT) {
+                tw[i] = twg[i];
+                wb[i] = half_step<L>(tw2, i);
+            }
+            block_copy_rt<4>(E * H, [&](int q) { return tabK[q]; }, [&](int q, float2 w) { K[q] = w; });
+            __syncthreads();
+        }
+        const float sg = ((t + L / 2) & 1) ? -1.f : 1.f;  // (-1)^f of the table: T is even, so it is the thread's
+#pragma unroll
+        for (int par = 0; par < 2; par++) {
+            float2 x[NE];
+#pragma unroll
+            for (int u = 0; u < NE; u++) {
+                const float2 w = cscale(v[u], sg);
+                x[(u + HS) % NE] = par && live ? cmul(w, wb[t + u * T]) : w;
+            }
+            col_fft<L, true, P>(x, t, ex + c, tw, live);
+            if (live)
+#pragma unroll
+                for (int u = 0; u < NE; u++) {
+                    const int y = window_at<L>(t + u * T, par, z.I0);
+                    if (y >= 0 && y < E) g2[y * H + k] = x[u];
+                }
+        }
     }
     __syncthreads();
-    const float2* src = G1 + ((size_t)e * E + x) * L * H;  // [j][k]
-    block_copy_rt<4>(
-        L * H, [&](int t) { return src[t]; },
-        [&](int t, float2 c) {
-            const int jj = t / H, k = t % H;
-            if ((jj - L / 2) & 1) c = make_float2(-c.x, -c.y);
-            const int n = (jj + L / 2) & (L - 1);
-            pens[k * LD + n] = c;
-            pens[(H + k) * LD + n] = cmul(c, wb[jj]);
-        });
-    block_copy_rt<3>(E * H, [&](int t) { return tabK[t]; }, [&](int t, float2 v) { K[t] = v; });
-    __syncthreads();
-    const int q = threadIdx.x >> 3, lane = threadIdx.x & 7;
-    fft64_reg(&pens[q * LD], lane, tw_cache<64>(tw, lane), true);
-    // g2(y, k) = pens[(par H + k) LD + m] with u = I0 + y - L = 2m + par
     const float scale = 8.f / ((float)(2 * L) * (float)(2 * L) * (float)(2 * L));
     float bv = -FLT_MAX;
     int bi = 0x7fffffff;
-    const int dx = z.ub2 - x, u0 = z.I0 - L;
-    for (int t = threadIdx.x; t < E * E; t += kCfT) {
-        const int y = t / E, zz = t % E;
-        const int dy = z.ub2 - y, dz = z.ub2 - zz;
-        const float rad = (float)(dx * dx + dy * dy + dz * dz);
-        if (!(rad < z.restr2)) continue;
-        const int u = u0 + y, par = u & 1, m = ((u - par) / 2) & (L - 1);
-        const float2* gy = &pens[par * H * LD + m];
-        float acc = 0.f;
-        for (int k = 0; k < H; k++) {
-            const float2 p = gy[k * LD], qv = K[zz * H + k];
-            acc = fmaf(p.x, qv.x, acc);
-            acc = fmaf(-p.y, qv.y, acc);
-        }
-        acc *= scale;
-        if (acc > bv || (acc == bv && t < bi)) {
-            bv = acc;
-            bi = t;
-        }
-    }
-    // first maximum over the workgroup (value descending, then index ascending: a total order, so the halving
-    // tree over any count gives the same result as a scan)
-    sv[threadIdx.x] = bv;
-    si[threadIdx.x] = bi;
-    __syncthreads();
-    for (int cnt = kCfT; cnt > 1;) {
-        const int st = (cnt + 1) / 2;
-        if ((int)threadIdx.x < cnt - st) {
-            const int r = threadIdx.x;
-            const float v2 = sv[r + st];
-            const int i2 = si[r + st];
-            if (v2 > sv[r] || (v2 == sv[r] && i2 < si[r])) {
-                sv[r] = v2;
-                si[r] = i2;
+    const int dx = z.ub2 - xi, nt = (E + 2) / 3;
+    for (int q = threadIdx.x; q < nt * nt; q += NT) {
+        const int y0 = 3 * (q / nt), z0 = 3 * (q % nt);
+        const float2 *gp[3], *kp[3];
+        bool any = false;
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            gp[r] = g2 + min(y0 + r, E - 1) * H;
+            kp[r] = K + min(z0 + r, E - 1) * H;
+#pragma unroll
+            for (int w = 0; w < 3; w++) {
+                const int dy = z.ub2 - (y0 + r), dz = z.ub2 - (z0 + w);
+                any = any || (float)(dx * dx + dy * dy + dz * dz) < z.restr2;
             }
         }
-        __syncthreads();
-        cnt = st;
+        if (!any) continue;
+        float acc[3][3] = {};
+#pragma unroll 2
+        for (int k = 0; k < H; k++) {
+            float2 g[3], w[3];
+#pragma unroll
+            for (int r = 0; r < 3; r++) {
+                g[r] = gp[r][k];
+                w[r] = kp[r][k];
+            }
+#pragma unroll
+            for (int r = 0; r < 3; r++)
+#pragma unroll
+                for (int s = 0; s < 3; s++) {
+                    acc[r][s] = fmaf(g[r].x, w[s].x, acc[r][s]);
+                    acc[r][s] = fmaf(-g[r].y, w[s].y, acc[r][s]);
+                }
+        }
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+#pragma unroll
+            for (int s = 0; s < 3; s++) {
+                const int y = y0 + r, zz = z0 + s, dy = z.ub2 - y, dz = z.ub2 - zz, id = y * E + zz;
+                if (y >= E || zz >= E || !((float)(dx * dx + dy * dy + dz * dz) < z.restr2)) continue;
+                const float val = acc[r][s] * scale;
+                if (val > bv || (val == bv && id < bi)) {
+                    bv = val;
+                    bi = id;
+                }
+            }
     }
+    for (int o = 32; o > 0; o >>= 1) {
+        const float v2 = __shfl_xor(bv, o, 64);
+        const int i2 = __shfl_xor(bi, o, 64);
+        if (v2 > bv || (v2 == bv && i2 < bi)) {
+            bv = v2;
+            bi = i2;
+        }
+    }
+    if ((threadIdx.x & 63) == 0) {
+        sv[threadIdx.x >> 6] = bv;
+        si[threadIdx.x >> 6] = bi;
+    }
+    __syncthreads();
     if (threadIdx.x == 0) {
-        best_val[(size_t)e * E + x] = sv[0];
-        best_idx[(size_t)e * E + x] = si[0];
+        for (int w = 1; w < NT / 64; w++)
+            if (sv[w] > bv || (sv[w] == bv && si[w] < bi)) {
+                bv = sv[w];
+                bi = si[w];
+            }
+        best_val[(size_t)e * E + xi] = bv;
+        best_idx[(size_t)e * E + xi] = bi;
     }
+}
+
+// One wavefront per evaluation: the first maximum over x, then k1_m and sum(W filter) from their partials, the
+// distance and the shift (FIM.h:1249-1322)
+__global__ void __launch_bounds__(64) k_peak_final(const float* __restrict__ best_val, const int* __restrict__ best_idx,
+                                                   const float* __restrict__ p_n1, const float* __restrict__ p_wf, int nb,
+                                                   const float* __restrict__ p_k1, float sum_filter, int overlap, CccSizes z,
+                                                   float* __restrict__ out) {
+    const int e = blockIdx.x, l = threadIdx.x, E = z.E;
+    const double n3 = (double)z.N * z.N * z.N;
+    const float n1 = ccc_norm(p_n1, nb, e, n3);
+    double wf = 0, k1 = 0;
+    for (int b = l; b < nb; b += 64) wf += p_wf[(size_t)e * nb + b];
+    for (int b = l; b < z.N; b += 64) k1 += p_k1[(size_t)e * z.N + b];
+    wf = wave_xsum(wf);
+    k1 = wave_xsum(k1);
+    float bv = -FLT_MAX;
+    int bx = 0x7fffffff, byz = 0x7fffffff;  // byz 0x7fffffff: nothing inside the mask
+    for (int x = l; x < E; x += 64) {
+        const float v = best_val[(size_t)e * E + x];
+        const int id = best_idx[(size_t)e * E + x];
+        if (id != 0x7fffffff && (byz == 0x7fffffff || v > bv)) {
+            bv = v;
+            bx = x;
+            byz = id;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        const float v2 = __shfl_xor(bv, o, 64);
+        const int x2 = __shfl_xor(bx, o, 64), id2 = __shfl_xor(byz, o, 64);
+        if (id2 != 0x7fffffff && (byz == 0x7fffffff || v2 > bv || (v2 == bv && x2 < bx))) {
+            bv = v2;
+            bx = x2;
+            byz = id2;
+        }
+    }
+    if (l != 0) return;
+    float px = 0.f, py = 0.f, pz = 0.f;
+    double maxT = -(double)FLT_MAX;
+    if (byz != 0x7fffffff) {
+        px = (float)bx;
+        py = (float)(byz / E);
+        pz = (float)(byz % E);
+        maxT = bv;
+    }
+    const float k1m = (float)(k1 / ((double)n1 * (double)n1));  // k1_m of the normalised reference
+    double peak = fmax(0.0, (double)k1m - maxT);
+    if (overlap) peak = peak / (double)(float)wf * (double)sum_filter;
+    float cp = (float)peak;
+    const double big = (double)(2 * z.N) * (2 * z.N) * (2 * z.N);
+    cp = (float)((double)cp / big / big);
+    const float c = (E - 1) / 2.0f;
+    out[e * 4 + 0] = cp;
+    out[e * 4 + 1] = (px - c) / 2.0f;
+    out[e * 4 + 2] = (py - c) / 2.0f;
+    out[e * 4 + 3] = (pz - c) / 2.0f;
 }
 
 // ------------------------------------------------------------------ host launchers
@@ -1111,48 +1217,60 @@ static void launch_c2r(const FftTables& T, const float2* in, float2* tmp, float*
 }
 
 template <int L>
+static void launch_planes(const FftTables& T, const PlaneOps& a, hipStream_t s) {
+    const float2* tw = T.tw.p + T.offset[fft_len_index(L)];
+    const unsigned nb = a.planes * (a.io1 ? 2 : 1);
+    static const std::string name = "k_c2r_r2c_plane<" + std::to_string(L) + ">";
+    ProfScope ps(T.prof, name.c_str(), 2.0 * nb * L * (L / 2 + 1) * sizeof(float2), s);
+    k_c2r_r2c_plane<L><<<nb, Plane<L>::THREADS, 0, s>>>(a, tw);
+}
+template <int L>
 static void launch_c2r_op_r2c(const FftTables& T, const float2* in, float2* io, int batch, int op, const float* aux,
-                              float* partials, hipStream_t s, bool fwd_i = true) {
+                              float* partials, hipStream_t s) {
     constexpr int H = L / 2 + 1;
     const float2* tw = T.tw.p + T.offset[fft_len_index(L)];
     const double vol_c = (double)batch * L * L * H * sizeof(float2);
-    StridedArgs si{in, io, (long)batch * L * H, (long)L * H, (long)L * L * H, (long)L * H, 1};
-    if (in) {
+    const StridedArgs si{in, io, (long)batch * L * H, (long)L * H, (long)L * L * H, (long)L * H, 1};
+    {
         ProfScope ps(T.prof, prof_name<L>(1), 2 * vol_c, s);
         launch_strided<L>(si, tw, s);
     }
-    {
-        static const std::string name = "k_c2r_r2c_plane<" + std::to_string(L) + ">";
-        ProfScope ps(T.prof, name.c_str(), 2 * vol_c, s);
-        k_c2r_r2c_plane<L><<<(unsigned)((long)batch * L), Plane<L>::THREADS, 0, s>>>(io, op, aux, partials, tw);
-    }
-    StridedArgs sf{io, io, (long)batch * L * H, (long)L * H, (long)L * L * H, (long)L * H, 0};
-    if (fwd_i) {
-        ProfScope ps(T.prof, prof_name<L>(1), 2 * vol_c, s);
-        launch_strided<L>(sf, tw, s);
-    }
+    launch_planes<L>(T, PlaneOps{io, nullptr, op, op, (unsigned)(batch * L), aux, partials}, s);
+    const StridedArgs sf{io, io, (long)batch * L * H, (long)L * H, (long)L * L * H, (long)L * H, 0};
+    ProfScope ps(T.prof, prof_name<L>(1), 2 * vol_c, s);
+    launch_strided<L>(sf, tw, s);
 }
 
-bool ccc_combine_fft_supported(const CccSizes& z) { return z.N == 64; }
-void launch_dftBC_fft(const FftTables& T, const float2* G1, const float2* tabK, const CccSizes& z, int n_eval,
-                      float* best_val, int* best_idx, hipStream_t s) {
-    ETTK_REQUIRE(ccc_combine_fft_supported(z), ETTK_ERR_UNSUPPORTED, "launch_dftBC_fft: box size must be 64");
-    const float2* tw64 = T.tw.p + T.offset[fft_len_index(64)];
-    const float2* tw128 = T.tw.p + T.offset[fft_len_index(128)];
-    const size_t shm = (size_t)z.E * z.H * sizeof(float2);
-    ensure_dynamic_lds((const void*)k_dftBC_fft, shm);
-    k_dftBC_fft<<<dim3(z.E, n_eval), kCfT, shm, s>>>(G1, tabK, z, best_val, best_idx, tw64, tw128);
-    ETTK_HIP(hipGetLastError());
+template <int L>
+static void launch_ccc_tail(const FftTables& T, const CccTailArgs& a, hipStream_t s) {
+    constexpr int H = L / 2 + 1;
+    const float2 *tw = T.tw.p + T.offset[fft_len_index(L)], *tw2 = T.tw.p + T.offset[fft_len_index(2 * L)];
+    const int nb = fft3_ccc_ipass_blocks(L), E = a.z.E;
+    const double Hb = (double)a.batch * L * L * H * sizeof(float2), Gb = (double)a.batch * E * L * H * sizeof(float2);
+    launch_planes<L>(T, PlaneOps{a.S1, a.S3, PLANE_OP_MASK, PLANE_OP_SQUARE_SHIFT, (unsigned)(a.batch * L), a.m1, a.p_k1}, s);
+    {
+        ProfScope ps(T.prof, "k_ccc_combine", 3 * Hb + Gb, s);
+        k_ccc_combine<L><<<dim3((L * H + ColShape<L>::P - 1) / ColShape<L>::P, a.batch), ColShape<L>::THREADS, 0, s>>>(
+            a.S1, a.S2, a.S3, a.Mfft, a.p_n1, a.p_n2, nb, a.z, a.G1, tw, tw2);
+    }
+    {
+        ProfScope ps(T.prof, "k_ccc_dftBC", Gb, s);
+        const size_t shm = (size_t)2 * E * H * sizeof(float2);
+        ensure_dynamic_lds((const void*)k_ccc_dftBC<L>, shm);
+        k_ccc_dftBC<L><<<dim3(E, a.batch), BcShape<L>::THREADS, shm, s>>>(a.G1, a.tabK, a.z, a.bval, a.bidx, tw, tw2);
+    }
+    k_peak_final<<<a.batch, 64, 0, s>>>(a.bval, a.bidx, a.p_n1, a.p_wf, nb, a.p_k1, a.sum_filter, a.overlap, a.z, a.out4);
 }
-void launch_combine_fftA(const FftTables& T, const float2* F1m, const float2* F2, const float2* Q, const float2* Mfft,
-                         const float* scalars, const CccSizes& z, int n_eval, float2* G1, bool forward_i, hipStream_t s) {
-    ETTK_REQUIRE(ccc_combine_fft_supported(z), ETTK_ERR_UNSUPPORTED, "launch_combine_fftA: box size must be 64");
-    const float2* tw64 = T.tw.p + T.offset[fft_len_index(64)];
-    const float2* tw128 = T.tw.p + T.offset[fft_len_index(128)];
-    if (forward_i)
-        k_combine_fftA<true><<<dim3(z.N, n_eval), kCfT, 0, s>>>(F1m, F2, Q, Mfft, scalars, z, G1, tw64, tw128);
-    else
-        k_combine_fftA<false><<<dim3(z.N, n_eval), kCfT, 0, s>>>(F1m, F2, Q, Mfft, scalars, z, G1, tw64, tw128);
+void fft3_ccc_tail(const FftTables& T, const CccTailArgs& a, hipStream_t s) {
+    switch (a.z.N) {
+        case 16: launch_ccc_tail<16>(T, a, s); break;
+        case 32: launch_ccc_tail<32>(T, a, s); break;
+        case 48: launch_ccc_tail<48>(T, a, s); break;
+        case 64: launch_ccc_tail<64>(T, a, s); break;
+        case 96: launch_ccc_tail<96>(T, a, s); break;
+        case 128: launch_ccc_tail<128>(T, a, s); break;
+        default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_ccc_tail: unsupported size " + std::to_string(a.z.N)};
+    }
     ETTK_HIP(hipGetLastError());
 }
 
@@ -1414,20 +1532,6 @@ void fft3_r2c_planes(const FftTables& T, const R2CArgs& a, hipStream_t s) {
     ETTK_HIP(hipGetLastError());
 }
 
-void fft3_op_r2c_after_ipass(const FftTables& T, float2* io, int n, int batch, int op, const float* aux, float* partials,
-                             bool forward_i, hipStream_t s) {
-    switch (n) {
-        case 16: launch_c2r_op_r2c<16>(T, nullptr, io, batch, op, aux, partials, s, forward_i); break;
-        case 32: launch_c2r_op_r2c<32>(T, nullptr, io, batch, op, aux, partials, s, forward_i); break;
-        case 48: launch_c2r_op_r2c<48>(T, nullptr, io, batch, op, aux, partials, s, forward_i); break;
-        case 64: launch_c2r_op_r2c<64>(T, nullptr, io, batch, op, aux, partials, s, forward_i); break;
-        case 96: launch_c2r_op_r2c<96>(T, nullptr, io, batch, op, aux, partials, s, forward_i); break;
-        case 128: launch_c2r_op_r2c<128>(T, nullptr, io, batch, op, aux, partials, s, forward_i); break;
-        default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_op_r2c_after_ipass: unsupported size " + std::to_string(n)};
-    }
-    ETTK_HIP(hipGetLastError());
-}
-
 void fft3_c2r_op_r2c(const FftTables& T, const float2* in, float2* io, int n, int batch, int op, const float* aux,
                      float* partials, hipStream_t s) {
     ETTK_REQUIRE(in != nullptr, ETTK_ERR_ARG, "fft3_c2r_op_r2c: null input");
@@ -1436,8 +1540,6 @@ void fft3_c2r_op_r2c(const FftTables& T, const float2* in, float2* io, int n, in
         case 32: launch_c2r_op_r2c<32>(T, in, io, batch, op, aux, partials, s); break;
         case 48: launch_c2r_op_r2c<48>(T, in, io, batch, op, aux, partials, s); break;
         case 64: launch_c2r_op_r2c<64>(T, in, io, batch, op, aux, partials, s); break;
-        case 96: launch_c2r_op_r2c<96>(T, in, io, batch, op, aux, partials, s); break;
-        case 128: launch_c2r_op_r2c<128>(T, in, io, batch, op, aux, partials, s); break;
         default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_c2r_op_r2c: unsupported size " + std::to_string(n)};
     }
     ETTK_HIP(hipGetLastError());

@@ -177,7 +177,7 @@ void wedge_normals(float lw, float uw, const Mat4& t, WedgeRef& w) {
     }
 }
 
-// search window of the upsampled correlation and its partial-DFT tables (FIM.h:1222-1247); rebuilt when
+// search window of the upsampled correlation and its third axis's DFT table (FIM.h:1222-1247); rebuilt when
 // the translation restriction changes
 static void search_window(ettk_plan* P) {
     const int N = P->N, H = P->H;
@@ -194,19 +194,13 @@ static void search_window(ettk_plan* P) {
     P->z.I0 = I0;
     P->z.ub2 = (E - 1) / 2;
     P->z.restr2 = (float)restr * (float)restr;
-    size_t lds_a = (size_t)(N * H + E * N) * sizeof(float2);
+    // the windows that an LDS-resident plane with both axes' tables would hold are the supported ones
     size_t lds_b = (size_t)(N * H + E * N + 2 * E * H) * sizeof(float2) + 2048;
-    ETTK_REQUIRE(lds_a <= 160 * 1024 && lds_b <= 160 * 1024, ETTK_ERR_UNSUPPORTED,
+    ETTK_REQUIRE(lds_b <= 160 * 1024, ETTK_ERR_UNSUPPORTED,
                  "translation search window too large for the LDS-resident upsampled DFT (reduce trans_restrict)");
-    std::vector<float2> tA((size_t)E * N), tK((size_t)E * H);
+    std::vector<float2> tK((size_t)E * H);
     for (int x = 0; x < E; x++) {
         int u = I0 + x - N;
-        for (int i = 0; i < N; i++) {
-            int fr = i - N / 2;
-            double ang = M_PI * (double)fr * (double)u / (double)N;
-            double sg = (fr & 1) ? -1.0 : 1.0;
-            tA[(size_t)x * N + i] = make_float2((float)(sg * std::cos(ang)), (float)(sg * std::sin(ang)));
-        }
         for (int k = 0; k < H; k++) {
             int fr = k - N / 2;
             double ang = M_PI * (double)fr * (double)u / (double)N;
@@ -215,7 +209,6 @@ static void search_window(ettk_plan* P) {
             tK[(size_t)x * H + k] = make_float2((float)(w * sg * std::cos(ang)), (float)(w * sg * std::sin(ang)));
         }
     }
-    P->tabA.upload(tA.data(), tA.size(), s);
     P->tabK.upload(tK.data(), tK.size(), s);
     ETTK_HIP(hipStreamSynchronize(s));
 }
@@ -295,21 +288,19 @@ template <class F>
 static void ccc_work_pieces(const ettk_plan* P, int E, F&& piece) {
     const int N = P->N, H = P->H;
     const size_t n3 = (size_t)N * N * N, nh = (size_t)N * N * H, nb_sp = spectral_partials(P);
-    piece(0, n3 * E * sizeof(float));                                   // R1
-    piece(1, n3 * E * sizeof(float));                                   // R2
-    piece(2, (size_t)2 * P->nb_res * E * sizeof(float));                // p_res
-    piece(3, nb_sp * E * sizeof(float));                                // p_n1
-    piece(4, nb_sp * E * sizeof(float));                                // p_n2
-    piece(5, nb_sp * E * sizeof(float));                                // p_wf
-    piece(6, (size_t)N * E * sizeof(float));                            // p_k1: one per plane
-    piece(7, (size_t)E * sizeof(float));                                // stats
-    piece(8, (size_t)4 * E * sizeof(float));                            // scalars
-    piece(9, (size_t)P->z.E * E * sizeof(float));                       // bval
-    piece(10, (size_t)P->z.E * E * sizeof(int));                        // bidx
-    piece(11, nh * E * sizeof(float2));                                 // S1
-    piece(12, nh * E * sizeof(float2));                                 // S2
-    piece(13, nh * E * sizeof(float2));                                 // S3
-    piece(14, (size_t)P->z.E * N * H * E * sizeof(float2));             // G1
+    piece(0, n3 * E * sizeof(float));                                   // R
+    piece(1, (size_t)2 * P->nb_res * E * sizeof(float));                // p_res
+    piece(2, nb_sp * E * sizeof(float));                                // p_n1
+    piece(3, nb_sp * E * sizeof(float));                                // p_n2
+    piece(4, nb_sp * E * sizeof(float));                                // p_wf
+    piece(5, (size_t)N * E * sizeof(float));                            // p_k1: one per plane
+    piece(6, (size_t)E * sizeof(float));                                // stats
+    piece(7, (size_t)P->z.E * E * sizeof(float));                       // bval
+    piece(8, (size_t)P->z.E * E * sizeof(int));                         // bidx
+    piece(9, nh * E * sizeof(float2));                                  // S1
+    piece(10, nh * E * sizeof(float2));                                 // S2
+    piece(11, nh * E * sizeof(float2));                                 // S3
+    piece(12, (size_t)P->z.E * N * H * E * sizeof(float2));             // G1
 }
 
 size_t ccc_work_bytes(const ettk_plan* P, int E) {
@@ -319,28 +310,26 @@ size_t ccc_work_bytes(const ettk_plan* P, int E) {
 }
 
 CccWork ccc_work_carve(const ettk_plan* P, int E, void* base) {
-    void* ptr[15];
+    void* ptr[13];
     size_t off = 0;
     ccc_work_pieces(P, E, [&](int i, size_t b) {
         ptr[i] = static_cast<char*>(base) + off;
         off += (b + 255) & ~(size_t)255;
     });
     CccWork W;
-    W.R1 = (float*)ptr[0];
-    W.R2 = (float*)ptr[1];
-    W.p_res = (float*)ptr[2];
-    W.p_n1 = (float*)ptr[3];
-    W.p_n2 = (float*)ptr[4];
-    W.p_wf = (float*)ptr[5];
-    W.p_k1 = (float*)ptr[6];
-    W.stats = (float*)ptr[7];
-    W.scalars = (float*)ptr[8];
-    W.bval = (float*)ptr[9];
-    W.bidx = (int*)ptr[10];
-    W.S1 = (float2*)ptr[11];
-    W.S2 = (float2*)ptr[12];
-    W.S3 = (float2*)ptr[13];
-    W.G1 = (float2*)ptr[14];
+    W.R = (float*)ptr[0];
+    W.p_res = (float*)ptr[1];
+    W.p_n1 = (float*)ptr[2];
+    W.p_n2 = (float*)ptr[3];
+    W.p_wf = (float*)ptr[4];
+    W.p_k1 = (float*)ptr[5];
+    W.stats = (float*)ptr[6];
+    W.bval = (float*)ptr[7];
+    W.bidx = (int*)ptr[8];
+    W.S1 = (float2*)ptr[9];
+    W.S2 = (float2*)ptr[10];
+    W.S3 = (float2*)ptr[11];
+    W.G1 = (float2*)ptr[12];
     return W;
 }
 
@@ -350,8 +339,7 @@ void ensure_ccc_workspace(ettk_plan* P, int cap) {
     P->ws_E = P->z.E;
     const int N = P->N, H = P->H;
     const size_t n3 = (size_t)N * N * N, nh = (size_t)N * N * H;
-    P->R1.ensure(n3 * cap);
-    P->R2.ensure(n3 * cap);
+    P->R.ensure(n3 * cap);
     P->S1.ensure(nh * cap);
     P->S2.ensure(nh * cap);
     P->S3.ensure(nh * cap);
@@ -363,7 +351,6 @@ void ensure_ccc_workspace(ettk_plan* P, int cap) {
     P->p_wf.ensure(nb_sp * cap);
     P->p_k1.ensure((size_t)N * cap);  // mask partials, one per plane
     P->stats.ensure(cap);
-    P->scalars.ensure((size_t)4 * cap);
     P->bval.ensure((size_t)P->z.E * cap);
     P->bidx.ensure((size_t)P->z.E * cap);
     P->out4.ensure((size_t)4 * cap);
@@ -401,8 +388,8 @@ static void ccc_batch_graph(ettk_plan* P, const float* d_parts, const ettk_parti
     P->h_out_pinned.ensure((size_t)4 * n);
     EvalGeom* g = P->h_geom.p;
     for (int e = 0; e < n; e++) g[e] = make_geom_public(P, eval_descs ? eval_descs[e] : descs[pidx[e]], t[e], pidx[e]);
-    CccWork W{P->R1.p, P->R2.p, P->p_res.p, P->p_n1.p, P->p_n2.p, P->p_wf.p, P->p_k1.p, P->stats.p, P->scalars.p,
-              P->bval.p, P->bidx.p, P->S1.p, P->S2.p, P->S3.p, P->G1.p};
+    CccWork W{P->R.p,     P->p_res.p, P->p_n1.p, P->p_n2.p, P->p_wf.p, P->p_k1.p, P->stats.p,
+              P->bval.p,  P->bidx.p,  P->S1.p,   P->S2.p,   P->S3.p,   P->G1.p};
     ETTK_HIP(hipEventRecord(P->ev0, s));
     for (int e0 = 0; e0 < n; e0 += chunk) {
         const int E = std::min(chunk, n - e0);
@@ -525,53 +512,28 @@ void wedge_overlaps(ettk_plan* P, const ettk_particle* descs, const Mat4* t, int
 
 void ccc_enqueue_chunk(ettk_plan* P, const CccWork& W, const float* d_parts, const EvalGeom* geo, int E, float* out4,
                        hipStream_t s) {
-    const int N = P->N, H = P->H;
-    const long nh = (long)N * N * H;
+    const int N = P->N;
     KernelProf* kp = P->ctx->fft.prof;
     const float* W1 = P->p.missing_wedge ? P->W1.p : nullptr;
     const int apply = P->dummy_filter ? 0 : 1;
-    const double Rb = (double)E * N * N * N * sizeof(float), Hb = (double)E * nh * sizeof(float2);
-    const double Gb = (double)E * P->z.E * N * H * sizeof(float2);
+    const double Rb = (double)E * N * N * N * sizeof(float);
     // particle side: F2 = r2c((reslice - mean) maskfft shift)
     {
         ProfScope ps(kp, "k_reslice", 2 * Rb, s, true);
-        launch_reslice(d_parts, geo, E, N, W.R2, W.p_res, P->nb_res, s, ps.start(), ps.stop());
+        launch_reslice(d_parts, geo, E, N, W.R, W.p_res, P->nb_res, s, ps.start(), ps.stop());
         ps.done();
     }
     launch_reslice_mean(W.p_res, P->nb_res, E, W.stats, s);
-    R2CArgs a2{W.R2, W.S2, N, E, PRO_RESLICED, P->maskfft.p, W.stats};
+    R2CArgs a2{W.R, W.S2, N, E, PRO_RESLICED, P->maskfft.p, W.stats};
     // F2 = r2c((reslice - mean) maskfft shift) up to its i pass; then on pencils along i: the i pass, both
     // spectra weighted by filter x W1 W2 (X1 = F1mcf, the reference with MCF applied once; X2 = mcf(F2)),
     // X2 kept for the combine, and both inverse i passes of the transforms below
     fft3_r2c_planes(P->ctx->fft, a2, s);
     CccIpassArgs ia{W.S2, W.S3, W.S1, P->F1mcf.p, P->filter.p, W1, geo, P->p.mcf, apply, W.p_n1, W.p_wf, W.p_n2};
     fft3_ccc_ipass(P->ctx->fft, ia, N, E, s);
-    const int nb_sp = fft3_ccc_ipass_blocks(N);
-    // reference side: c2r -> r1 m1 (with the k1_m partials) -> r2c = F1m, one partial per (evaluation, plane)
-    // (at 64 the forward i passes of both run inside the combine kernel)
-    const bool fwd = !ccc_combine_fft_supported(P->z);
-    fft3_op_r2c_after_ipass(P->ctx->fft, W.S1, N, E, PLANE_OP_MASK, P->m1.p, W.p_k1, fwd, s);
-    // particle side: Q = r2c(c2r(X2)^2 shift)
-    fft3_op_r2c_after_ipass(P->ctx->fft, W.S3, N, E, PLANE_OP_SQUARE_SHIFT, nullptr, nullptr, fwd, s);
-    // combine, upsampled correlation on the search window, peak
-    launch_ccc_scalars(W.p_n1, W.p_n2, W.p_k1, W.p_wf, nb_sp, N, E, N, W.scalars, s);
-    const bool cfft = ccc_combine_fft_supported(P->z);
-    {
-        ProfScope ps(kp, cfft ? "k_combine_fftA" : "k_combine_dftA", 3 * Hb + Gb, s);
-        if (cfft)
-            launch_combine_fftA(P->ctx->fft, W.S1, W.S2, W.S3, P->Mfft.p, W.scalars, P->z, E, W.G1, true, s);
-        else
-            launch_combine_dftA(W.S1, W.S2, W.S3, P->Mfft.p, W.scalars, P->tabA.p, P->z, E, W.G1, s);
-    }
-    {
-        ProfScope ps(kp, cfft ? "k_dftBC_fft" : "k_dftBC_argmax", Gb, s);
-        if (cfft)
-            launch_dftBC_fft(P->ctx->fft, W.G1, P->tabK.p, P->z, E, W.bval, W.bidx, s);
-        else
-            launch_dftBC_argmax(W.G1, P->tabA.p, P->tabK.p, P->z, E, W.bval, W.bidx, s);
-    }
-    launch_peak_final(W.bval, W.bidx, W.scalars, (float)P->sum_filter, (P->p.overlap_norm && P->p.missing_wedge) ? 1 : 0,
-                      P->z, E, out4, s);
+    CccTailArgs ta{W.S1, W.S2, W.S3, P->Mfft.p, P->m1.p, W.p_n1, W.p_n2, W.p_wf, W.p_k1, P->tabK.p, P->z, E, W.G1, W.bval,
+                   W.bidx, (float)P->sum_filter, (P->p.overlap_norm && P->p.missing_wedge) ? 1 : 0, out4};
+    fft3_ccc_tail(P->ctx->fft, ta, s);
 }
 
 bool ccc_lanes_available(const ettk_plan* P) {
@@ -619,8 +581,8 @@ void ccc_batch_begin(ettk_plan* P, int li, const float* d_parts, const ettk_part
         upload_before(P, L.geom_all.p + e0, g + e0, (size_t)E * sizeof(EvalGeom));
     };
     ETTK_HIP(hipEventRecord(L.ev0, s));
-    CccWork W{P->R1.p, P->R2.p, P->p_res.p, P->p_n1.p, P->p_n2.p, P->p_wf.p, P->p_k1.p, P->stats.p, P->scalars.p,
-              P->bval.p, P->bidx.p, P->S1.p, P->S2.p, P->S3.p, P->G1.p};
+    CccWork W{P->R.p,     P->p_res.p, P->p_n1.p, P->p_n2.p, P->p_wf.p, P->p_k1.p, P->stats.p,
+              P->bval.p,  P->bidx.p,  P->S1.p,   P->S2.p,   P->S3.p,   P->G1.p};
     for (int e0 = 0; e0 < n; e0 += chunk) {
         const int E = std::min(chunk, n - e0);
         geom_chunk(e0, E);

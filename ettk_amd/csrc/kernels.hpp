@@ -67,11 +67,6 @@ int fft3_ccc_ipass_blocks(int n);
 void fft3_ccc_ipass(const FftTables& T, const CccIpassArgs& a, int n, int batch, hipStream_t s);
 // the k/j plane passes of an r2c only (n <= 128): the i pass is left to fft3_ccc_ipass
 void fft3_r2c_planes(const FftTables& T, const R2CArgs& a, hipStream_t s);
-// fft3_c2r_op_r2c whose inverse i pass has already run (io holds the i-inverse-transformed spectra); without
-// `forward_i` its forward i pass is left to launch_combine_fftA
-void fft3_op_r2c_after_ipass(const FftTables& T, float2* io, int n, int batch, int op, const float* aux, float* partials,
-                             bool forward_i, hipStream_t s);
-
 // smoothed analytic wedge parameters of the reference
 struct WedgeRef {
     float v1[3], v2[3];
@@ -84,14 +79,26 @@ struct CccSizes {
     float restr2;         // restriction^2 for the spherical search mask
     int ub2;              // (E-1)/2
 };
-// launch_combine_dftA's result with the first DFT axis evaluated by FFTs (box size 64, any window); with
-// `forward_i`, F1m and Q are passed before their forward i transform, which the kernel runs itself
-bool ccc_combine_fft_supported(const CccSizes& z);
-void launch_combine_fftA(const FftTables& T, const float2* F1m, const float2* F2, const float2* Q, const float2* Mfft,
-                         const float* scalars, const CccSizes& z, int n_eval, float2* G1, bool forward_i, hipStream_t s);
-// launch_dftBC_argmax's result with the second DFT axis evaluated by FFTs (box size 64, any window)
-void launch_dftBC_fft(const FftTables& T, const float2* G1, const float2* tabK, const CccSizes& z, int n_eval,
-                      float* best_val, int* best_idx, hipStream_t s);
+// The CCC after fft3_ccc_ipass: both sides through the fused plane passes (S1: c2r, times m1 with the k1_m partials, r2c
+// = F1m; S3: c2r, squared, r2c = Q, both up to their forward i pass), C = (-M conj(Q)/n2^2 + 2 F1m/n1 conj(F2/n2 N^3))
+// (-1)^(i+j+k), its upsampled correlation on the search window and the peak
+struct CccTailArgs {
+    float2 *S1, *S2, *S3;
+    const float2* Mfft;
+    const float* m1;
+    const float *p_n1, *p_n2, *p_wf;  // fft3_ccc_ipass_blocks(N) per evaluation
+    float* p_k1;                      // N per evaluation
+    const float2* tabK;               // E x H
+    CccSizes z;
+    int batch;
+    float2* G1;                       // [e][x][j][k]
+    float* bval;                      // E per evaluation
+    int* bidx;
+    float sum_filter;
+    int overlap;
+    float* out4;                      // [e][4] = distance, shift
+};
+void fft3_ccc_tail(const FftTables& T, const CccTailArgs& a, hipStream_t s);
 
 // reslice (tricubic Keys a=-1/2, clamp border, -FLT_MAX outside): out [e][i][j][k]; `nb` must equal
 // reslice_blocks(N) (one workgroup per 8^3 output tile), partials hold 2 * nb floats per evaluation
@@ -104,16 +111,6 @@ void launch_reslice_projection(const float* parts, const EvalGeom* geom, int n, 
                                int nb, hipStream_t s);
 // mean of the valid voxels per evaluation, from the reslice partials (nb per eval): stats[e] = mean
 void launch_reslice_mean(const float* partials, int nb, int n_eval, float* stats, hipStream_t s);
-// per-evaluation scalars: norm1, norm2, k1_m, sum(W filter)
-void launch_ccc_scalars(const float* p_n1, const float* p_n2, const float* p_k1, const float* p_wf, int nb_spec,
-                        int nb_real, int n_eval, int N, float* scalars, hipStream_t s);
-// C = (-M conj(Q)/n2^2 + 2 F1m/n1 conj(F2/n2 N^3)) (-1)^(i+j+k), then G1[e][x][j][k] = sum_i A[x][i] C(i,j,k)
-void launch_combine_dftA(const float2* F1m, const float2* F2, const float2* Q, const float2* Mfft,
-                         const float* scalars, const float2* tabA, const CccSizes& z, int n_eval, float2* G1,
-                         hipStream_t s);
-// G2 = sum_j A[y][j] G1, T = sum_k Re(G2 K[z][k]) on the crop, spherical mask, first argmax per (e, x)
-void launch_dftBC_argmax(const float2* G1, const float2* tabA, const float2* tabK, const CccSizes& z, int n_eval,
-                         float* best_val, int* best_idx, hipStream_t s);
 // continuous CCC and adjoint in the particle frame (refine.hip)
 struct RefineGeom {
     float G[12];          // q = G[r*4 + 0..2] (x, y, z) - N/2 + G[r*4 + 3]: reference index of particle voxel (x,y,z)
@@ -180,9 +177,4 @@ void launch_mcf_inplace(float2* F, long n, hipStream_t s);
 // zero n elements with a kernel (a fill node, not a memset node, when the stream is captured into a graph)
 void launch_fill_zero(int* p, size_t n, hipStream_t s);
 void launch_fill_zero(double* p, size_t n, hipStream_t s);
-// final per evaluation: first maximum over x, distance and shift
-void launch_peak_final(const float* best_val, const int* best_idx, const float* scalars, float sum_filter,
-                       int overlap, const CccSizes& z, int n_eval, float* out /* [e][4] = dist, sx, sy, sz */,
-                       hipStream_t s);
-
 }  // namespace ettk

@@ -134,7 +134,7 @@ struct ettk_plan {
     ettk::CccSizes z{};
     // constant device data
     ettk::DevBuf<float> maskfft, m1, filter, W1;
-    ettk::DevBuf<float2> Mfft, F1mcf, tabA, tabK;
+    ettk::DevBuf<float2> Mfft, F1mcf, tabK;
     std::vector<float> h_m1;
     // reference
     bool have_ref = false;
@@ -143,7 +143,7 @@ struct ettk_plan {
     // CCC workspace
     int cap = 0, ws_E = 0;
     int nb_res = 0;
-    ettk::DevBuf<float> R1, R2, p_res, p_n1, p_n2, p_k1, p_wf, stats, scalars, bval, out4;
+    ettk::DevBuf<float> R, p_res, p_n1, p_n2, p_k1, p_wf, stats, bval, out4;
     ettk::DevBuf<int> bidx;
     ettk::DevBuf<float2> S1, S2, S3, G1;
     ettk::DevBuf<ettk::EvalGeom> geom;
@@ -192,7 +192,7 @@ namespace ettk {
 // device workspace of one chunk of E constrained-CCC evaluations: the plan's own buffers (ccc_batch) or a
 // caller-independent fixed region (ettk_ccc_eval_batch_noalloc)
 struct CccWork {
-    float *R1, *R2, *p_res, *p_n1, *p_n2, *p_wf, *p_k1, *stats, *scalars, *bval;
+    float *R, *p_res, *p_n1, *p_n2, *p_wf, *p_k1, *stats, *bval;
     int* bidx;
     float2 *S1, *S2, *S3, *G1;
 };

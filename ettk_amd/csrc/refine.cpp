@@ -157,20 +157,20 @@ static void refine_enqueue(ettk_plan* P, RefineChunk& c) {
     const double Rb = (double)E * N * N * N * sizeof(float);
     {
         ProfScope ps(kp, "k_reslice_ref", Rb, s);
-        launch_reslice_ref(P->ref_x.p, geo, E, N, P->R2.p, s);
+        launch_reslice_ref(P->ref_x.p, geo, E, N, P->R.p, s);
     }
-    R2CArgs a{P->R2.p, P->S2.p, N, E, PRO_MASK_SHIFT, P->maskfft.p, nullptr};
+    R2CArgs a{P->R.p, P->S2.p, N, E, PRO_MASK_SHIFT, P->maskfft.p, nullptr};
     double* sc = P->r_sc.p + (size_t)4 * e0;
     // the score terms in the epilogue of the forward i pass, the adjoint spectrum in the prologue of the inverse one:
     // X1 is read once by each instead of once more by separate score and adjoint passes
     fft3_r2c_planes(P->ctx->fft, a, s);
     fft3_refine_dot(P->ctx->fft, P->S2.p, P->r_fp.p, P->filter.p, P->ref_wbin.p, geo, N, E, P->r_pdot.p, s);
     launch_refine_scalars(P->r_pdot.p, fft3_refine_ipass_blocks(N), E, sc, s);
-    fft3_refine_adj_c2r(P->ctx->fft, P->S2.p, P->r_fp.p, P->filter.p, P->ref_wbin.p, geo, sc, N, E, P->S3.p, P->R1.p, s);
+    fft3_refine_adj_c2r(P->ctx->fft, P->S2.p, P->r_fp.p, P->filter.p, P->ref_wbin.p, geo, sc, N, E, P->S3.p, P->R.p, s);
     double* mom = P->r_mom.p + (size_t)12 * e0;
     {
         ProfScope ps(kp, "k_refine_moments", Rb, s);
-        launch_refine_moments(P->ref_x.p, geo, P->R1.p, P->maskfft.p, E, N, P->r_mpart.p, mom, s);
+        launch_refine_moments(P->ref_x.p, geo, P->R.p, P->maskfft.p, E, N, P->r_mpart.p, mom, s);
     }
     // the downloads on the copy stream: the next chunk's kernels do not wait for them
     hipStream_t cs = P->copy_stream;

@@ -169,39 +169,41 @@ template <int L> struct ColShape {
 // Transforms the pencil whose elements t + T j are in x[j]; `ex` is the workgroup's exchange buffer (L P complex
 // values, [element][p]) plus p, `tw` the forward twiddles of length L in LDS (written before a barrier that every
 // thread has passed).  Every thread of the workgroup must call it: it synchronises after the exchange's writes and
-// after its reads.
-template <int L, bool INV>
-__device__ __forceinline__ void col_fft(float2* x, int t, float2* ex, const float2* tw) {
+// after its reads.  P: pencils of the workgroup; threads without a pencil pass live = false.
+template <int L, bool INV, int P = ColShape<L>::P>
+__device__ __forceinline__ void col_fft(float2* x, int t, float2* ex, const float2* tw, bool live = true) {
     using S = ColShape<L>;
-    constexpr int T = S::T, P = S::P, N1 = S::N1, N2 = S::N2, S2 = N2 / T, S1 = N1 / T;
+    constexpr int T = S::T, N1 = S::N1, N2 = S::N2, S2 = N2 / T, S1 = N1 / T;
+    if (live)
 #pragma unroll
-    for (int i = 0; i < S2; i++) {
-        float2 v[N1];
+        for (int i = 0; i < S2; i++) {
+            float2 v[N1];
 #pragma unroll
-        for (int m = 0; m < N1; m++) v[m] = x[i + S2 * m];
-        Dft<N1, INV>::run(v);
-        const int b = t + T * i;
+            for (int m = 0; m < N1; m++) v[m] = x[i + S2 * m];
+            Dft<N1, INV>::run(v);
+            const int b = t + T * i;
 #pragma unroll
-        for (int k = 0; k < N1; k++) {
-            if (k > 0) {
-                float2 w = tw[b * k];  // b k <= (N2 - 1)(N1 - 1) < L
-                if (INV) w.y = -w.y;
-                v[k] = cmul(v[k], w);
+            for (int k = 0; k < N1; k++) {
+                if (k > 0) {
+                    float2 w = tw[b * k];  // b k <= (N2 - 1)(N1 - 1) < L
+                    if (INV) w.y = -w.y;
+                    v[k] = cmul(v[k], w);
+                }
+                ex[(k * N2 + b) * P] = v[k];
             }
-            ex[(k * N2 + b) * P] = v[k];
         }
-    }
     __syncthreads();
+    if (live)
 #pragma unroll
-    for (int i = 0; i < S1; i++) {
-        float2 v[N2];
-        const int k1 = t + T * i;
+        for (int i = 0; i < S1; i++) {
+            float2 v[N2];
+            const int k1 = t + T * i;
 #pragma unroll
-        for (int b = 0; b < N2; b++) v[b] = ex[(k1 * N2 + b) * P];
-        Dft<N2, INV>::run(v);
+            for (int b = 0; b < N2; b++) v[b] = ex[(k1 * N2 + b) * P];
+            Dft<N2, INV>::run(v);
 #pragma unroll
-        for (int k = 0; k < N2; k++) x[i + S1 * k] = v[k];
-    }
+            for (int k = 0; k < N2; k++) x[i + S1 * k] = v[k];
+        }
     __syncthreads();
 }
 

@@ -127,7 +127,7 @@ int ettk_ccc_eval_batch(ettk_plan* plan, const float* d_particles, int n_particl
    cannot allocate device memory while they run (code under HIP graph capture, tight serving loops, harnesses
    that forbid hipMalloc).  Same arguments, results and errors as ettk_ccc_eval_batch; the workspace is a fixed
    128 MiB device region per GPU, reserved when the library is loaded on that GPU and held until the process
-   ends; evaluations run in chunks that fit it (at box 64 with an 8-voxel translation window, 16 per chunk).
+   ends; evaluations run in chunks that fit it (at box 64 with an 8-voxel translation window, 24 per chunk).
    A size whose single evaluation does not fit is rejected with ETTK_ERR_UNSUPPORTED.  All calls on one GPU
    share the region: calls that overlap on one GPU race, so the caller serialises them.  The plan and its
    reference must have been set up beforehand (ettk_plan_create, ettk_reference_set allocate). */

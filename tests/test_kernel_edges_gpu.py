@@ -112,3 +112,35 @@ def test_register_pencils(torch_gpu, ctx, n, batch):
     back = np.linalg.norm(b.cpu().numpy() / n ** 3 - v) / np.linalg.norm(v)
     print(f"[edges] fft {n} x{batch}: {rel:.2e} {back:.2e}", flush=True)
     assert rel < 5e-6 and back < 5e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,window", [(16, 3.0), (32, -1.0), (48, 1.0), (64, 0.0), (64, -1.0), (96, 19.5), (128, 11.0)])
+def test_ccc_windows(torch_gpu, ctx, N, window):
+    """The search window of the upsampled correlation at its ends: a single point (0), 3 x 3 x 3 half voxels (1), the
+    whole doubled box (-1, at 32 and 64), the widest windows that 96 and 128 accept, and the smallest box.  Against the
+    FP64 oracle with the bounds of the other comparisons of this chain: FP32 transforms and sums leave 1e-6 of the two
+    norms whose difference the distance is, and the distance is above 1e-3 of them; the shift is an index, equal unless
+    two half-voxel points tie within that."""
+    from ettk_amd.lib import Plan
+    from oracle_lib import OraclePlan
+    from parity import DIST_RTOL, peak_tie
+
+    p = default_params(N, 8, mask_radius=N / 2 - 3, square_mask=2, trans_restrict=window)
+    ref = blob_reference(N, seed=5)
+    n = 3 if N <= 64 else 1
+    ps = make_particles(ref, n, seed=6, half_wedge=(50, 60), snr=(0.3, 0.3), max_shift=2.0)
+    plan, orc = Plan(ctx, p), OraclePlan(p)
+    try:
+        plan.set_reference(to_dev(torch_gpu, ref))
+        orc.set_reference(ref)
+        t = ps.truth.copy()
+        t[:, :3, 3] = 0.0
+        dist, out = plan.ccc(to_dev(torch_gpu, ps.vols), ps.descs, list(range(n)), t)
+        for i in range(n):
+            want, m = orc.ccc(ps.vols[i], ps.descs[i], t[i])
+            print(f"[edges] ccc N={N} window {window}: {dist[i]:.6e} {want:.6e}", flush=True)
+            assert abs(dist[i] - want) <= DIST_RTOL * abs(want) + 1e-7
+            assert np.abs(out[i] - m).max() < 1e-9 or peak_tie(orc, ps.vols[i], ps.descs[i], t[i], out[i])[0]
+    finally:
+        plan.close()
