@@ -15,47 +15,56 @@ __device__ __forceinline__ float wedge_bin(const float* v1, const float* v2, int
     float b = v2[0] * di + v2[1] * dj + v2[2] * dk;
     return (a * b <= 0.f) ? 1.f : 0.f;
 }
+// taps of a position: 3 inside, 2 at the borders, renormalised (constants: the same divisions at compile time)
 __device__ __forceinline__ void tap3(int idx, int n, float* w) {
-    const float g = 0.88249690258459540286f;  // exp(-1/8)
-    float l = idx > 0 ? g : 0.f, r = idx < n - 1 ? g : 0.f;
-    float inv = 1.f / (l + 1.f + r);
-    w[0] = l * inv;
-    w[1] = inv;
-    w[2] = r * inv;
+    constexpr float g = 0.88249690258459540286f;  // exp(-1/8)
+    constexpr float in = 1.f / (g + 1.f + g), edge = 1.f / (1.f + g);
+    const bool first = idx <= 0, last = idx >= n - 1;
+    w[1] = first || last ? edge : in;
+    w[0] = first ? 0.f : last ? g * edge : g * in;
+    w[2] = last ? 0.f : first ? g * edge : g * in;
 }
-__device__ inline float wedge_smooth(const float* v1, const float* v2, int i, int j, int k, int N, int nk) {
-    // Away from both planes the 27 binary samples all equal the centre's: the smoothed value is then 0 or the
-    // kernel's sum, accumulated in the same order as the full stencil below (so the value is identical).
+// Away from both planes the 27 binary samples all equal the centre's: true when they do, with that sample
+__device__ __forceinline__ bool wedge_uniform(const float* v1, const float* v2, int i, int j, int k, int N, bool& in) {
     const float di = (float)(i - N / 2), dj = (float)(j - N / 2), dk = (float)(k - N / 2);
     const float a0 = v1[0] * di + v1[1] * dj + v1[2] * dk, b0 = v2[0] * di + v2[1] * dj + v2[2] * dk;
     const float r1 = fabsf(v1[0]) + fabsf(v1[1]) + fabsf(v1[2]), r2 = fabsf(v2[0]) + fabsf(v2[1]) + fabsf(v2[2]);
-    const bool uniform = fabsf(a0) > r1 * 1.001f + 1e-3f && fabsf(b0) > r2 * 1.001f + 1e-3f;
-    if (uniform && a0 * b0 > 0.f) return 0.f;
+    in = !(a0 * b0 > 0.f);
+    return fabsf(a0) > r1 * 1.001f + 1e-3f && fabsf(b0) > r2 * 1.001f + 1e-3f;
+}
+// the kernel's sum at (i, j, k), accumulated in the same order as the stencil of ones would be: the smoothed value where
+// all samples are 1
+__device__ __forceinline__ float wedge_ones(int i, int j, int k, int N, int nk) {
     float wi[3], wj[3], wk[3];
     tap3(i, N, wi);
     tap3(j, N, wj);
     tap3(k, nk, wk);
-    if (uniform) {
-        float acc = 0.f;
+    float acc = 0.f;
 #pragma unroll
-        for (int a = 0; a < 3; a++) {
-            if (wi[a] == 0.f) continue;
-            float sj = 0.f;
+    for (int a = 0; a < 3; a++) {
+        if (wi[a] == 0.f) continue;
+        float sj = 0.f;
 #pragma unroll
-            for (int b = 0; b < 3; b++) {
-                if (wj[b] == 0.f) continue;
-                float sk = 0.f;
+        for (int b = 0; b < 3; b++) {
+            if (wj[b] == 0.f) continue;
+            float sk = 0.f;
 #pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    if (wk[c] == 0.f) continue;
-                    sk += wk[c] * 1.f;
-                }
-                sj += wj[b] * sk;
+            for (int c = 0; c < 3; c++) {
+                if (wk[c] == 0.f) continue;
+                sk += wk[c] * 1.f;
             }
-            acc += wi[a] * sj;
+            sj += wj[b] * sk;
         }
-        return acc;
+        acc += wi[a] * sj;
     }
+    return acc;
+}
+// the 27-sample stencil
+__device__ inline float wedge_stencil(const float* v1, const float* v2, int i, int j, int k, int N, int nk) {
+    float wi[3], wj[3], wk[3];
+    tap3(i, N, wi);
+    tap3(j, N, wj);
+    tap3(k, nk, wk);
     float acc = 0.f;
 #pragma unroll
     for (int a = -1; a <= 1; a++) {
@@ -75,6 +84,11 @@ __device__ inline float wedge_smooth(const float* v1, const float* v2, int i, in
         acc += wi[a + 1] * sj;
     }
     return acc;
+}
+__device__ inline float wedge_smooth(const float* v1, const float* v2, int i, int j, int k, int N, int nk) {
+    bool in;
+    if (wedge_uniform(v1, v2, i, j, k, N, in)) return in ? wedge_ones(i, j, k, N, nk) : 0.f;
+    return wedge_stencil(v1, v2, i, j, k, N, nk);
 }
 
 }  // namespace ettk
