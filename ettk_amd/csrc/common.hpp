@@ -94,6 +94,13 @@ __device__ __forceinline__ void st_stream(float2* p, float2 v) {
     __builtin_nontemporal_store(w, reinterpret_cast<nt_float2*>(p));
 }
 
+// Element at a byte offset from a pointer that is the same for the whole workgroup: the address then takes one 32-bit
+// register instead of a 64-bit pair per element.
+template <class T>
+__device__ __forceinline__ T& at_byte(T* base, unsigned off) {
+    return *reinterpret_cast<T*>((char*)base + off);
+}
+
 // Workgroup-wide copies in which every global load of a round is issued before the first loaded value is used,
 // so a round costs one memory latency instead of one per element.  Thread t moves elements t, t + NT, ...;
 // out-of-range slots re-read the last element and are dropped.

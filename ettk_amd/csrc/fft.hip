@@ -123,14 +123,6 @@ __device__ __forceinline__ TwCache<L> tw_cache(const float2* tw, int lane) {
     return c;
 }
 
-// Orders the LDS accesses of one wavefront: the LDS instructions of a wavefront execute in order, so threads of
-// one wavefront exchanging data through LDS only need the compiler kept from reordering those accesses.
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // every thread of the workgroup must call it (it ends with a workgroup barrier, after which the whole pencil is
 // visible to every thread).  The 8 threads of a pencil (lanes 8q .. 8q+7 of the workgroup) share a wavefront,
 // so the exchange inside needs only wavefront ordering.  The 8 x 8 exchange goes through rows of 9
@@ -408,10 +400,11 @@ __global__ void __launch_bounds__(ColShape<L>::THREADS) k_ccc_ipass(CccIpassArgs
     const bool valid = p < LH;
     const int pc = valid ? p : 0, pj = pc / H, pk = pc % H;
     const size_t vol = (size_t)e * L * LH;
+    const unsigned lo = (t * LH + pc) * 8;  // byte offset of this thread's first element of a spectrum
     float2* __restrict__ xp = ex + threadIdx.x % S::P;
     float2 x[NE];
 #pragma unroll
-    for (int u = 0; u < NE; u++) x[u] = ld_stream(&a.S2[vol + (size_t)(t + u * S::T) * LH + pc]);
+    for (int u = 0; u < NE; u++) x[u] = ld_stream(&at_byte(a.S2 + vol + u * S::T * LH, lo));
     for (int q = threadIdx.x; q < L; q += S::THREADS) tw[q] = twg[q];
     __syncthreads();
     col_fft<L, false>(x, t, xp, tw);
@@ -423,9 +416,8 @@ __global__ void __launch_bounds__(ColShape<L>::THREADS) k_ccc_ipass(CccIpassArgs
     float s2 = 0.f, swf = 0.f;
 #pragma unroll
     for (int u = 0; u < NE; u++) {
-        const size_t h = (size_t)(t + u * S::T) * LH + pc;
-        fw[u] = a.filter[h];
-        w1[u] = a.W1 ? a.W1[h] : 1.f;
+        fw[u] = at_byte(a.filter + u * S::T * LH, lo / 2);
+        w1[u] = a.W1 ? at_byte(a.W1 + u * S::T * LH, lo / 2) : 1.f;
     }
     if (!g.full) {
         // Smoothed wedge W2.  About one element in ten lies near a plane and needs the 27-sample stencil, but nearly
@@ -469,7 +461,7 @@ __global__ void __launch_bounds__(ColShape<L>::THREADS) k_ccc_ipass(CccIpassArgs
         if (a.apply) z = cscale(z, fw[u]);
         if (i == dc_i && pj == dc_j && pk == dc_k) z = make_float2(0.f, 0.f);
         if (valid) {
-            st_stream(&a.S2[vol + (size_t)i * LH + pc], z);
+            st_stream(&at_byte(a.S2 + vol + u * S::T * LH, lo), z);
             s2 += hw * (z.x * z.x + z.y * z.y);
             swf += fw[u];
         }
@@ -479,10 +471,10 @@ __global__ void __launch_bounds__(ColShape<L>::THREADS) k_ccc_ipass(CccIpassArgs
     // reference side: its spectrum loads are issued before the particle side's inverse transform is stored
     float2 f1[NE];
 #pragma unroll
-    for (int u = 0; u < NE; u++) f1[u] = a.F1mcf[(size_t)(t + u * S::T) * LH + pc];
+    for (int u = 0; u < NE; u++) f1[u] = at_byte(a.F1mcf + u * S::T * LH, lo);
     if (valid)
 #pragma unroll
-        for (int u = 0; u < NE; u++) st_stream(&a.S3[vol + (size_t)(t + u * S::T) * LH + pc], x[u]);
+        for (int u = 0; u < NE; u++) st_stream(&at_byte(a.S3 + vol + u * S::T * LH, lo), x[u]);
     float s1 = 0.f;
 #pragma unroll
     for (int u = 0; u < NE; u++) {
@@ -496,7 +488,7 @@ __global__ void __launch_bounds__(ColShape<L>::THREADS) k_ccc_ipass(CccIpassArgs
     col_fft<L, true>(x, t, xp, tw);
     if (valid)
 #pragma unroll
-        for (int u = 0; u < NE; u++) st_stream(&a.S1[vol + (size_t)(t + u * S::T) * LH + pc], x[u]);
+        for (int u = 0; u < NE; u++) st_stream(&at_byte(a.S1 + vol + u * S::T * LH, lo), x[u]);
     const float t1 = block_sum_nt<S::THREADS>(s1, sred);
     const float tf = block_sum_nt<S::THREADS>(swf, sred);
     const float t2 = block_sum_nt<S::THREADS>(s2, sred);
@@ -762,114 +754,132 @@ struct PlaneOps {
     const float* mask;  // PLANE_OP_MASK
     float* partials;    // PLANE_OP_MASK
 };
+// The columns (transforms along j, one per k) and the row pairs (transforms along k) of the plane take turns in
+// registers: inverse j on the columns straight from global memory, one pass through LDS to the row pairs, both k
+// transforms and the operation in registers, one pass back, forward j, store.  The L/2 columns below Nyquist and the
+// L/2 row pairs occupy the workgroup's threads exactly; the Nyquist column goes through one wavefront beside them.  The
+// inverse keeps the real part of the DC and Nyquist columns, as FFTW's c2r does.  Bound by LDS (14 accesses per element
+// of the half plane, against 26 with every transform's pencils staged in LDS and the DC and Nyquist columns packed into
+// one pencil): both sides of 240 evaluations at 64^3 take 228 us against 402, of 36 at 128^3 375 against 596.
+template <int L> struct OpPlane {
+    using S = ColShape<L>;
+    static constexpr int H = L / 2 + 1, T = S::T, E = S::E, LR = kRowLd<L>;
+    static constexpr int HS = T == 8 ? (H + 7) / 8 * 8 - 4 : H + 1;  // row stride of the plane: row pairs spread as LR does
+    static constexpr int THREADS = L / 2 * T;
+    static constexpr int LDS = L * HS > L / 2 * LR ? L * HS : L / 2 * LR;  // columns' exchange, the plane, or row pencils
+    static_assert(HS >= H && (T == 8 ? HS % 8 == 4 : HS % 4 == 2), "row stride");
+    // wavefronts per SIMD with which as many workgroups share a CU as its LDS holds
+    static constexpr int WAVES = L == 96 ? 3 : 4;
+};
 template <int L>
-__global__ void __launch_bounds__(Plane<L>::THREADS) k_c2r_r2c_plane(PlaneOps a, const float2* __restrict__ twg) {
-    using PL = Plane<L>;
-    constexpr int H = PL::H, LD = PL::LD, T = PL::THREADS;
-    constexpr int NZ = ((L / 2) * L + T - 1) / T;
-    constexpr int NS = ((L / 2) * 2 * H + T - 1) / T;
-    constexpr int NFW = T / 64, REM = T % 64;  // full waves, threads of the partial wave
-    __shared__ float2 buf[H * LD];
+__global__ void __launch_bounds__(OpPlane<L>::THREADS, OpPlane<L>::WAVES) k_c2r_r2c_plane(PlaneOps a,
+                                                                                          const float2* __restrict__ twg) {
+    using O = OpPlane<L>;
+    constexpr int H = O::H, HS = O::HS, T = O::T, E = O::E, LR = O::LR, NT = O::THREADS, C = L / 2;
+    __shared__ float2 buf[O::LDS];
+    __shared__ float2 nyq_pen[LR];
+    __shared__ float nyq[L];
     __shared__ float2 tw[L];
-    __shared__ float sred[NFW + REM + 1];
+    __shared__ float sred[NT / 64 + NT % 64 + 1];
     const bool second = blockIdx.x >= a.planes;
     const long plane = second ? blockIdx.x - a.planes : blockIdx.x;
     const int op = second ? a.op1 : a.op0;
-    const float* __restrict__ aux = a.mask;
-    float* __restrict__ partials = a.partials;
     const int pi = (int)(plane % L);
-    const float2 twv = twg[threadIdx.x % L];  // stored after the staging loads are in flight
-    float2* ip = (second ? a.io1 : a.io0) + plane * L * H;
-    block_copy<T, L * H>([&](int t) { return ip[t]; }, [&](int t, float2 v) { buf[(t % H) * LD + t / H] = v; });
-    if (threadIdx.x < L) tw[threadIdx.x] = twv;
-    __syncthreads();
-    pack_dc_nyquist<L>(buf);
-    __syncthreads();
-    const int q = threadIdx.x / PL::TPP, lane = threadIdx.x % PL::TPP;
-    const TwCache<L> twc = tw_cache<L>(tw, lane);
-    pencil_fft<L>(&buf[q * LD], lane, tw, twc, true);
-    // c2r along k (as k_c2r_plane)
-    float2 zr[NZ];
+    float2* __restrict__ ip = (second ? a.io1 : a.io0) + plane * L * H;
+    // columns: c = k, elements j = ct + T u; row pairs: rows 2 q and 2 q + 1, elements k = rt + T u
+    const int c = threadIdx.x % C, ct = threadIdx.x / C, q = threadIdx.x / T, rt = threadIdx.x % T;
+    float2 x[E];
 #pragma unroll
-    for (int u = 0; u < NZ; u++) {
-        const int t = threadIdx.x + u * T;
-        if (t < (L / 2) * L) zr[u] = c2r_row_pair<L>(buf, t / L, t % L);
+    for (int u = 0; u < E; u++) x[u] = at_byte(ip + T * u * H, (ct * H + c) * 8);
+    for (int i = threadIdx.x; i < L; i += NT) tw[i] = twg[i];
+    __syncthreads();
+    col_fft<L, true, C>(x, ct, buf + c, tw);
+#pragma unroll
+    for (int u = 0; u < E; u++) {
+        if (c == 0) x[u].y = 0.f;
+        buf[(ct + T * u) * HS + c] = x[u];
+    }
+    if (threadIdx.x < T) {
+#pragma unroll
+        for (int u = 0; u < E; u++) x[u] = at_byte(ip + T * u * H, (rt * H + C) * 8);
+        row_fft<L, true>(x, rt, nyq_pen, tw);
+#pragma unroll
+        for (int u = 0; u < E; u++) nyq[rt + T * u] = x[u].x;
     }
     __syncthreads();
+    // Z(k) = A(k) + i B(k) of rows 2q and 2q + 1 over the full length, A(L - k) = conj A(k)
 #pragma unroll
-    for (int u = 0; u < NZ; u++) {
-        const int t = threadIdx.x + u * T;
-        if (t < (L / 2) * L) buf[(t / L) * LD + (t % L)] = zr[u];
+    for (int u = 0; u < E; u++) {
+        if (E > 8 && u % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // at most 8 LDS reads ahead of their use
+        const int k = rt + T * u;
+        if (k == C) {
+            x[u] = make_float2(nyq[2 * q], nyq[2 * q + 1]);
+            continue;
+        }
+        const int kk = k < C ? k : L - k;
+        const float2 A = buf[2 * q * HS + kk], B = buf[(2 * q + 1) * HS + kk];
+        x[u] = k < C ? make_float2(A.x - B.y, A.y + B.x) : make_float2(A.x + B.y, B.x - A.y);
     }
-    __syncthreads();
-    pencil_fft<L>(&buf[q * LD], lane, tw, twc, true);
-    __syncthreads();
-    // buf[p LD + x] = (r(row 2p, x), r(row 2p + 1, x)): the pointwise operation in place
+    __syncthreads();  // the plane is read: its storage becomes the row pencils'
     float sacc = 0.f;
+    float2* __restrict__ pen = buf + q * LR;
+    const float* __restrict__ mp = a.mask + (size_t)pi * L * L;
+    const unsigned mo = (2 * q * L + rt) * 4;
+    row_fft<L, true>(x, rt, pen, tw);
+    // x[u] = (r(row 2q), r(row 2q + 1)) at rt + T u
     if (op == PLANE_OP_MASK) {
-        // mask values of rows j0, j0 + 1 at x: all loads in flight before the first use
-        const float* __restrict__ mp = aux + (size_t)pi * L * L;
-        block_copy<T, (L / 2) * L>(
-            [&](int t) { return make_float2(mp[(2 * (t / L)) * L + t % L], mp[(2 * (t / L) + 1) * L + t % L]); },
-            [&](int t, float2 m) {
-                const int pp = t / L, x = t % L;
-                float2 z = buf[pp * LD + x];
-                sacc += z.x * z.x * m.x;
-                sacc += z.y * z.y * m.y;
-                z.x *= m.x;
-                z.y *= m.y;
-                buf[pp * LD + x] = z;
-            });
+#pragma unroll
+        for (int u0 = 0; u0 < E; u0 += 4) {  // eight mask values in flight at a time: the registers hold the pencils
+            __builtin_amdgcn_sched_barrier(0);
+            float2 m[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) m[u] = make_float2(at_byte(mp + T * (u0 + u), mo), at_byte(mp + T * (u0 + u) + L, mo));
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                float2& z = x[u0 + u];
+                sacc += z.x * z.x * m[u].x;
+                sacc += z.y * z.y * m[u].y;
+                z.x *= m[u].x;
+                z.y *= m[u].y;
+            }
+        }
     } else {
-        for (int t = threadIdx.x; t < (L / 2) * L; t += T) {
-            const int pp = t / L, x = t % L, j0 = 2 * pp;
-            float2 z = buf[pp * LD + x];
-            const float sg = ((pi + j0 + x) & 1) ? -1.0f : 1.0f;
-            z.x = z.x * z.x * sg;
-            z.y = z.y * z.y * (-sg);
-            buf[pp * LD + x] = z;
-        }
+        const float sg = ((pi + rt) & 1) ? -1.0f : 1.0f;  // T and 2 q are even
+#pragma unroll
+        for (int u = 0; u < E; u++) x[u] = make_float2(x[u].x * x[u].x * sg, x[u].y * x[u].y * -sg);
     }
+    row_fft<L, false>(x, rt, pen, tw);
+#pragma unroll
+    for (int u = 0; u < E; u++) pen[rt + T * u] = x[u];
     if (op == PLANE_OP_MASK) {
-        // deterministic block sum: shuffles inside the full waves, the partial wave's values through LDS
-        const int w = threadIdx.x >> 6;
-        if (w < NFW) {
-            for (int o = 32; o > 0; o >>= 1) sacc += __shfl_down(sacc, o, 64);
-            if ((threadIdx.x & 63) == 0) sred[w] = sacc;
-        } else {
-            sred[NFW + (threadIdx.x & 63)] = sacc;
-        }
+        const float tot = block_sum_nt<NT>(sacc, sred);
+        if (threadIdx.x == 0) a.partials[plane] = tot;
     }
     __syncthreads();
-    if (op == PLANE_OP_MASK && threadIdx.x == 0) {
-        float tot = 0.f;
-        for (int i = 0; i < NFW + REM; i++) tot += sred[i];
-        partials[plane] = tot;
-    }
-    // r2c along k then j (as k_r2c_plane after its load)
-    pencil_fft<L>(&buf[q * LD], lane, tw, twc, false);
-    float2 o[NS];
+    const int cm = (L - c) % L;
+    // column c of row j from the packed pair: (Z(c) + conj Z(-c)) / 2 for even rows, (Z(c) - conj Z(-c)) / 2i for odd
+    // ones; j = ct + T u has ct's parity
+    if (threadIdx.x < T) {
 #pragma unroll
-    for (int u = 0; u < NS; u++) {
-        const int t = threadIdx.x + u * T;
-        if (t < (L / 2) * 2 * H) {
-            const int pp = t / (2 * H), r = t % (2 * H), which = r / H, k = r % H;
-            const float2 z = buf[pp * LD + k], zc = cconj(buf[pp * LD + ((L - k) % L)]);
-            o[u] = which == 0 ? cscale(cadd(z, zc), 0.5f) : make_float2(0.5f * (z.y - zc.y), -0.5f * (z.x - zc.x));
+        for (int u = 0; u < E; u++) {
+            const float2 z = buf[((rt >> 1) + T / 2 * u) * LR + C];  // real rows: Z(C) = X(C) of the one + i X(C) of the other
+            x[u] = make_float2(rt & 1 ? z.y : z.x, 0.f);
         }
-    }
-    __syncthreads();
+        row_fft<L, false>(x, rt, nyq_pen, tw);
 #pragma unroll
-    for (int u = 0; u < NS; u++) {
-        const int t = threadIdx.x + u * T;
-        if (t < (L / 2) * 2 * H) {
-            const int pp = t / (2 * H), r = t % (2 * H), which = r / H, k = r % H;
-            r2c_split_store<L>(buf, pp, which, k, o[u]);
-        }
+        for (int u = 0; u < E; u++) at_byte(ip + T * u * H, (rt * H + C) * 8) = x[u];
+    }
+#pragma unroll
+    for (int u = 0; u < E; u++) {
+        if (E > 8 && u % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+        const float2* pp = buf + ((ct >> 1) + T / 2 * u) * LR;
+        const float2 z = pp[c], zc = cconj(pp[cm]);
+        x[u] = ct & 1 ? make_float2(0.5f * (z.y - zc.y), -0.5f * (z.x - zc.x)) : cscale(cadd(z, zc), 0.5f);
     }
     __syncthreads();
-    pencil_fft<L>(&buf[q * LD], lane, tw, twc, false);
-    for (int t = threadIdx.x; t < L * H; t += blockDim.x) ip[t] = r2c_half_at<L>(buf, t / H, t % H);
+    col_fft<L, false, C>(x, ct, buf + c, tw);
+#pragma unroll
+    for (int u = 0; u < E; u++) at_byte(ip + T * u * H, (ct * H + c) * 8) = x[u];
 }
 
 // ------------------------------------------------------------------ combine + first DFT axis by FFT
@@ -920,14 +930,14 @@ __global__ void __launch_bounds__(ColShape<L>::THREADS) k_ccc_combine(const floa
     const int p = blockIdx.x * S::P + threadIdx.x % S::P;  // pencil (j, k) = (p / H, p % H)
     const bool valid = p < LH;
     const int pc = valid ? p : 0;
-    const size_t vol = (size_t)e * L * LH + pc;
+    const size_t vol = (size_t)e * L * LH;
+    const unsigned lo = (t * LH + pc) * 8;  // byte offset of this thread's first element of a spectrum
     float2* __restrict__ xp = ex + threadIdx.x % S::P;
     float2 f1[NE], q[NE];
 #pragma unroll
     for (int u = 0; u < NE; u++) {
-        const size_t h = vol + (size_t)(t + u * T) * LH;
-        f1[u] = ld_stream(&F1m[h]);
-        q[u] = ld_stream(&Q[h]);
+        f1[u] = ld_stream(&at_byte(F1m + vol + u * T * LH, lo));
+        q[u] = ld_stream(&at_byte(Q + vol + u * T * LH, lo));
     }
     for (int i = threadIdx.x; i < L; i += S::THREADS) {
         tw[i] = twg[i];
@@ -946,10 +956,9 @@ __global__ void __launch_bounds__(ColShape<L>::THREADS) k_ccc_combine(const floa
     const float a = sg * (2.f * (float)(L * L * L) / (n1 * n2)), b = sg / (n2 * n2);
 #pragma unroll
     for (int u = 0; u < NE; u++) {
-        const size_t i = t + u * T;
-        const float2 f2 = ld_stream(&F2[vol + i * LH]), m = Mfft[i * LH + pc];
+        const float2 f2 = ld_stream(&at_byte(F2 + vol + u * T * LH, lo)), m = at_byte(Mfft + u * T * LH, lo);
         f1[u] = csub(cscale(cmulc(f1[u], f2), a), cscale(cmulc(m, q[u]), b));
-        q[u] = cmul(f1[u], wb[i]);
+        q[u] = cmul(f1[u], wb[t + u * T]);
     }
     // element f mod L = i + L/2 mod L: a rotation of the slots by HS
 #pragma unroll
@@ -1000,7 +1009,7 @@ __global__ void __launch_bounds__(BcShape<L>::THREADS) k_ccc_dftBC(const float2*
         const bool live = t < T && k < H;
         float2 v[NE];
 #pragma unroll
-        for (int u = 0; u < NE; u++) v[u] = live ? src[(t + u * T) * H + k] : make_float2(0.f, 0.f);
+        for (int u = 0; u < NE; u++) v[u] = live ? at_byte(src + u * T * H, (t * H + k) * 8) : make_float2(0.f, 0.f);
         if (r == 0) {
             for (int i = threadIdx.x; i < L; i += NT) {
                 tw[i] = twg[i];
@@ -1253,7 +1262,7 @@ static void launch_planes(const FftTables& T, const PlaneOps& a, hipStream_t s) 
     const unsigned nb = a.planes * (a.io1 ? 2 : 1);
     static const std::string name = "k_c2r_r2c_plane<" + std::to_string(L) + ">";
     ProfScope ps(T.prof, name.c_str(), 2.0 * nb * L * (L / 2 + 1) * sizeof(float2), s);
-    k_c2r_r2c_plane<L><<<nb, Plane<L>::THREADS, 0, s>>>(a, tw);
+    k_c2r_r2c_plane<L><<<nb, OpPlane<L>::THREADS, 0, s>>>(a, tw);
 }
 template <int L>
 static void launch_c2r_op_r2c(const FftTables& T, const float2* in, float2* io, int batch, int op, const float* aux,

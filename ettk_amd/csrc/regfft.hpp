@@ -207,4 +207,52 @@ __device__ __forceinline__ void col_fft(float2* x, int t, float2* ex, const floa
     __syncthreads();
 }
 
+// The same transform for a pencil whose T threads are consecutive lanes of one wavefront: `pen` is the pencil's own
+// exchange storage, kRowLd<L> complex values, and the exchange needs only the wavefront's LDS order.  Rows of N2 + 1 and a
+// pencil stride of 16 banks (T = 8) or 8 or 24 banks (T = 4) modulo 32 let neither the writes nor the reads of half a
+// wavefront collide in LDS banks.
+template <int L>
+static constexpr int kRowLd = ColShape<L>::N1 * (ColShape<L>::N2 + 1) + (L == 128 ? 8 : L == 32 ? 4 : 0);
+// Orders the LDS accesses of one wavefront: the LDS instructions of a wavefront execute in order, so threads of
+// one wavefront exchanging data through LDS only need the compiler kept from reordering those accesses.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+template <int L, bool INV>
+__device__ __forceinline__ void row_fft(float2* x, int t, float2* pen, const float2* tw) {
+    using S = ColShape<L>;
+    constexpr int T = S::T, N1 = S::N1, N2 = S::N2, S2 = N2 / T, S1 = N1 / T;
+#pragma unroll
+    for (int i = 0; i < S2; i++) {
+        float2 v[N1];
+#pragma unroll
+        for (int m = 0; m < N1; m++) v[m] = x[i + S2 * m];
+        Dft<N1, INV>::run(v);
+        const int b = t + T * i;
+#pragma unroll
+        for (int k = 0; k < N1; k++) {
+            if (k > 0) {
+                float2 w = tw[b * k];
+                if (INV) w.y = -w.y;
+                v[k] = cmul(v[k], w);
+            }
+            pen[k * (N2 + 1) + b] = v[k];
+        }
+    }
+    wave_lds_order();
+#pragma unroll
+    for (int i = 0; i < S1; i++) {
+        float2 v[N2];
+        const int k1 = t + T * i;
+#pragma unroll
+        for (int b = 0; b < N2; b++) v[b] = pen[k1 * (N2 + 1) + b];
+        Dft<N2, INV>::run(v);
+#pragma unroll
+        for (int k = 0; k < N2; k++) x[i + S1 * k] = v[k];
+    }
+    wave_lds_order();
+}
+
 }  // namespace ettk
