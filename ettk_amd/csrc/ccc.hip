@@ -55,55 +55,67 @@ __device__ __forceinline__ bool inside_fp64(const double* md, int i, int j, int 
 }
 
 // One workgroup reslices an 8x8x8 tile of the output from the LDS-staged box of the particle (tricubic.hpp).
-// Measured on 256 evaluations at 64^3 (one launch): 654 us, against 775 us for an 18^3 box at strides 19/343,
-// 8x8 planes per wavefront and two reductions; outputs bit-identical.
 // kUse names the caller in kernel traces (0: CCC evaluations, 1: S^2 projection); the code is the same
 template <int kUse>
-__global__ void __launch_bounds__(kThreads) k_reslice(const float* __restrict__ parts, const EvalGeom* __restrict__ geom,
+__global__ void __launch_bounds__(kThreads, 7) k_reslice(const float* __restrict__ parts, const EvalGeom* __restrict__ geom,
                                                        int N, float* __restrict__ out, float* __restrict__ partials) {
     static_assert(kThreads == kTriThreads, "the staging's thread map");
     __shared__ float2 sh[kThreads / 64];
-    __shared__ float box[kBox * kSZ];
+    __shared__ float box[kBoxWords];
     int e, tb;
     xcd_eval_tile(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, e, tb);
-    const EvalGeom g = geom[e];
-    const float* vol = parts + (size_t)g.particle * N * N * N;
-    const long n3 = (long)N * N * N;
+    const EvalGeom& g = geom[e];
+    const size_t n3 = (size_t)N * N * N;
+    const float* vol = parts + g.particle * n3;
     const int nt = N / kTile;
-    const int ti = tb / (nt * nt), tj = (tb / nt) % nt, tk = tb % nt;
-    const int i0 = ti * kTile, j0 = tj * kTile, k0 = tk * kTile;
+    const int i0 = tb / (nt * nt) * kTile, j0 = (tb / nt) % nt * kTile, k0 = tb % nt * kTile;
     int lo[3], hi[3];
-    const bool fits = tile_box(g.m, i0, j0, k0, lo, hi);
+    bool inside;
+    const bool fits = tile_box(g.m, i0, j0, k0, N, N, N, lo, hi, inside);
     if (fits) stage_tile_box(vol, N, N, N, lo, hi, box);
+    const int lo1[3] = {lo[0] + 1, lo[1] + 1, lo[2] + 1};
+    int i, j, k;
+    tile_voxel(i, j, k);
+    i += i0;
+    j += j0;
+    k += k0;
+    const float fj = (float)j, fk = (float)k;
+    float pjk[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) pjk[a] = g.m[3 + a] * fj + g.m[6 + a] * fk;
+    float* __restrict__ oe = out + e * n3;
+    const unsigned off = ((i * N + j) * N + k) * 4u;
     __syncthreads();
-    float s = 0.f, c = 0.f;
+    float s = 0.f;
+    int c = 0;
     const float lob = -0.5f, hib = (float)N - 0.5f;
-    for (int t = threadIdx.x; t < kTile * kTile * kTile; t += blockDim.x) {
-        int i, j, k;
-        tile_voxel(t, i, j, k);
-        i += i0;
-        j += j0;
-        k += k0;
-        float px = g.m[0] * i + g.m[3] * j + g.m[6] * k + g.m[9];
-        float py = g.m[1] * i + g.m[4] * j + g.m[7] * k + g.m[10];
-        float pz = g.m[2] * i + g.m[5] * j + g.m[8] * k + g.m[11];
-        float v = -FLT_MAX;
-        bool in = px >= lob && px <= hib && py >= lob && py <= hib && pz >= lob && pz <= hib;
-        if (near_border(px, lob, hib) || near_border(py, lob, hib) || near_border(pz, lob, hib))
-            in = inside_fp64(g.md, i, j, k, -0.5, N - 0.5, N - 0.5, N - 0.5);
-        if (in) {
-            v = fits ? sample_box(box, lo, hi, px, py, pz) : sample_global(vol, N, N, N, px, py, pz);
+#pragma unroll
+    for (int h = 0; h < 2; h++, i += 4) {
+        const float fi = (float)i;
+        const float px = g.m[0] * fi + pjk[0] + g.m[9];
+        const float py = g.m[1] * fi + pjk[1] + g.m[10];
+        const float pz = g.m[2] * fi + pjk[2] + g.m[11];
+        float v;
+        if (inside && fits) {
+            v = sample_box(box, lo1, px, py, pz);
             s += v;
-            c += 1.f;
+            c += 64;
+        } else {
+            bool in = px >= lob && px <= hib && py >= lob && py <= hib && pz >= lob && pz <= hib;
+            if (near_border(px, lob, hib) || near_border(py, lob, hib) || near_border(pz, lob, hib))
+                in = inside_fp64(g.md, i, j, k, -0.5, N - 0.5, N - 0.5, N - 0.5);
+            v = -FLT_MAX;
+            if (in) {
+                v = fits ? sample_box(box, lo1, px, py, pz) : sample_global(vol, N, N, N, px, py, pz);
+                s += v;
+            }
+            c += __popcll(__ballot(in));
         }
-        out[(size_t)e * n3 + ((size_t)i * N + j) * N + k] = v;
+        at_byte(oe + (size_t)h * 4 * N * N, off) = v;
     }
-    // the tile's (sum, count) in one reduction: butterfly per wavefront, then the wavefronts in order
-    for (int o = 32; o > 0; o >>= 1) {
-        s += __shfl_xor(s, o, 64);
-        c += __shfl_xor(c, o, 64);
-    }
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = make_float2(s, c);
+    // the tile's (sum, count): per wavefront, then the wavefronts in order
+    s = wave_sum_last(s);
+    if ((threadIdx.x & 63) == 63) sh[threadIdx.x >> 6] = make_float2(s, (float)c);
     __syncthreads();
     if (threadIdx.x == 0) {
         float ts = 0.f, tc = 0.f;

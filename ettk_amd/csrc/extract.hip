@@ -21,11 +21,11 @@ constexpr int kExT = kTriThreads;
 // One workgroup per 8x8x8 tile of an output box, interpolated from the LDS-staged box of the tomogram its stencils
 // touch (tricubic.hpp); tiles at the far sides of a box whose size is not a multiple of 8 are partial.  Per-tile
 // (sum, count) of the valid samples.  Bound by the LDS reads of the taps, as the CCC reslice.  The call on 60 boxes of
-// 64^3 takes 216 us; with every tap read from global memory it took 1558 us.
-__global__ void __launch_bounds__(kExT) k_extract(const float* __restrict__ tomo, int nx, int ny, int nz,
+// 64^3 takes 201 us; with every tap read from global memory it took 1558 us.
+__global__ void __launch_bounds__(kExT, 7) k_extract(const float* __restrict__ tomo, int nx, int ny, int nz,
                                                   const ExtractGeom* __restrict__ geom, int N, float* __restrict__ out,
                                                   float* __restrict__ partials) {
-    __shared__ float box[kBox * kSZ];
+    __shared__ float box[kBoxWords];
     __shared__ float sh[2][kExT / 64];
     int p, tb;
     xcd_eval_tile(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, p, tb);  // neighbouring tiles share their lines in one L2
@@ -34,46 +34,48 @@ __global__ void __launch_bounds__(kExT) k_extract(const float* __restrict__ tomo
     const int nt = (N + kTile - 1) / kTile;
     const int z0 = (tb / (nt * nt)) * kTile, y0 = ((tb / nt) % nt) * kTile, x0 = (tb % nt) * kTile;
     int lo[3], hi[3];
-    const bool fits = tile_box(g.m, x0, y0, z0, lo, hi);
+    bool inside;
+    const bool fits = tile_box(g.m, x0, y0, z0, nx, ny, nz, lo, hi, inside);
     if (fits) stage_tile_box(tomo, nx, ny, nz, lo, hi, box);
+    const int lo1[3] = {lo[0] + 1, lo[1] + 1, lo[2] + 1};
+    int x, y, z;
+    tile_voxel(z, y, x);
+    x += x0;
+    y += y0;
+    z += z0;
     __syncthreads();
-    float s = 0.f, c = 0.f;
+    float s = 0.f;
+    int c = 0;
     const float hx = nx - 0.5f, hy = ny - 0.5f, hz = nz - 0.5f;
-    for (int t = threadIdx.x; t < kTile * kTile * kTile; t += kExT) {
-        int x, y, z;
-        tile_voxel(t, z, y, x);
-        x += x0;
-        y += y0;
-        z += z0;
-        if (x >= N || y >= N || z >= N) continue;
+#pragma unroll 1
+    for (int h = 0; h < 2; h++, z += 4) {
+        const bool live = x < N && y < N && z < N;
         const float px = g.m[0] * x + g.m[3] * y + g.m[6] * z + g.m[9];
         const float py = g.m[1] * x + g.m[4] * y + g.m[7] * z + g.m[10];
         const float pz = g.m[2] * x + g.m[5] * y + g.m[8] * z + g.m[11];
         float v = -FLT_MAX;
-        bool in = px >= -0.5f && px <= hx && py >= -0.5f && py <= hy && pz >= -0.5f && pz <= hz;
+        bool in = inside || (px >= -0.5f && px <= hx && py >= -0.5f && py <= hy && pz >= -0.5f && pz <= hz);
         auto near = [](float p, float hi) { return fabsf(p + 0.5f) < 1e-3f || fabsf(p - hi) < 1e-3f; };
-        if (near(px, hx) || near(py, hy) || near(pz, hz)) {
+        if (!inside && (near(px, hx) || near(py, hy) || near(pz, hz))) {
             const double* md = g.md;
             const double qx = md[0] * x + md[3] * y + md[6] * z + md[9];
             const double qy = md[1] * x + md[4] * y + md[7] * z + md[10];
             const double qz = md[2] * x + md[5] * y + md[8] * z + md[11];
             in = qx >= -0.5 && qx <= nx - 0.5 && qy >= -0.5 && qy <= ny - 0.5 && qz >= -0.5 && qz <= nz - 0.5;
         }
+        in = in && live;
         if (in) {
-            v = fits ? sample_box(box, lo, hi, px, py, pz) : sample_global(tomo, nx, ny, nz, px, py, pz);
+            v = fits ? sample_box(box, lo1, px, py, pz) : sample_global(tomo, nx, ny, nz, px, py, pz);
             s += v;
-            c += 1.f;
         }
-        out[(size_t)p * n3 + ((size_t)z * N + y) * N + x] = v;
+        c += __popcll(__ballot(in));
+        if (live) out[(size_t)p * n3 + ((size_t)z * N + y) * N + x] = v;
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        s += __shfl_down(s, off, 64);
-        c += __shfl_down(c, off, 64);
-    }
+    s = wave_sum_last(s);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) {
+    if (lane == 63) {
         sh[0][w] = s;
-        sh[1][w] = c;
+        sh[1][w] = (float)c;
     }
     __syncthreads();
     if (threadIdx.x == 0) {

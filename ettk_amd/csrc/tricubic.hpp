@@ -8,14 +8,24 @@
 // consecutive words.  A non-rigid map whose box does not fit reads the clamped taps from global memory instead.
 // Each wavefront interpolates a 4x4x4 block of the tile: the taps of its voxels then cover a compact region of the
 // box and, with the row and plane strides 17 and 300, fall on fewer common LDS banks than those of an 8x8 plane.  A
-// 17^3 box at these strides (20 KB) lets 8 workgroups share a CU's 160 KB of LDS.
+// 17^3 box at these strides (20 KB) lets 7 workgroups share a CU.
+//
+// Bound by LDS and VALU together (both 83% busy; the taps' words collide on banks 2.9 times in half a wavefront), so the
+// rest of a tile is kept cheap: the box's bounds and the staging's plane addresses are scalar, tiles away from the
+// volume's border test no sample, the box has a margin instead of a clamp per sample, counts are ballots and sums DPP.
+// 240 evaluations at 64^3: 605 us, 686 before; extraction of 60 boxes 157 against 176 us.  Layouts that trade bank
+// conflicts for address arithmetic are slower: voxel (x, y, z) on bank (x & 3) + 4 (y & 3) + 16 (z & 1) with the taps
+// visited in a lane's own conflict-free order 675 us (VALU-bound, 1.5 times the instructions), without the z digit 721;
+// pairs or quads of words per voxel read 20% faster by themselves but leave 3 workgroups or fewer per CU.
 #pragma once
 #include "common.hpp"
 
 namespace ettk {
 
 static constexpr int kTriThreads = 256;
-static constexpr int kTile = 8, kBox = 17, kSY = 17, kSZ = 300;
+static constexpr int kTile = 8, kBox = 17;
+static constexpr int kSY = 17, kSZ = 300, kBoxWords = kBox * kSZ;
+static_assert(kBox % 6 == 5, "the staging writes planes in sixes, the last five");
 static constexpr float kTriTol = 7.62939453125e-06f;  // VTK's floor tolerance (2^-17)
 
 __device__ __forceinline__ void keys_w(float f, float* w) {  // vtkTricubicInterpWeights
@@ -27,67 +37,97 @@ __device__ __forceinline__ void keys_w(float f, float* w) {  // vtkTricubicInter
 }
 
 // staged box [lo, hi] per input axis (x, y, z) of the tile at (i0, j0, k0) under the map m (columns of the output axes,
-// then the offset); it may reach outside the volume.  False when the map's box does not fit.
-__device__ __forceinline__ bool tile_box(const float* m, int i0, int j0, int k0, int lo[3], int hi[3]) {
+// then the offset); it may reach outside the volume.  A margin of 1e-3 voxels keeps every sample's stencil in the box
+// whatever FP32 rounding does to its position.  False when the map's box does not fit.  `inside`: every sample of the
+// tile lies in an nx x ny x nz volume, away from its border, so that no sample's validity needs a test.
+__device__ __forceinline__ bool tile_box(const float* m, int i0, int j0, int k0, int nx, int ny, int nz, int lo[3],
+                                         int hi[3], bool& inside) {
     bool fits = true;
+    inside = true;
+    const int n[3] = {nx, ny, nz};
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         float c0 = m[a] * i0 + m[3 + a] * j0 + m[6 + a] * k0 + m[9 + a];
         float ext = (kTile - 1) * (fabsf(m[a]) + fabsf(m[3 + a]) + fabsf(m[6 + a]));
         float mn = c0 + (kTile - 1) * (fminf(m[a], 0.f) + fminf(m[3 + a], 0.f) + fminf(m[6 + a], 0.f));
-        lo[a] = (int)floorf(mn + kTriTol) - 1;
-        hi[a] = (int)floorf(mn + ext + kTriTol) + 2;
+        // the same for every thread: kept in scalar registers, and with them the staging's row and plane arithmetic
+        lo[a] = __builtin_amdgcn_readfirstlane((int)floorf(mn - 1e-3f) - 1);
+        hi[a] = __builtin_amdgcn_readfirstlane((int)floorf(mn + ext + 1e-3f) + 2);
         if (!(hi[a] - lo[a] + 1 <= kBox) || !(fabsf(mn) < 1e6f)) fits = false;
+        if (!(mn > -0.49f && mn + ext < (float)n[a] - 0.51f)) inside = false;
     }
+    // the staging's offsets within a plane are 32-bit bytes; positions beyond 1e4 voxels round by more than the margin
+    if ((unsigned long long)nx * ny >= (1ull << 30) || !(fmaxf((float)nx, fmaxf((float)ny, (float)nz)) < 1e4f)) fits = false;
     return fits;
 }
 
-// the box into LDS (kBox * kSZ floats): a 2-D thread map over (y, x), a loop over z, coordinates clamped to the volume
+// the box into LDS (kBoxWords floats): a 2-D thread map over (y, x), a loop over z whose plane addresses are scalar,
+// coordinates clamped to the volume
 __device__ __forceinline__ void stage_tile_box(const float* __restrict__ vol, int nx, int ny, int nz, const int lo[3],
                                                const int hi[3], float* box) {
     constexpr int kRows = kTriThreads / kBox;
-    const int t = threadIdx.x;
+    const int x = threadIdx.x % kBox, y0 = threadIdx.x / kBox;
     const int wx = hi[0] - lo[0] + 1, wy = hi[1] - lo[1] + 1, wz = hi[2] - lo[2] + 1;
-    const int x = t % kBox, y0 = t / kBox;
-    if (t < kBox * kRows && x < wx) {
-        const int gx = min(max(lo[0] + x, 0), nx - 1);
-        for (int y = y0; y < wy; y += kRows) {
+    const size_t plane = (size_t)nx * ny;
+    const int gx = min(max(lo[0] + x, 0), nx - 1);
+#pragma unroll
+    for (int pass = 0; pass < (kBox + kRows - 1) / kRows; pass++) {
+        const int y = y0 + pass * kRows;
+        if (y0 < kRows && x < wx && y < wy) {
             const int gy = min(max(lo[1] + y, 0), ny - 1);
-            const float* src = vol + (size_t)gy * nx + gx;
-#pragma unroll 6
-            for (int z = 0; z < wz; z++) {
-                const int gz = min(max(lo[2] + z, 0), nz - 1);
-                box[z * kSZ + y * kSY + x] = src[(size_t)gz * ny * nx];
+            const unsigned off = ((unsigned)gy * nx + gx) * 4u;
+            float* dst = box + y * kSY + x;
+            // the plane's address advances in scalar registers; it stays where the clamped coordinate does
+            const float* src = vol + (size_t)min(max(lo[2], 0), nz - 1) * plane;
+            for (int z = 0; z < wz; z += 6, dst += 6 * kSZ) {  // six loads in flight; planes past the box are written unused
+                float r[6];
+#pragma unroll
+                for (int u = 0; u < 6; u++) {
+                    r[u] = at_byte(src, off);
+                    const unsigned g = (unsigned)(lo[2] + z + u);  // step from this plane to the next one inside the volume
+                    src += g < (unsigned)(nz - 1) ? plane : 0;
+                }
+#pragma unroll
+                for (int u = 0; u < 5; u++) dst[u * kSZ] = r[u];
+                if (z + 5 < kBox) dst[5 * kSZ] = r[5];
             }
         }
     }
 }
 
-// voxel (offset within the tile) of item t < 512: t >> 6 numbers the tile's eight 4x4x4 blocks, t & 63 the voxel
-// within its block; axis c runs fastest
-__device__ __forceinline__ void tile_voxel(int t, int& a, int& b, int& c) {
-    const int sb = t >> 6, l = t & 63;
-    a = 4 * (sb >> 2) + (l >> 4);
-    b = 4 * ((sb >> 1) & 1) + ((l >> 2) & 3);
-    c = 4 * (sb & 1) + (l & 3);
+// Thread t of the workgroup takes voxel (a, b, c) of the tile and voxel (a + 4, b, c): a 4x4x4 block per wavefront, axis c
+// fastest.
+__device__ __forceinline__ void tile_voxel(int& a, int& b, int& c) {
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    a = l >> 4;
+    b = 4 * ((w >> 1) & 1) + ((l >> 2) & 3);
+    c = 4 * (w & 1) + (l & 3);
 }
 
-// the sample at (px, py, pz) from the staged box
-__device__ __forceinline__ float sample_box(const float* box, const int lo[3], const int hi[3], float px, float py,
-                                            float pz) {
+// sum over a wavefront, in its last lane: row shifts, then row broadcasts (a fixed order, no LDS)
+__device__ __forceinline__ float wave_sum_last(float v) {
+#define ETTK_DPP_ADD(ctrl, rows) \
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rows, 0xf, false))
+    ETTK_DPP_ADD(0x111, 0xf);  // row_shr:1
+    ETTK_DPP_ADD(0x112, 0xf);  // row_shr:2
+    ETTK_DPP_ADD(0x114, 0xf);  // row_shr:4
+    ETTK_DPP_ADD(0x118, 0xf);  // row_shr:8
+    ETTK_DPP_ADD(0x142, 0xa);  // row_bcast:15
+    ETTK_DPP_ADD(0x143, 0xc);  // row_bcast:31
+#undef ETTK_DPP_ADD
+    return v;
+}
+
+// the sample at (px, py, pz) from the staged box, whose voxel lo + 1 is lo1
+__device__ __forceinline__ float sample_box(const float* box, const int lo1[3], float px, float py, float pz) {
     const float xx = px + kTriTol, yy = py + kTriTol, zz = pz + kTriTol;
-    int ix = (int)floorf(xx), iy = (int)floorf(yy), iz = (int)floorf(zz);
-    // the box was sized from the tile's corners; a sample within rounding of a voxel boundary can floor one voxel
-    // outside it: take the neighbouring cubic piece at f just outside [0, 1) instead (the Keys kernel is C1, the
-    // value agrees to O(f^2) of a few ulps)
-    ix = min(max(ix, lo[0] + 1), hi[0] - 2);
-    iy = min(max(iy, lo[1] + 1), hi[1] - 2);
-    iz = min(max(iz, lo[2] + 1), hi[2] - 2);
+    const float fx = floorf(xx), fy = floorf(yy), fz = floorf(zz);
+    const int x0 = (int)fx - lo1[0], y0 = (int)fy - lo1[1], z0 = (int)fz - lo1[2];  // the stencil's start in the box
     float wx[4], wy[4], wz[4];
-    keys_w(xx - ix, wx);
-    keys_w(yy - iy, wy);
-    keys_w(zz - iz, wz);
-    const float* b0 = box + (iz - 1 - lo[2]) * kSZ + (iy - 1 - lo[1]) * kSY + (ix - 1 - lo[0]);
+    keys_w(xx - fx, wx);
+    keys_w(yy - fy, wy);
+    keys_w(zz - fz, wz);
+    const float* b0 = box + z0 * kSZ + y0 * kSY + x0;
     float acc = 0.f;
 #pragma unroll
     for (int a = 0; a < 4; a++) {
