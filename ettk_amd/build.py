@@ -21,7 +21,7 @@ HIP_FLAGS = ["-O3", "--offload-arch=gfx950", "-std=c++17", "-fPIC", "-Wall", "-W
 # align.cpp runs the Powell refinements as C++20 coroutines
 STD_OVERRIDE = {"align.cpp": "-std=c++20"}
 SOURCES = ["fft.hip", "ccc.hip", "so3.hip", "refine.hip", "host.cpp", "align.cpp", "refine.cpp", "avg.hip", "avg.cpp",
-           "noalloc.hip", "extract.hip", "classify.cpp", "tune.cpp", "cand.hip"]
+           "noalloc.hip", "extract.hip", "project.hip", "classify.cpp", "tune.cpp", "cand.hip"]
 
 
 def build_lib(verbose: bool = False) -> Path:

@@ -213,21 +213,6 @@ __device__ __forceinline__ float r2c_load(const R2CArgs& a, long row, int k) {
     long ij = row % ((long)L * L);
     int i = (int)(ij / L), j = (int)(ij % L);
     float sg = ((i + j + k) & 1) ? -1.0f : 1.0f;
-    if (a.pro == PRO_PAD_MASKED) {
-        // cartesianToSpherical (ProjRot.h:265-318): the masked image (image - mean) * mask + mean sits in the
-        // corner [0, ns)^3 of the (2 ns)^3 box, the rest holds the value of voxel (0,0,0); times (-1)^(i+j+k)
-        const long b = row / ((long)L * L);
-        const int ns = a.ns;
-        const float* st = a.stats + b * 4;
-        if (i < ns && j < ns && k < ns) {
-            long o = ((long)i * ns + j) * ns + k;
-            float x = a.in[b * (long)ns * ns * ns + o];
-            float img = (x == -3.402823466e+38f) ? 0.0f : x - st[0];
-            float v = st[3] != 0.f ? (img - st[1]) * a.aux0[o] + st[1] : img;
-            return v * sg;
-        }
-        return st[2] * sg;
-    }
     float x = a.in[row * L + k];
     if (a.pro == PRO_NONE) return x;
     switch (a.pro) {
@@ -660,12 +645,6 @@ __global__ void __launch_bounds__(Plane<L>::THREADS) k_r2c_plane(R2CArgs a, cons
             if (a.aux0) r2c_stage_plane<L, PRO_RESLICED, true>(a, pi, src, mean, buf);
             else r2c_stage_plane<L, PRO_RESLICED, false>(a, pi, src, mean, buf);
             break;
-        default:
-            for (int t = threadIdx.x; t < L * L; t += blockDim.x) {
-                const int j = t / L, x = t % L;
-                float* f = reinterpret_cast<float*>(&buf[(j >> 1) * LD + x]);
-                f[j & 1] = r2c_load<L>(a, ((long)pb * L + pi) * L + j, x);
-            }
     }
     if (threadIdx.x < L) tw[threadIdx.x] = twv;
     __syncthreads();
@@ -1200,8 +1179,7 @@ static void launch_r2c(const FftTables& T, const R2CArgs& a, float2* scratch, hi
     const float2* tw = T.tw.p + T.offset[fft_len_index(L)];
     long npairs = (long)a.batch * L * L / 2;
     const double vol_c = (double)a.batch * L * L * H * sizeof(float2);  // one pass over the half spectrum
-    const double vol_r = a.pro == PRO_PAD_MASKED ? (double)a.batch * a.ns * a.ns * a.ns * sizeof(float)
-                                                 : (double)a.batch * L * L * L * sizeof(float);
+    const double vol_r = (double)a.batch * L * L * L * sizeof(float);
     if constexpr (L <= 128) {
         // passes k and j fused per (b, i) plane
         ProfScope ps(T.prof, plane_name<L>(0), vol_r + vol_c, s);
@@ -1559,7 +1537,6 @@ void fft3_refine_adj_c2r(const FftTables& T, const float2* X1, const float2* FP,
 }
 
 void fft3_r2c_planes(const FftTables& T, const R2CArgs& a, hipStream_t s) {
-    ETTK_REQUIRE(a.pro != PRO_PAD_MASKED, ETTK_ERR_ARG, "fft3_r2c_planes: padded prologue not supported");
     switch (a.n) {
         case 16: launch_r2c_planes<16>(T, a, s); break;
         case 32: launch_r2c_planes<32>(T, a, s); break;

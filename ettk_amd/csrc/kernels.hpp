@@ -67,6 +67,18 @@ int fft3_ccc_ipass_blocks(int n);
 void fft3_ccc_ipass(const FftTables& T, const CccIpassArgs& a, int n, int batch, hipStream_t s);
 // the k/j plane passes of an r2c only (n <= 128): the i pass is left to fft3_ccc_ipass
 void fft3_r2c_planes(const FftTables& T, const R2CArgs& a, hipStream_t s);
+// |F| (|F|^(1/2) with mcf) of the box of (2n)^3 whose corner holds the masked image and whose rest its pad constant,
+// times (-1)^(i+j+k): mag[b][i][j][k], k = 0 .. n + 1 (the row repeats |F| past the middle by one element).  Elements
+// farther than `rad` from (n, n, n) are left as they are.
+struct PadMagArgs {
+    const float* in;     // [b][n][n][n]; -FLT_MAX: invalid
+    const float* mask;   // [n][n][n]
+    const float* stats;  // per image {valid mean, image mean, pad constant, mask on}
+    float2* F;           // workspace [b][n][2n][n + 2]
+    float* mag;          // [b][2n][2n][n + 2]
+    int batch, rad, mcf;
+};
+void fft3_pad_magnitude(const FftTables& T, const PadMagArgs& a, int n, hipStream_t s);
 // smoothed analytic wedge parameters of the reference
 struct WedgeRef {
     float v1[3], v2[3];

@@ -224,20 +224,11 @@ __global__ void __launch_bounds__(64) k_proj_final(const float* __restrict__ R, 
     }
 }
 
-// |F| (|F|^(1/2) with MCF) of the (2N)^3 half spectrum
-__global__ void k_magnitude(const float2* __restrict__ F, float* __restrict__ mag, long n, int mcf) {
-    for (long h = blockIdx.x * (long)blockDim.x + threadIdx.x; h < n; h += (long)gridDim.x * blockDim.x) {
-        float2 z = F[h];
-        float m2 = z.x * z.x + z.y * z.y;
-        mag[h] = mcf ? sqrtf(sqrtf(m2)) : sqrtf(m2);
-    }
-}
-
-// full-size magnitude volume as ProjRot.h:327-338 leaves it: A(i,j,k) for k <= M/2 is |F| except the i = 0
+// full-size magnitude volume (rows of M/2 + 2 stored, fft3_pad_magnitude) as ProjRot.h:327-338 leaves it: A(i,j,k) for k <= M/2 is |F| except the i = 0
 // plane (0); for k > M/2: i = 0 -> 0, j = 0 -> the pad constant (the loop never overwrites those voxels of
 // the padded image), otherwise the mirrored value |F|(M-i, M-j, M-k)
 __device__ __forceinline__ float mag_at(const float* __restrict__ mag, int M, int i, int j, int k, float padc) {
-    const int Hm = M / 2 + 1;
+    const int Hm = M / 2 + 2;
     if (i == 0) return 0.f;
     if (k <= M / 2) return mag[((size_t)i * M + j) * Hm + k];
     if (j == 0) return padc;
@@ -260,7 +251,7 @@ __global__ void __launch_bounds__(kT) k_sph_sample(const float* __restrict__ mag
     const int lane = threadIdx.x % kLanes;
     const bool live = t < n * n;
     const int jp = live ? t / n : 0, kt = live ? t % n : 0;
-    const float* mg = mag + (size_t)b * M * M * (M / 2 + 1);
+    const float* mg = mag + (size_t)b * M * M * (M / 2 + 2);
     const float padc = st[b * 4 + 2];
     const float Bf = (float)B;
     const double phi = M_PI / 4.0 / Bf + jp * (2.0 * M_PI / 4.0 / Bf);
@@ -282,13 +273,13 @@ __global__ void __launch_bounds__(kT) k_sph_sample(const float* __restrict__ mag
             w[a][2] = -((ft3 - 4) * f - 1) * fd2;
             w[a][3] = f * fd2 * fm1;
         }
-        // the 4x4x4 stencil lies inside the stored half (k <= M/2) or entirely in the mirrored half, away from the
-        // i = 0 plane, the j = 0 column of the mirror and the wrap: then its taps sit at fixed strides (the values
-        // mag_at would return); otherwise every tap goes through mag_at
-        const int i0 = idx[0] - 1, j0 = idx[1] - 1, k0 = idx[2] - 1, Hm = M / 2 + 1;
-        const bool ij_in = i0 >= 1 && i0 + 3 <= M - 1 && j0 >= 0 && j0 + 3 <= M - 1;
-        const bool direct = ij_in && k0 >= 0 && k0 + 3 <= M / 2;
-        const bool mirror = ij_in && j0 >= 1 && k0 >= M / 2 + 1 && k0 + 3 <= M - 1;
+        // the 4x4x4 stencil lies in the stored rows (k <= M/2 + 1) or its mirror image does, away from the i = 0 plane,
+        // the j = 0 column and the wrap: then its taps sit at fixed strides (the values mag_at would return);
+        // otherwise every tap goes through mag_at
+        const int i0 = idx[0] - 1, j0 = idx[1] - 1, k0 = idx[2] - 1, Hm = M / 2 + 2;
+        const bool ij_in = i0 >= 1 && i0 + 3 <= M - 1 && j0 >= 1 && j0 + 3 <= M - 1;
+        const bool direct = ij_in && k0 >= 0 && k0 + 3 <= M / 2 + 1;
+        const bool mirror = ij_in && !direct && k0 + 3 <= M - 1 && k0 >= M / 2 - 1;
         double v = 0;
         if (direct || mirror) {
             const long si = direct ? (long)M * Hm : -(long)M * Hm, sj = direct ? Hm : -Hm;
@@ -1215,12 +1206,12 @@ static int band_hi(const ettk_plan* P) {
 void project_images(ettk_plan* P, const float* d_parts, const ettk_particle* descs, const int* pidx, int n, bool is_ref,
                     float* d_Pp, const EvalGeom* h_geom) {
     So3State& S = so3(P);
-    const int N = P->N, M = 2 * N, B = S.B, Hm = N + 1;
-    const size_t n3 = (size_t)N * N * N, nbig = (size_t)M * M * Hm;
+    const int N = P->N, M = 2 * N, B = S.B;
+    const size_t n3 = (size_t)N * N * N, nbig = (size_t)M * M * (N + 2);
     hipStream_t s = P->stream;
     const int CH = 32;
     S.projR.ensure(n3 * CH);
-    S.projF.ensure(nbig * CH);
+    S.projF.ensure(nbig / 2 * CH);
     S.projMag.ensure(nbig * CH);
     S.projStats.ensure(4 * CH);
     S.projSum.ensure((size_t)kProjParts * CH);
@@ -1249,10 +1240,9 @@ void project_images(ettk_plan* P, const float* d_parts, const ettk_particle* des
         k_proj_final<<<cn, 64, 0, s>>>(S.projR.p, S.projSum.p, P->m1.p, N, P->p.mask_radius != 0.0f ? 1 : 0,
                                        S.projStats.p);
         ETTK_HIP(hipGetLastError());
-        R2CArgs a{S.projR.p, S.projF.p, M, cn, PRO_PAD_MASKED, P->m1.p, S.projStats.p, N};
-        fft3_r2c(P->ctx->fft, a, nullptr, s);
-        k_magnitude<<<2048, kT, 0, s>>>(S.projF.p, S.projMag.p, (long)nbig * cn, P->p.mcf);
-        ETTK_HIP(hipGetLastError());
+        // the stencils of the outermost shell reach 3.5 voxels past it; a wrapped tap lies nearer the centre
+        PadMagArgs a{S.projR.p, P->m1.p, S.projStats.p, S.projF.p, S.projMag.p, cn, band_hi(P) + 4, P->p.mcf};
+        fft3_pad_magnitude(P->ctx->fft, a, N, s);
         dim3 grid((4 * B * B + kT / kLanes - 1) / (kT / kLanes), cn);
         ProfScope ps(P->ctx->fft.prof, "k_sph_sample", (double)cn * ((double)nbig * 4 + 16.0 * B * B), s);
         k_sph_sample<<<grid, kT, 0, s>>>(S.projMag.p, S.projStats.p, M, B, band_lo(P), band_hi(P),

@@ -144,3 +144,31 @@ def test_ccc_windows(torch_gpu, ctx, N, window):
             assert np.abs(out[i] - m).max() < 1e-9 or peak_tie(orc, ps.vols[i], ps.descs[i], t[i], out[i])[0]
     finally:
         plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,band,mask", [(16, (0.0, 0.5), True), (48, (0.0, 0.5), False), (96, (0.1, 0.3), True),
+                                         (128, (0.0, 0.5), True)])
+def test_projection_box_sizes(torch_gpu, ctx, N, band, mask):
+    """The padded spectrum at every pencil shape (the smallest box, 4 threads and 24 elements per pencil, the
+    largest with the narrower column steps), with a band that leaves most of it out and without the mask.  FP32
+    transforms of (2N)^3 elements: 2^-24 per level, at most 24 levels, is 1.5e-6 of the rms magnitude per
+    element; the 4..128 shells of one ray add to at least their mean, so 1e-5 of the largest value leaves a factor of 6."""
+    from ettk_amd.lib import Plan
+    from oracle_lib import OraclePlan
+
+    p = default_params(N, 8, mask_radius=(N / 2 - 3) if mask else 0.0, square_mask=2, bp_lo=band[0], bp_hi=band[1])
+    g = np.random.default_rng(N)
+    ps = make_particles(blob_reference(N, seed=3), 2, seed=4, half_wedge=(50, 60), snr=(0.5, 0.5), max_shift=1.0)
+    vols = (ps.vols / ps.vols.std() + g.standard_normal(ps.vols.shape) + 1.0).astype(np.float32)
+    plan, orc = Plan(ctx, p), OraclePlan(p)
+    try:
+        pp = plan.project(to_dev(torch_gpu, vols), ps.descs)
+        err = 0.0
+        for i in range(2):
+            want = orc.project(vols[i], ps.descs[i])
+            err = max(err, np.abs(pp[i] - want).max() / np.abs(want).max())
+        print(f"[edges] projection N={N} band {band} mask {mask} err {err:.2e}", flush=True)
+        assert err < 1e-5
+    finally:
+        plan.close()
