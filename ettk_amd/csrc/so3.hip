@@ -235,100 +235,184 @@ __device__ __forceinline__ float mag_at(const float* __restrict__ mag, int M, in
     return mag[((size_t)(M - i) * M + (M - j)) * Hm + (M - k)];
 }
 
-// One S^2 sample per group of kLanes consecutive threads; the radial shells r = bandL..bandU are split over the
-// lanes and summed with wavefront shuffles.  Tricubic Keys weights (a = -1/2) with the 2^-17 floor tolerance
-// and wrap-around taps, FP64 like the double image of the reference.
 static constexpr int kLanes = 8;
 __device__ __forceinline__ int wrap_idx(int x, int M) { return x < 0 ? x + M : (x >= M ? x - M : x); }
 
-__global__ void __launch_bounds__(kT) k_sph_sample(const float* __restrict__ mag, const float* __restrict__ st, int M,
-                                                    int B, int bandL, int bandU, float* __restrict__ Pp) {
-    // one particle per XCD at a time: its magnitude volume is gathered through that XCD's L2 only
-    int b, tile;
-    xcd_eval_tile(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, b, tile);
-    const int n = 2 * B;
-    const int t = tile * (kT / kLanes) + threadIdx.x / kLanes;
-    const int lane = threadIdx.x % kLanes;
-    const bool live = t < n * n;
-    const int jp = live ? t / n : 0, kt = live ? t % n : 0;
-    const float* mg = mag + (size_t)b * M * M * (M / 2 + 2);
-    const float padc = st[b * 4 + 2];
-    const float Bf = (float)B;
-    const double phi = M_PI / 4.0 / Bf + jp * (2.0 * M_PI / 4.0 / Bf);
-    const double th = kt * (M_PI / Bf);
-    const double sp = sin(phi), cp = cos(phi), ct = cos(th), stt = sin(th);
-    const double origin = -(M - 1) / 2.0 - 0.5;
-    double sum = 0;
-    for (int r = bandL + lane; live && r <= bandU; r += kLanes) {
-        double p[3] = {r * sp * ct - origin, r * sp * stt - origin, r * cp - origin};
-        int idx[3];
-        double w[3][4];
+// Tricubic Keys weights (a = -1/2) with the 2^-17 floor tolerance and wrap-around taps, FP64 like the double image of the
+// reference.  Sums run along k first: a row of 4 taps is one load and is used up before the next.
+struct SphStencil {
+    int lo[3];       // first tap
+    double w[3][4];
+    __device__ __forceinline__ void set(const double* p) {
+        for (int a = 0; a < 3; a++) lo[a] = (int)floor(p[a] + 7.62939453125e-06) - 1;
+        weigh(p);
+    }
+    __device__ __forceinline__ void weigh(const double* p) {
         for (int a = 0; a < 3; a++) {
-            double xx = p[a] + 7.62939453125e-06;
-            idx[a] = (int)floor(xx);
-            double f = xx - idx[a];
+            double f = p[a] + 7.62939453125e-06 - (lo[a] + 1);
             double fm1 = f - 1, fd2 = f * 0.5, ft3 = f * 3;
             w[a][0] = -fd2 * fm1 * fm1;
             w[a][1] = ((ft3 - 2) * fd2 - 1) * fm1;
             w[a][2] = -((ft3 - 4) * f - 1) * fd2;
             w[a][3] = f * fd2 * fm1;
         }
-        // the 4x4x4 stencil lies in the stored rows (k <= M/2 + 1) or its mirror image does, away from the i = 0 plane,
-        // the j = 0 column and the wrap: then its taps sit at fixed strides (the values mag_at would return);
-        // otherwise every tap goes through mag_at
-        const int i0 = idx[0] - 1, j0 = idx[1] - 1, k0 = idx[2] - 1, Hm = M / 2 + 2;
-        const bool ij_in = i0 >= 1 && i0 + 3 <= M - 1 && j0 >= 1 && j0 + 3 <= M - 1;
-        const bool direct = ij_in && k0 >= 0 && k0 + 3 <= M / 2 + 1;
-        const bool mirror = ij_in && !direct && k0 + 3 <= M - 1 && k0 >= M / 2 - 1;
-        double v = 0;
-        if (direct || mirror) {
-            const long si = direct ? (long)M * Hm : -(long)M * Hm, sj = direct ? Hm : -Hm;
-            const float* pb = direct ? mg + ((long)i0 * M + j0) * Hm + k0
-                                     : mg + ((long)(M - i0) * M + (M - j0)) * Hm + (M - k0);
-            // the 4 taps along k of row (cx, cy) are consecutive floats (ascending in the stored half, descending
-            // in the mirror): one 16-byte load at their 4-byte-aligned start (global loads of four dwords need
-            // only dword alignment on this architecture)
-            float tap[4][4][4];  // [cz][cy][cx]
-#pragma unroll
-            for (int cy = 0; cy < 4; cy++)
-#pragma unroll
-                for (int cx = 0; cx < 4; cx++) {
-                    const float* lo4 = pb + cy * sj + cx * si - (direct ? 0 : 3);
-                    float r[4];
-                    __builtin_memcpy(r, lo4, sizeof(r));
-#pragma unroll
-                    for (int cz = 0; cz < 4; cz++) tap[cz][cy][cx] = direct ? r[cz] : r[3 - cz];
-                }
-#pragma unroll
-            for (int cz = 0; cz < 4; cz++) {
-                double vy = 0;
-#pragma unroll
-                for (int cy = 0; cy < 4; cy++) {
-                    double vx = 0;
-#pragma unroll
-                    for (int cx = 0; cx < 4; cx++) vx += w[0][cx] * (double)tap[cz][cy][cx];
-                    vy += w[1][cy] * vx;
-                }
-                v += w[2][cz] * vy;
-            }
-        } else {
-            for (int cz = 0; cz < 4; cz++) {
-                const int kz = wrap_idx(idx[2] - 1 + cz, M);
-                double vy = 0;
-                for (int cy = 0; cy < 4; cy++) {
-                    const int jy = wrap_idx(idx[1] - 1 + cy, M);
-                    double vx = 0;
-                    for (int cx = 0; cx < 4; cx++)
-                        vx += w[0][cx] * (double)mag_at(mg, M, wrap_idx(idx[0] - 1 + cx, M), jy, kz, padc);
-                    vy += w[1][cy] * vx;
-                }
-                v += w[2][cz] * vy;
-            }
-        }
-        sum += v;
     }
-    for (int o = kLanes / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kLanes);
-    if (live && lane == 0) Pp[(size_t)b * n * n + t] = (float)sum;
+    // every tap and its mirror image lies away from the i = 0 plane, the j = 0 column and the wrap
+    __device__ __forceinline__ bool interior(int M) const {
+        return lo[0] >= 1 && lo[0] + 3 <= M - 1 && lo[1] >= 1 && lo[1] + 3 <= M - 1 && lo[2] >= 0 && lo[2] + 3 <= M - 1;
+    }
+    // row (cy, cx) of taps tap(cy, cx, cz); REV: the taps run backwards along every axis
+    template <bool REV> __device__ __forceinline__ double row(const float* r) const {
+        double v = 0;
+#pragma unroll
+        for (int cz = 0; cz < 4; cz++) v += w[2][REV ? 3 - cz : cz] * (double)r[cz];
+        return v;
+    }
+    template <bool REV> __device__ __forceinline__ double wx(int c) const { return w[0][REV ? 3 - c : c]; }
+    template <bool REV> __device__ __forceinline__ double wy(int c) const { return w[1][REV ? 3 - c : c]; }
+};
+// one sample: from the stored rows (k <= M/2 + 1) or their mirror image where the stencil allows it (the values mag_at
+// would return), else tap by tap
+__device__ __forceinline__ double sph_value(const float* __restrict__ mg, int M, float padc, SphStencil& s) {
+    const int Hm = M / 2 + 2;
+    const bool in = s.interior(M), direct = in && s.lo[2] + 3 <= M / 2 + 1, mirror = in && !direct && s.lo[2] >= M / 2 - 1;
+    double v = 0;
+    if (direct || mirror) {
+        if (mirror)
+            for (int a = 0; a < 3; a++) {
+                s.lo[a] = M - 3 - s.lo[a];
+                double w0 = s.w[a][0], w1 = s.w[a][1];
+                s.w[a][0] = s.w[a][3];
+                s.w[a][1] = s.w[a][2];
+                s.w[a][2] = w1;
+                s.w[a][3] = w0;
+            }
+        const unsigned o = (((unsigned)s.lo[0] * M + s.lo[1]) * Hm + s.lo[2]) * 4;
+#pragma unroll
+        for (int cx = 0; cx < 4; cx++) {
+            double vy = 0;
+#pragma unroll
+            for (int cy = 0; cy < 4; cy++) {
+                float r[4];
+                __builtin_memcpy(r, &at_byte(mg + (size_t)(cx * M + cy) * Hm, o), sizeof(r));
+                vy += s.wy<false>(cy) * s.row<false>(r);
+            }
+            v += s.wx<false>(cx) * vy;
+        }
+    } else {
+#pragma unroll 1
+        for (int cx = 0; cx < 4; cx++) {
+            const int kx = wrap_idx(s.lo[0] + cx, M);
+            double vy = 0;
+#pragma unroll
+            for (int cy = 0; cy < 4; cy++) {
+                float r[4];
+#pragma unroll
+                for (int cz = 0; cz < 4; cz++)
+                    r[cz] = mag_at(mg, M, kx, wrap_idx(s.lo[1] + cy, M), wrap_idx(s.lo[2] + cz, M), padc);
+                vy += s.wy<false>(cy) * s.row<false>(r);
+            }
+            v += (cx == 0 ? s.w[0][0] : cx == 1 ? s.w[0][1] : cx == 2 ? s.w[0][2] : s.w[0][3]) * vy;
+        }
+    }
+    return v;
+}
+
+// One ray and its opposite per group of kLanes consecutive threads; the radial shells r = bandL..bandU are split over the
+// lanes and summed with wavefront shuffles.  The opposite sample lies at the mirror image of the position up to the floor
+// tolerance and reads the mirror images of the same taps: they are loaded once and weighted twice.  (Where a coordinate
+// lies within the tolerance of a voxel, its floor would start a tap later; the kernel has a continuous derivative, so
+// the four taps taken at f <= 1 + 2^-16 give its value to 2^-32 of the curvature.)  A wavefront holds 8 rays that differ in
+// phi by 8 shells: one plane through the z axis, where a 128-byte line along k serves many samples (neighbours in theta
+// share none).  Its consecutive lanes are the shells of a ray near the axis and the rays of a shell near the equator,
+// whichever runs along k, so that neighbouring lanes' loads fall into one line.
+// Bound by the rate of L1 accesses (53 per load with shells in consecutive lanes everywhere) and by the FP64 sums.  32
+// images of 64^3, 4096 rays of 61 shells: 103 us; 280 with every ray on its own and neighbours in theta side by side.
+static constexpr int kRays = kT / kLanes;
+__global__ void __launch_bounds__(kT) k_sph_sample(const float* __restrict__ mag, const float* __restrict__ st, int M,
+                                                    int B, int bandL, int bandU, float* __restrict__ Pp) {
+    __shared__ double dir[kRays][3];
+    // one particle per XCD at a time: its magnitude volume is gathered through that XCD's L2 only
+    int b, tile;
+    xcd_eval_tile(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, b, tile);
+    const int n = 2 * B;
+    if (threadIdx.x < kRays) {
+        const int t = tile * kRays + threadIdx.x;
+        const double phi = M_PI / 4.0 / (float)B + (B + t % B) * (2.0 * M_PI / 4.0 / (float)B);
+        const double th = t / B * (M_PI / (float)B);
+        dir[threadIdx.x][0] = sin(phi) * cos(th);
+        dir[threadIdx.x][1] = sin(phi) * sin(th);
+        dir[threadIdx.x][2] = cos(phi);
+    }
+    __syncthreads();
+    const int wl = threadIdx.x % 64, w0 = tile * kRays + threadIdx.x / 64 * (64 / kLanes);  // lane, first ray of the wave
+    const bool equator = 2 * (w0 % B) < B;
+    const int ray = threadIdx.x / 64 * (64 / kLanes) + (equator ? wl % kLanes : wl / kLanes);
+    const int lane = equator ? wl / kLanes : wl % kLanes;
+    const int t = tile * kRays + ray;
+    const bool live = t < B * n;
+    const int jp = B + t % B, kt = t / B;  // phi > pi / 2: the ray runs through the stored half
+    const float* mg = mag + (size_t)b * M * M * (M / 2 + 2);
+    const float padc = st[b * 4 + 2];
+    const double dx = dir[ray][0], dy = dir[ray][1], dz = dir[ray][2];
+    const double origin = -(M - 1) / 2.0 - 0.5;
+    double sum = 0, opp = 0;
+    unsigned left = 0;  // shells of this lane whose stencils reach the wrap (at most M / 2 / kLanes = 16 shells in all)
+    for (int m = 0, r = bandL + lane; live && r <= bandU; m++, r += kLanes) {
+        const double pa[3] = {r * dx - origin, r * dy - origin, r * dz - origin};
+        const double pb[3] = {-r * dx - origin, -r * dy - origin, -r * dz - origin};
+        SphStencil sa, sb;
+        sa.set(pa);
+        if (sa.interior(M) && sa.lo[2] + 3 <= M / 2 + 1) {
+            for (int a = 0; a < 3; a++) sb.lo[a] = M - 3 - sa.lo[a];
+            sb.weigh(pb);
+            const int Hm = M / 2 + 2;
+            const unsigned o = (((unsigned)sa.lo[0] * M + sa.lo[1]) * Hm + sa.lo[2]) * 4;
+            double va = 0, vb = 0;
+#pragma unroll
+            for (int cx = 0; cx < 4; cx++) {
+                double ya = 0, yb = 0;
+#pragma unroll
+                for (int cy = 0; cy < 4; cy++) {
+                    float q[4];
+                    // 4 consecutive floats at a 4-byte-aligned start: one load (global loads of four dwords need
+                    // only dword alignment on this architecture)
+                    __builtin_memcpy(q, &at_byte(mg + (size_t)(cx * M + cy) * Hm, o), sizeof(q));
+                    ya += sa.wy<false>(cy) * sa.row<false>(q);
+                    yb += sb.wy<true>(cy) * sb.row<true>(q);
+                }
+                va += sa.wx<false>(cx) * ya;
+                vb += sb.wx<true>(cx) * yb;
+            }
+            sum += va;
+            opp += vb;
+        } else left |= 1u << m;
+    }
+    // the rest one by one (in their own loop: its registers would halve the waves in flight of the loop above)
+#pragma unroll 1
+    for (; left; left &= left - 1) {
+        const int r = bandL + lane + (__ffs(left) - 1) * kLanes;
+#pragma unroll 1
+        for (int h = 0; h < 2; h++) {
+            const double sg = h ? -r : r;
+            const double p[3] = {sg * dx - origin, sg * dy - origin, sg * dz - origin};
+            SphStencil s1;
+            s1.set(p);
+            const double v = sph_value(mg, M, padc, s1);
+            if (h == 0) sum += v;
+            else opp += v;
+        }
+    }
+    static_assert(kLanes * kLanes == 64, "rays by shells of a wavefront");
+    for (int o = kLanes / 2; o > 0; o >>= 1) {
+        sum += __shfl_xor(sum, equator ? o * kLanes : o, 64);
+        opp += __shfl_xor(opp, equator ? o * kLanes : o, 64);
+    }
+    if (live && lane == 0) {
+        float* out = Pp + (size_t)b * n * n;
+        out[jp * n + kt] = (float)sum;
+        out[(n - 1 - jp) * n + (kt + B) % n] = (float)opp;
+    }
 }
 
 // ============================================================== soft instances: assemble S^2 samples
@@ -1243,7 +1327,7 @@ void project_images(ettk_plan* P, const float* d_parts, const ettk_particle* des
         // the stencils of the outermost shell reach 3.5 voxels past it; a wrapped tap lies nearer the centre
         PadMagArgs a{S.projR.p, P->m1.p, S.projStats.p, S.projF.p, S.projMag.p, cn, band_hi(P) + 4, P->p.mcf};
         fft3_pad_magnitude(P->ctx->fft, a, N, s);
-        dim3 grid((4 * B * B + kT / kLanes - 1) / (kT / kLanes), cn);
+        dim3 grid((2 * B * B + kRays - 1) / kRays, cn);
         ProfScope ps(P->ctx->fft.prof, "k_sph_sample", (double)cn * ((double)nbig * 4 + 16.0 * B * B), s);
         k_sph_sample<<<grid, kT, 0, s>>>(S.projMag.p, S.projStats.p, M, B, band_lo(P), band_hi(P),
                                          d_Pp + (size_t)c0 * 4 * B * B);
