@@ -1533,8 +1533,7 @@ static int so3_correlate_entry(ettk_plan* P, int n, const double* sig, const dou
         const size_t n3 = (size_t)8 * B * B * B;
         S.C.ensure(n3 * n);
         soft_given(P, n, sig, pat, S.C.p, scaled);
-        ETTK_HIP(hipMemcpyAsync(out_c, S.C.p, n3 * n * sizeof(double), hipMemcpyDeviceToHost, P->stream));
-        ETTK_HIP(hipStreamSynchronize(P->stream));
+        download_staged(S.down, out_c, S.C.p, n3 * n * sizeof(double), P->stream);
     } catch (const Error& e) {
         set_error(e.msg);
         return e.code;

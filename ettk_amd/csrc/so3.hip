@@ -12,6 +12,9 @@
 // Rockmore 2008): direct quadrature with FP64 Legendre tables and FP64 Wigner-d three-term recurrences.
 #include <cfloat>
 #include <cmath>
+#include <cstring>
+#include <system_error>
+#include <thread>
 
 #include "so3.hpp"
 
@@ -1562,6 +1565,68 @@ void sph_rotate(ettk_plan* P, int n, const float* h_img, const double* h_t, floa
     ETTK_HIP(hipMemcpyAsync(h.data(), out.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, s));
     ETTK_HIP(hipStreamSynchronize(s));
     for (size_t q = 0; q < h.size(); q++) h_out[q] = (float)h[q];
+}
+
+bool DownloadRing::ready() {
+    if (buf.n == 0) {
+        try {
+            buf.ensure(kSlots * kSlotBytes);
+        } catch (const Error&) {
+            (void)hipGetLastError();
+            return false;
+        }
+    }
+    for (hipEvent_t& e : ev)
+        if (!e) ETTK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return true;
+}
+
+// The runtime's copy into pageable memory moves 12.6 MB (six correlations at B = 32) in 694 us, 860 where the pages of
+// the result are touched for the first time.  The card writes pinned memory in 229 us; one host thread that copies it on
+// needs 161 us, or 430 with those page faults, so every slot has its own thread, which waits for the slot's transfer, copies
+// it and starts the next one.  The threads start while the kernels run: 550 us from the launches to the last byte, with one
+// thread 650.  Slots of 1, 2 and 4 MB: 762, 710, 780 us for the call.
+void download_staged(DownloadRing& ring, void* dst, const void* src, size_t bytes, hipStream_t s) {
+    constexpr size_t kPiece = DownloadRing::kSlotBytes;
+    constexpr int K = DownloadRing::kSlots;
+    if (bytes <= kPiece || !ring.ready()) {  // one piece has nothing to hide behind
+        ETTK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+        ETTK_HIP(hipStreamSynchronize(s));
+        return;
+    }
+    const int np = (int)((bytes + kPiece - 1) / kPiece), nw = std::min(np, K);
+    auto size = [&](int c) { return std::min(kPiece, bytes - c * kPiece); };
+    auto issue = [&](int c) {
+        const hipError_t e = hipMemcpyAsync(ring.buf.p + (c % K) * kPiece, (const char*)src + c * kPiece, size(c),
+                                            hipMemcpyDeviceToHost, s);
+        return e == hipSuccess ? hipEventRecord(ring.ev[c % K], s) : e;
+    };
+    int device = 0;
+    ETTK_HIP(hipGetDevice(&device));
+    for (int c = 0; c < nw; c++) ETTK_HIP(issue(c));
+    hipError_t err[K] = {};
+    auto slot = [&](int w) {
+        err[w] = hipSetDevice(device);
+        for (int c = w; c < np && err[w] == hipSuccess; c += K) {
+            err[w] = hipEventSynchronize(ring.ev[w]);
+            if (err[w] != hipSuccess) break;
+            std::memcpy((char*)dst + c * kPiece, ring.buf.p + w * kPiece, size(c));
+            if (c + K < np) err[w] = issue(c + K);
+        }
+    };
+    std::thread th[K];
+    for (int w = 1; w < nw; w++) {
+        try {
+            th[w] = std::thread(slot, w);
+        } catch (const std::system_error&) {  // no thread to be had: this one takes the slot below
+        }
+    }
+    slot(0);
+    for (int w = 1; w < nw; w++) {
+        if (th[w].joinable()) th[w].join();
+        else slot(w);
+    }
+    for (hipError_t e : err) ETTK_HIP(e);
 }
 
 void soft_given(ettk_plan* P, int nq, const double* h_sig, const double* h_pat, double* d_C, int scaled) {

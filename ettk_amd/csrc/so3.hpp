@@ -48,6 +48,24 @@ struct LmBuffers {
     PinnedBuf<double> hpval;
 };
 
+// Pinned slots through which a large result reaches pageable memory in pieces
+struct DownloadRing {
+    static constexpr int kSlots = 4;
+    static constexpr size_t kSlotBytes = size_t(1) << 21;
+    PinnedBuf<char> buf;
+    hipEvent_t ev[kSlots] = {};
+    DownloadRing() = default;
+    DownloadRing(const DownloadRing&) = delete;
+    DownloadRing& operator=(const DownloadRing&) = delete;
+    ~DownloadRing() {
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
+    }
+    bool ready();  // allocates on first use; false where pinned memory cannot be had
+};
+// src (device) to dst (host) behind the work on `s`; returns when dst is written
+void download_staged(DownloadRing& ring, void* dst, const void* src, size_t bytes, hipStream_t s);
+
 struct So3State {
     int B = 0;
     int d_slice = 0;
@@ -77,6 +95,7 @@ struct So3State {
     DevBuf<float> Pp2, W2, Mx;
     DevBuf<double> C, Cc;
     DevBuf<ComboOp> ops;
+    DownloadRing down;  // results of ettk_so3_correlate_batch
     std::vector<std::unique_ptr<LmBuffers>> lm_pool;  // one slot per chunk in flight
     // host inputs of a search call (spherical wedges, reslice geometry), pinned for asynchronous uploads
     PinnedBuf<float> hW2;

@@ -172,3 +172,24 @@ def test_projection_box_sizes(torch_gpu, ctx, N, band, mask):
         assert err < 1e-5
     finally:
         plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,pairs", [(16, 8), (16, 11), (32, 5)])
+def test_correlations_in_pieces(torch_gpu, ctx, B, pairs):
+    """Results that fill one piece of the download exactly, leave a remainder in the second, and use the first slot
+    again, against the same pairs one call each.  FP64 sums whose order may depend on the batch: 2B x 2B x B terms,
+    1e-12 of the largest value."""
+    from ettk_amd.lib import Plan
+
+    g = np.random.default_rng(B + pairs)
+    sig, pat = g.standard_normal((2, pairs, 2 * B, 2 * B))
+    plan = Plan(ctx, default_params(32, B))
+    try:
+        got = plan.so3_correlate(sig, pat)
+        for i in range(pairs):
+            one = plan.so3_correlate(sig[i], pat[i])[0]
+            err = np.abs(got[i] - one).max() / np.abs(one).max()
+            assert err < 1e-12, (i, err)
+    finally:
+        plan.close()
