@@ -467,15 +467,19 @@ __global__ void k_ppmax(const float* __restrict__ Pp1, const float* __restrict__
 }
 
 // ============================================================== S^2 transforms (FP64)
+// The S^2 samples of nq signals and, in the same launch, nq patterns (q >= nq; null: signals only): with one side per
+// launch a batch of six pairs fills a fifth of the chip.
 // ring DFT: fm[q][j][m] = sum_k f[q][j][k] e^{-i m phi_k}, m = 0..2B-1 (negative orders at 2B+m)
-__global__ void k_ring_dft(const double* __restrict__ f, const double2* __restrict__ tw, int B, double2* __restrict__ fm) {
+__global__ void k_ring_dft(const double* __restrict__ f, const double* __restrict__ f2, int nq,
+                           const double2* __restrict__ tw, int B, double2* __restrict__ fm) {
     const int n = 2 * B, q = blockIdx.y;
+    const double* src = q < nq ? f + (size_t)q * n * n : f2 + (size_t)(q - nq) * n * n;
     __shared__ double2 stw[256];
     for (int t = threadIdx.x; t < n; t += blockDim.x) stw[t] = tw[t];
     __syncthreads();
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n * n; t += gridDim.x * blockDim.x) {
         int j = t / n, m = t % n;
-        const double* row = f + ((size_t)q * n + j) * n;
+        const double* row = src + (size_t)j * n;
         double re = 0, im = 0;
         for (int k = 0; k < n; k++) {
             double2 w = stw[(m * k) % n];
@@ -485,10 +489,14 @@ __global__ void k_ring_dft(const double* __restrict__ f, const double2* __restri
         fm[((size_t)q * n + j) * n + m] = make_double2(re, im);
     }
 }
-// Legendre quadrature: c[q][l^2+l+m] = sum_j LF[|m|][l][j] fm[q][j][m] ((-1)^m for m < 0)
-__global__ void k_legendre_fwd(const double2* __restrict__ fm, const double* __restrict__ LF, int B, double2* __restrict__ c) {
-    const int n = 2 * B, q = blockIdx.y;
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < B * B; t += gridDim.x * blockDim.x) {
+// Legendre quadrature: c[q][l^2+l+m] = sum_j LF[|m|][l][j] fm[q][j][m] ((-1)^m for m < 0).  Eight lanes share a
+// coefficient: the table is read in whole 64-byte lines and the chain of dependent sums is an eighth as long.
+// Six pairs at B = 32 (12 of them here): 4.9 us; two launches of a thread per coefficient took 38.
+constexpr int kLegLanes = 8;
+__global__ void k_legendre_fwd(const double2* __restrict__ fm, const double* __restrict__ LF, int B, int nq,
+                               double2* __restrict__ c, double2* __restrict__ c2) {
+    const int n = 2 * B, q = blockIdx.y, lane = threadIdx.x % kLegLanes;
+    for (int t = (blockIdx.x * blockDim.x + threadIdx.x) / kLegLanes; t < B * B; t += gridDim.x * blockDim.x / kLegLanes) {
         int l = (int)sqrt((double)t);
         while (l * l > t) l--;
         while ((l + 1) * (l + 1) <= t) l++;
@@ -498,13 +506,17 @@ __global__ void k_legendre_fwd(const double2* __restrict__ fm, const double* __r
         const double2* src = fm + (size_t)q * n * n;
         int col = m < 0 ? n + m : m;
         double re = 0, im = 0;
-        for (int j = 0; j < n; j++) {
+        for (int j = lane; j < n; j += kLegLanes) {
             double2 z = src[(size_t)j * n + col];
             re += tab[j] * z.x;
             im += tab[j] * z.y;
         }
+        for (int o = kLegLanes / 2; o > 0; o >>= 1) {
+            re += __shfl_xor(re, o, kLegLanes);
+            im += __shfl_xor(im, o, kLegLanes);
+        }
         double sg = (m < 0 && (am & 1)) ? -1.0 : 1.0;
-        c[(size_t)q * B * B + t] = make_double2(sg * re, sg * im);
+        if (lane == 0) (q < nq ? c + (size_t)q * B * B : c2 + (size_t)(q - nq) * B * B)[t] = make_double2(sg * re, sg * im);
     }
 }
 // inverse: g[q][j][m] = sum_l c(l,m) Pbar_l^|m|(theta_j) ((-1)^m for m < 0)
@@ -1365,7 +1377,7 @@ void soft_core(ettk_plan* P, const std::vector<SoftInst>& inst, double* d_C) {
     const int B = S.B, n = 2 * B, nq = (int)inst.size();
     const long n3 = (long)n * n * n;
     hipStream_t s = P->stream;
-    S.fm.ensure((size_t)nq * n * n);
+    S.fm.ensure((size_t)2 * nq * n * n);
     S.cs.ensure((size_t)nq * B * B);
     S.cp.ensure((size_t)nq * B * B);
     S.vals.ensure((size_t)2 * nq);
@@ -1374,10 +1386,9 @@ void soft_core(ettk_plan* P, const std::vector<SoftInst>& inst, double* d_C) {
     S.g.ensure((size_t)2 * nq * n * n);
     S.Rr.ensure((size_t)2 * nq * n * n);
     S.wv.ensure((size_t)2 * nq);
-    k_ring_dft<<<dim3(16, nq), kT, 0, s>>>(S.sig.p, S.tw.p, B, S.fm.p);
-    k_legendre_fwd<<<dim3(8, nq), kT, 0, s>>>(S.fm.p, S.legF.p, B, S.cs.p);
-    k_ring_dft<<<dim3(16, nq), kT, 0, s>>>(S.pat.p, S.tw.p, B, S.fm.p);
-    k_legendre_fwd<<<dim3(8, nq), kT, 0, s>>>(S.fm.p, S.legF.p, B, S.cp.p);
+    const unsigned leg_blocks = (B * B * kLegLanes + kT - 1) / kT;
+    k_ring_dft<<<dim3(16, 2 * nq), kT, 0, s>>>(S.sig.p, S.pat.p, nq, S.tw.p, B, S.fm.p);
+    k_legendre_fwd<<<dim3(leg_blocks, 2 * nq), kT, 0, s>>>(S.fm.p, S.legF.p, B, nq, S.cs.p, S.cp.p);
     if (mfma_synthesis(B)) {
         const int nqp = (nq + 15) & ~15, Q8 = (nq + 7) / 8, BB = B * B;
         S.csT.ensure((size_t)BB * nqp);
@@ -1462,7 +1473,7 @@ void so3_search_reserve(ettk_plan* P, int cn) {
     S.inst.ensure(nq);
     S.sig.ensure(nq * nn);
     S.pat.ensure(nq * nn);
-    S.fm.ensure(nq * nn);
+    S.fm.ensure(2 * nq * nn);
     S.cs.ensure(nq * B * B);
     S.cp.ensure(nq * B * B);
     S.vals.ensure(2 * nq);
@@ -1555,8 +1566,8 @@ void sph_rotate(ettk_plan* P, int n, const float* h_img, const double* h_t, floa
     r.ensure((size_t)n * B * B);
     g.ensure((size_t)n * nn);
     out.ensure((size_t)n * nn);
-    k_ring_dft<<<dim3(16, n), kT, 0, s>>>(f.p, S.tw.p, B, fm.p);
-    k_legendre_fwd<<<dim3(8, n), kT, 0, s>>>(fm.p, S.legF.p, B, c.p);
+    k_ring_dft<<<dim3(16, n), kT, 0, s>>>(f.p, nullptr, n, S.tw.p, B, fm.p);
+    k_legendre_fwd<<<dim3((B * B * kLegLanes + kT - 1) / kT, n), kT, 0, s>>>(fm.p, S.legF.p, B, n, c.p, nullptr);
     k_rotate_coef_angles<<<n, kT, (size_t)B * (2 * B - 1) * sizeof(double2), s>>>(c.p, a.p, B, r.p);
     k_legendre_inv<<<dim3(16, n), kT, 0, s>>>(r.p, S.legI.p, B, g.p);
     k_ring_idft<<<dim3(16, n), kT, 0, s>>>(g.p, S.tw.p, B, out.p);
