@@ -193,3 +193,38 @@ def test_correlations_in_pieces(torch_gpu, ctx, B, pairs):
             assert err < 1e-12, (i, err)
     finally:
         plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [32, 96])
+def test_wedge_at_lattice_rotations(torch_gpu, ctx, N):
+    """Rotations by multiples of 45 degrees put the tilt axis along lattice directions, where a line of samples lies on
+    both wedge planes and the last bit of the plane values decides: the distances are pinned to those the 27-sample
+    stencil gave when every element evaluated its own.  FP32 transforms, 2^-24 per level of at most 24: 1.4e-6 of a
+    score of at most 1; samples on the other side move these distances by 1e-5 and more."""
+    import json
+    import math
+    from pathlib import Path
+
+    from ettk_amd.lib import Plan
+
+    def turn(axis, deg):
+        a, r, (i, j) = math.radians(deg), np.eye(3), [(1, 2), (2, 0), (0, 1)][axis]
+        r[i, i] = r[j, j] = math.cos(a)
+        r[i, j], r[j, i] = -math.sin(a), math.sin(a)
+        return r
+
+    want = np.array(json.loads((Path(__file__).parent / "golden" / "wedge_lattice.json").read_text())[str(N)])
+    rots = [turn(2, a) @ turn(0, b) @ turn(2, g) for a in (0, 45, 90, 135) for b in (0, 45, 90) for g in (0, 45, 270)]
+    ref = blob_reference(N, seed=3)
+    ps = make_particles(ref, 2, seed=4, half_wedge=(50, 60), snr=(0.5, 0.5), max_shift=1.0)
+    t = np.tile(np.eye(4), (len(rots), 1, 1))
+    t[:, :3, :3] = rots
+    plan = Plan(ctx, default_params(N, 8, mask_radius=N / 2 - 3, square_mask=2))
+    try:
+        plan.set_reference(to_dev(torch_gpu, ref))
+        d, _ = plan.ccc(to_dev(torch_gpu, ps.vols), ps.descs, np.arange(len(rots), dtype=np.int32) % 2, t)
+        print(f"[edges] wedge N={N} err {np.abs(d - want).max():.2e}", flush=True)
+        assert np.abs(d - want).max() < 2e-6
+    finally:
+        plan.close()
