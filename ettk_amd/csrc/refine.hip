@@ -78,9 +78,9 @@ __device__ __forceinline__ void ref_pos(const RefineGeom& g, int N, int x, int y
 // border), is staged in LDS at fixed strides, so the divergent gathers become LDS reads and every sample equals
 // the clamped-tap global one; a sample that rounds one voxel past the box keeps the box's edge cell with its
 // fraction just outside [0, 1) (the same value to a few ulps).  A 15^3 box (13.5 KB) lets 10 workgroups share a
-// CU, which hides the staging loads' latency: on 128 evaluations at 64^3 the reference reslice takes 155 us per
-// launch and the adjoint moments 180 us, against 185 and 221 us with an 18^3 box staged whole.  A map whose box
-// does not fit samples from global memory instead.
+// CU, which hides the staging loads' latency (an 18^3 box staged whole took 1.2 times as long); the box's bounds and
+// the staging's plane addresses are scalar.  40 evaluations at 64^3: reference reslice 48 us, adjoint moments 60, where
+// addresses per lane took 51 and 65.  A map whose box does not fit samples from global memory instead.
 static constexpr int kRT = 8, kRB = 15;
 
 __device__ __forceinline__ bool stage_ref_box(const float* __restrict__ vol, int N, const RefineGeom& g, int x0,
@@ -93,26 +93,33 @@ __device__ __forceinline__ bool stage_ref_box(const float* __restrict__ vol, int
         const float c0 = r[0] * ((float)x0 - h) + r[1] * ((float)y0 - h) + r[2] * ((float)z0 - h) + r[3];
         const float mn = c0 + (kRT - 1) * (fminf(r[0], 0.f) + fminf(r[1], 0.f) + fminf(r[2], 0.f));
         const float ext = (kRT - 1) * (fabsf(r[0]) + fabsf(r[1]) + fabsf(r[2]));
-        lo[a] = (int)floorf(mn);
-        hi[a] = (int)floorf(mn + ext) + 1;
+        // the same for every thread: in scalar registers, with the plane addresses of the staging below
+        lo[a] = __builtin_amdgcn_readfirstlane((int)floorf(mn));
+        hi[a] = __builtin_amdgcn_readfirstlane((int)floorf(mn + ext) + 1);
         if (!(hi[a] - lo[a] + 1 <= kRB) || !(fabsf(mn) < 1e6f)) fits = false;
     }
     if (fits) {
         // 2-D thread map over (y, x) of the box, loop over z; coordinates clamped to the volume
-        constexpr int kRows = kT / kRB;
-        const int t = threadIdx.x;
+        static_assert(kT / kRB >= kRB && kRB % 5 == 0, "one pass over a plane, whole steps of z");
+        const int x = threadIdx.x % kRB, y = threadIdx.x / kRB;
         const int wx = hi[0] - lo[0] + 1, wy = hi[1] - lo[1] + 1, wz = hi[2] - lo[2] + 1;
-        const int x = t % kRB, yb = t / kRB;
-        if (t < kRB * kRows && x < wx) {
-            const int gx = min(max(lo[0] + x, 0), N - 1);
-            for (int y = yb; y < wy; y += kRows) {
-                const int gy = min(max(lo[1] + y, 0), N - 1);
-                const float* src = vol + (size_t)gy * N + gx;
-#pragma unroll 5
-                for (int z = 0; z < wz; z++) {
-                    const int gz = min(max(lo[2] + z, 0), N - 1);
-                    box[(z * kRB + y) * kRB + x] = src[(size_t)gz * N * N];
+        if (x < wx && y < wy) {
+            const int gx = min(max(lo[0] + x, 0), N - 1), gy = min(max(lo[1] + y, 0), N - 1);
+            const unsigned off = ((unsigned)gy * N + gx) * 4u;
+            float* dst = box + y * kRB + x;
+            const size_t plane = (size_t)N * N;
+            // the plane's address advances in scalar registers; it stays where the clamped coordinate does
+            const float* src = vol + (size_t)min(max(lo[2], 0), N - 1) * plane;
+            for (int z = 0; z < wz; z += 5, dst += 5 * kRB * kRB) {  // five loads in flight; planes past the box unused
+                float r[5];
+#pragma unroll
+                for (int u = 0; u < 5; u++) {
+                    r[u] = at_byte(src, off);
+                    const unsigned g = (unsigned)(lo[2] + z + u);  // step from this plane to the next one inside the volume
+                    src += g < (unsigned)(N - 1) ? plane : 0;
                 }
+#pragma unroll
+                for (int u = 0; u < 5; u++) dst[u * kRB * kRB] = r[u];
             }
         }
     }
