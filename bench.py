@@ -148,7 +148,7 @@ def main() -> int:
     kernels = {}
     for name in ("k_fft_strided<64>", "k_r2c_plane<64>", "k_c2r_plane<64>", "k_c2r_r2c_plane<64>", "k_ccc_ipass<64>",
                  "k_reslice",
-                 "k_ccc_combine", "k_ccc_dftBC", "k_fft_strided<128>", "k_r2c_rows<128>",
+                 "k_ccc_combine", "k_ccc_dftBC", "k_pad_planes", "k_pad_mag",
                  "k_reslice_ref", "k_refine_ipass_dot", "k_refine_ipass_adj", "k_refine_moments", "k_sph_sample",
                  "k_so3_synth_fft", "k_so3_synth_mfma", "k_so3_fft2", "k_rotate_coef", "k_extrema", "k_combine",
                  "k_localmax"):
