@@ -71,7 +71,7 @@ __global__ void __launch_bounds__(kThreads, 7) k_reslice(const float* __restrict
     const int i0 = tb / (nt * nt) * kTile, j0 = (tb / nt) % nt * kTile, k0 = tb % nt * kTile;
     int lo[3], hi[3];
     bool inside;
-    const bool fits = tile_box(g.m, i0, j0, k0, N, N, N, lo, hi, inside);
+    const bool fits = tile_box(g.m, i0, j0, k0, N, N, N, kMarginMin, lo, hi, inside);  // N <= 128
     if (fits) stage_tile_box(vol, N, N, N, lo, hi, box);
     const int lo1[3] = {lo[0] + 1, lo[1] + 1, lo[2] + 1};
     int i, j, k;
@@ -96,7 +96,7 @@ __global__ void __launch_bounds__(kThreads, 7) k_reslice(const float* __restrict
         const float py = g.m[1] * fi + pjk[1] + g.m[10];
         const float pz = g.m[2] * fi + pjk[2] + g.m[11];
         float v;
-        if (inside && fits) {
+        if (inside) {
             v = sample_box(box, lo1, px, py, pz);
             s += v;
             c += 64;

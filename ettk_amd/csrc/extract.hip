@@ -35,7 +35,7 @@ __global__ void __launch_bounds__(kExT, 7) k_extract(const float* __restrict__ t
     const int z0 = (tb / (nt * nt)) * kTile, y0 = ((tb / nt) % nt) * kTile, x0 = (tb % nt) * kTile;
     int lo[3], hi[3];
     bool inside;
-    const bool fits = tile_box(g.m, x0, y0, z0, nx, ny, nz, lo, hi, inside);
+    const bool fits = tile_box(g.m, x0, y0, z0, nx, ny, nz, tile_margin(max(nx, max(ny, nz)), N), lo, hi, inside);
     if (fits) stage_tile_box(tomo, nx, ny, nz, lo, hi, box);
     const int lo1[3] = {lo[0] + 1, lo[1] + 1, lo[2] + 1};
     int x, y, z;

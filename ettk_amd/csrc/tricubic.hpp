@@ -36,12 +36,24 @@ __device__ __forceinline__ void keys_w(float f, float* w) {  // vtkTricubicInter
     w[3] = f * fd2 * fm1;
 }
 
+// What the staged box reaches beyond the tile's transformed corners, so that every sample's stencil lies in it whatever
+// FP32 rounding does to the positions.  A sample inside the volume has terms of m[0..2] x + ... + m[9..11] whose magnitudes
+// add up to A <= n + 4 N for a volume of n and an output box of N voxels per axis (a map that fits has rows of absolute sum
+// below 2).  In any order, fused or not, a position with its floor tolerance takes 7 roundings of at most 2^-24 A, a bound
+// of the box 9: 2^-20 A together, and the small terms of 7 voxels below 1e-5, kTriTol below 1e-5.  Up to N = 128 the floor
+// of 1e-3 covers it; with the floor alone a box of 1024^3 cut beyond coordinate 8192 read taps that were not staged.
+// A rigid map (corners 12.13 voxels apart at most) fits kBox with margins up to 0.43, coordinates of 4e5.
+static constexpr float kMarginMin = 1e-3f, kMarginUlp = 9.5367431640625e-07f, kMarginSmall = 2e-5f;
+__device__ __forceinline__ float tile_margin(int n, int N) {
+    return fmaxf(kMarginMin, kMarginUlp * ((float)n + 4.f * (float)N) + kMarginSmall);
+}
+
 // staged box [lo, hi] per input axis (x, y, z) of the tile at (i0, j0, k0) under the map m (columns of the output axes,
-// then the offset); it may reach outside the volume.  A margin of 1e-3 voxels keeps every sample's stencil in the box
-// whatever FP32 rounding does to its position.  False when the map's box does not fit.  `inside`: every sample of the
-// tile lies in an nx x ny x nz volume, away from its border, so that no sample's validity needs a test.
-__device__ __forceinline__ bool tile_box(const float* m, int i0, int j0, int k0, int nx, int ny, int nz, int lo[3],
-                                         int hi[3], bool& inside) {
+// then the offset); it may reach outside the volume.  False when the map's box does not fit.  `inside`: the box fits and
+// every sample of the tile lies in an nx x ny x nz volume, more than 1e-3 away from its border, so that no sample's
+// validity needs a test.
+__device__ __forceinline__ bool tile_box(const float* m, int i0, int j0, int k0, int nx, int ny, int nz, float margin,
+                                         int lo[3], int hi[3], bool& inside) {
     bool fits = true;
     inside = true;
     const int n[3] = {nx, ny, nz};
@@ -51,13 +63,14 @@ __device__ __forceinline__ bool tile_box(const float* m, int i0, int j0, int k0,
         float ext = (kTile - 1) * (fabsf(m[a]) + fabsf(m[3 + a]) + fabsf(m[6 + a]));
         float mn = c0 + (kTile - 1) * (fminf(m[a], 0.f) + fminf(m[3 + a], 0.f) + fminf(m[6 + a], 0.f));
         // the same for every thread: kept in scalar registers, and with them the staging's row and plane arithmetic
-        lo[a] = __builtin_amdgcn_readfirstlane((int)floorf(mn - 1e-3f) - 1);
-        hi[a] = __builtin_amdgcn_readfirstlane((int)floorf(mn + ext + 1e-3f) + 2);
-        if (!(hi[a] - lo[a] + 1 <= kBox) || !(fabsf(mn) < 1e6f)) fits = false;
-        if (!(mn > -0.49f && mn + ext < (float)n[a] - 0.51f)) inside = false;
+        lo[a] = __builtin_amdgcn_readfirstlane((int)floorf(mn - margin) - 1);
+        hi[a] = __builtin_amdgcn_readfirstlane((int)floorf(mn + ext + margin) + 2);
+        // a map too steep, or a tile too far away, for these whole numbers does not fit either
+        if (!(ext < (float)kBox) || !(fabsf(mn) < 1e6f) || hi[a] - lo[a] + 1 > kBox) fits = false;
+        if (!(mn > -0.499f + margin && mn + ext < (float)n[a] - 0.501f - margin)) inside = false;
     }
-    // the staging's offsets within a plane are 32-bit bytes; positions beyond 1e4 voxels round by more than the margin
-    if ((unsigned long long)nx * ny >= (1ull << 30) || !(fmaxf((float)nx, fmaxf((float)ny, (float)nz)) < 1e4f)) fits = false;
+    if ((unsigned long long)nx * ny >= (1ull << 30)) fits = false;  // the staging's offsets within a plane are 32-bit bytes
+    inside = inside && fits;
     return fits;
 }
 
