@@ -1260,6 +1260,28 @@ static void launch_c2r_op_r2c(const FftTables& T, const float2* in, float2* io, 
 }
 
 template <int L>
+static size_t window_lds(int E) {  // k_ccc_dftBC's dynamic LDS: two E x (L / 2 + 1) tables
+    return (size_t)2 * E * (L / 2 + 1) * sizeof(float2);
+}
+template <int L>
+static size_t window_lds_all(int E) {
+    hipFuncAttributes at{};
+    ETTK_HIP(hipFuncGetAttributes(&at, (const void*)k_ccc_dftBC<L>));
+    return at.sharedSizeBytes + window_lds<L>(E);
+}
+size_t fft3_ccc_window_lds(int n, int E) {
+    switch (n) {
+        case 16: return window_lds_all<16>(E);
+        case 32: return window_lds_all<32>(E);
+        case 48: return window_lds_all<48>(E);
+        case 64: return window_lds_all<64>(E);
+        case 96: return window_lds_all<96>(E);
+        case 128: return window_lds_all<128>(E);
+        default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_ccc_window_lds: unsupported size " + std::to_string(n)};
+    }
+}
+
+template <int L>
 static void launch_ccc_tail(const FftTables& T, const CccTailArgs& a, hipStream_t s) {
     constexpr int H = L / 2 + 1;
     const float2 *tw = T.tw.p + T.offset[fft_len_index(L)], *tw2 = T.tw.p + T.offset[fft_len_index(2 * L)];
@@ -1273,7 +1295,7 @@ static void launch_ccc_tail(const FftTables& T, const CccTailArgs& a, hipStream_
     }
     {
         ProfScope ps(T.prof, "k_ccc_dftBC", Gb, s);
-        const size_t shm = (size_t)2 * E * H * sizeof(float2);
+        const size_t shm = window_lds<L>(E);
         ensure_dynamic_lds((const void*)k_ccc_dftBC<L>, shm);
         k_ccc_dftBC<L><<<dim3(E, a.batch), BcShape<L>::THREADS, shm, s>>>(a.G1, a.tabK, a.z, a.bval, a.bidx, tw, tw2);
     }

@@ -194,10 +194,13 @@ static void search_window(ettk_plan* P) {
     P->z.I0 = I0;
     P->z.ub2 = (E - 1) / 2;
     P->z.restr2 = (float)restr * (float)restr;
-    // the windows that an LDS-resident plane with both axes' tables would hold are the supported ones
-    size_t lds_b = (size_t)(N * H + E * N + 2 * E * H) * sizeof(float2) + 2048;
-    ETTK_REQUIRE(lds_b <= 160 * 1024, ETTK_ERR_UNSUPPORTED,
-                 "translation search window too large for the LDS-resident upsampled DFT (reduce trans_restrict)");
+    // The windows the library offers: up to the whole doubled box at 16, 32, 48 and 64, 19.5 voxels at 96 and 11 at 128 (what
+    // a plane with both axes' tables takes of 160 KB; callers rely on wider ones being refused).
+    ETTK_REQUIRE((size_t)(N * H + E * N + 2 * E * H) * sizeof(float2) + 2048 <= kMaxLds, ETTK_ERR_UNSUPPORTED,
+                 "translation search window too large for this box size (reduce trans_restrict)");
+    // and what the kernel that evaluates them needs
+    ETTK_REQUIRE(fft3_ccc_window_lds(N, E) <= kMaxLds, ETTK_ERR_UNSUPPORTED,
+                 "translation search window does not fit a workgroup's LDS (reduce trans_restrict)");
     std::vector<float2> tK((size_t)E * H);
     for (int x = 0; x < E; x++) {
         int u = I0 + x - N;

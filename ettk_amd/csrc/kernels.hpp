@@ -111,6 +111,9 @@ struct CccTailArgs {
     float* out4;                      // [e][4] = distance, shift
 };
 void fft3_ccc_tail(const FftTables& T, const CccTailArgs& a, hipStream_t s);
+// LDS of a workgroup of its window kernel for a window of E points per axis: the kernel's own arrays and what a launch adds
+static constexpr size_t kMaxLds = 160 * 1024;
+size_t fft3_ccc_window_lds(int n, int E);
 
 // reslice (tricubic Keys a=-1/2, clamp border, -FLT_MAX outside): out [e][i][j][k]; `nb` must equal
 // reslice_blocks(N) (one workgroup per 8^3 output tile), partials hold 2 * nb floats per evaluation
