@@ -1579,6 +1579,8 @@ void fft3_c2r_op_r2c(const FftTables& T, const float2* in, float2* io, int n, in
         case 32: launch_c2r_op_r2c<32>(T, in, io, batch, op, aux, partials, s); break;
         case 48: launch_c2r_op_r2c<48>(T, in, io, batch, op, aux, partials, s); break;
         case 64: launch_c2r_op_r2c<64>(T, in, io, batch, op, aux, partials, s); break;
+        case 96: launch_c2r_op_r2c<96>(T, in, io, batch, op, aux, partials, s); break;
+        case 128: launch_c2r_op_r2c<128>(T, in, io, batch, op, aux, partials, s); break;
         default: throw Error{ETTK_ERR_UNSUPPORTED, "fft3_c2r_op_r2c: unsupported size " + std::to_string(n)};
     }
     ETTK_HIP(hipGetLastError());

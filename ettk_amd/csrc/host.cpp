@@ -674,18 +674,9 @@ static void plan_release(ettk_plan* P) {
     if (us) (void)hipStreamDestroy(us);
 }
 
-extern "C" {
-
-const char* ettk_last_error(void) { return g_err.c_str(); }
-
-int ettk_fft3(ettk_ctx* ctx, int n, int batch, int kind, const void* in, void* out, const float* aux) {
-    ETTK_API_BEGIN
-    ETTK_REQUIRE(ctx && in && out && batch > 0, ETTK_ERR_ARG, "ettk_fft3: bad argument");
-    ETTK_REQUIRE(fft_len_index(n) >= 0, ETTK_ERR_UNSUPPORTED, "ettk_fft3: unsupported size " + std::to_string(n));
-    ETTK_REQUIRE(kind >= ETTK_FFT_R2C && kind <= ETTK_FFT_SQUARE, ETTK_ERR_ARG, "ettk_fft3: unknown kind");
-    ETTK_REQUIRE(kind < ETTK_FFT_MASK || n <= 64, ETTK_ERR_UNSUPPORTED,
-                 "ettk_fft3: the fused transforms need n <= 64");
-    ETTK_REQUIRE(kind != ETTK_FFT_MASK || aux, ETTK_ERR_ARG, "ettk_fft3: ETTK_FFT_MASK needs the mask");
+namespace ettk {
+// ettk_fft3 behind its checks, with the fused transforms at every size that the CCC runs them at (n <= 128)
+void fft3_run(ettk_ctx* ctx, int n, int batch, int kind, const void* in, void* out, const float* aux) {
     ETTK_HIP(hipSetDevice(ctx->device));
     hipStream_t s = ctx->stream;
     const size_t nh = (size_t)n * n * (n / 2 + 1);
@@ -712,6 +703,22 @@ int ettk_fft3(ettk_ctx* ctx, int n, int batch, int kind, const void* in, void* o
             break;
     }
     ETTK_HIP(hipStreamSynchronize(s));
+}
+}  // namespace ettk
+
+extern "C" {
+
+const char* ettk_last_error(void) { return g_err.c_str(); }
+
+int ettk_fft3(ettk_ctx* ctx, int n, int batch, int kind, const void* in, void* out, const float* aux) {
+    ETTK_API_BEGIN
+    ETTK_REQUIRE(ctx && in && out && batch > 0, ETTK_ERR_ARG, "ettk_fft3: bad argument");
+    ETTK_REQUIRE(fft_len_index(n) >= 0, ETTK_ERR_UNSUPPORTED, "ettk_fft3: unsupported size " + std::to_string(n));
+    ETTK_REQUIRE(kind >= ETTK_FFT_R2C && kind <= ETTK_FFT_SQUARE, ETTK_ERR_ARG, "ettk_fft3: unknown kind");
+    ETTK_REQUIRE(kind < ETTK_FFT_MASK || n <= 64, ETTK_ERR_UNSUPPORTED,
+                 "ettk_fft3: the fused transforms are offered for n <= 64");
+    ETTK_REQUIRE(kind != ETTK_FFT_MASK || aux, ETTK_ERR_ARG, "ettk_fft3: ETTK_FFT_MASK needs the mask");
+    fft3_run(ctx, n, batch, kind, in, out, aux);
     ETTK_API_END
 }
 
