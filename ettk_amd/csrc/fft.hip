@@ -1146,7 +1146,16 @@ __global__ void __launch_bounds__(64) k_peak_final(const float* __restrict__ bes
 }
 
 // ------------------------------------------------------------------ host launchers
-// profile record names: k_r2c_rows<L>, k_fft_strided<L>, k_c2r_rows<L>
+// Which form a strided pass takes.  In registers it is faster at every length: over 0.5 GB at 16, 32, 48, 64, 96 and 128,
+// 6.1, 6.7, 6.2, 6.5, 6.2 and 6.6 TB/s against 5.7, 6.0, 3.8, 6.3, 3.9 and 6.3 staged in LDS.  Up to 64 it stays staged for
+// its rounding, not its accuracy: the 20 steps of the refinement amplify a last bit of these spectra to 1e-2 of a pose,
+// and poses at 48 and 64 are kept as earlier versions gave them.
+template <int L>
+static constexpr bool staged_pencils() {
+    return L <= 64;
+}
+
+// profile record names: k_r2c_rows<L>, the strided pass that runs (k_fft_strided<L> or k_fft_col<L>), k_c2r_rows<L>
 template <int L>
 static const char* plane_name(int which) {
     static const std::string n[2] = {"k_r2c_plane<" + std::to_string(L) + ">", "k_c2r_plane<" + std::to_string(L) + ">"};
@@ -1154,14 +1163,15 @@ static const char* plane_name(int which) {
 }
 template <int L>
 static const char* prof_name(int which) {
-    static const std::string n[3] = {"k_r2c_rows<" + std::to_string(L) + ">", "k_fft_strided<" + std::to_string(L) + ">",
+    static const std::string n[3] = {"k_r2c_rows<" + std::to_string(L) + ">",
+                                     (staged_pencils<L>() ? "k_fft_strided<" : "k_fft_col<") + std::to_string(L) + ">",
                                      "k_c2r_rows<" + std::to_string(L) + ">"};
     return n[which].c_str();
 }
 
 template <int L>
 static void launch_strided(const StridedArgs& a, const float2* tw, hipStream_t s) {
-    if constexpr (L <= 64) {
+    if constexpr (staged_pencils<L>()) {
         using S = StridedShape<L>;
         k_fft_strided<L><<<(unsigned)((a.npencils + S::P - 1) / S::P), S::THREADS, 0, s>>>(a, tw);
     } else {

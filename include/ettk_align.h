@@ -327,7 +327,7 @@ int ettk_extract_batch(ettk_ctx* ctx, const float* d_tomogram, int nx, int ny, i
 
 /* Measurement hooks (no reference counterpart).  ettk_profile(ctx, 1) resets and enables per-kernel HIP-event
    timing on the context's stream; ettk_profile_query returns, for one kernel name (e.g. "k_fft_strided<64>",
-   "k_reslice", "k_combine_dftA"), the summed launch time in ms, the launch count and the algorithmic bytes
+   "k_reslice", "k_ccc_combine"), the summed launch time in ms, the launch count and the algorithmic bytes
    those launches move (one read of every input and one write of every output). */
 int ettk_profile(ettk_ctx* ctx, int enable);
 int ettk_profile_query(ettk_ctx* ctx, const char* kernel, double* total_ms, long long* launches, double* bytes);
