@@ -22,23 +22,6 @@ namespace ettk {
 
 static constexpr int kThreads = 256;
 
-__device__ __forceinline__ float wave_sum(float v) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    return v;
-}
-// block sum (result valid in thread 0)
-__device__ __forceinline__ float block_sum(float v, float* sh) {
-    v = wave_sum(v);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) sh[w] = v;
-    __syncthreads();
-    float r = 0.f;
-    if (threadIdx.x == 0)
-        for (int i = 0; i < (int)(blockDim.x + 63) / 64; i++) r += sh[i];
-    __syncthreads();
-    return r;
-}
-
 // ------------------------------------------------------------------ reslice
 // Validity of a sample is decided in FP32 unless it lies within 1e-3 of the border, where the FP64 map decides
 // (the reference places samples in FP64: a sample that FP32 rounding moves across the border would otherwise

@@ -339,7 +339,6 @@ void fft_tables_init(FftTables& T, hipStream_t s);
 // The r2c load applies an element-wise prologue selected by `pro`.
 enum Prologue : int {
     PRO_NONE = 0,        // x
-    PRO_SQUARE_SHIFT,    // x*x*(-1)^(i+j+k)
     PRO_MASK_SHIFT,      // x*aux0[i,j,k]*(-1)^(i+j+k)
     PRO_RESLICED,        // valid(x) ? (x - mean_b) * aux0 * (-1)^(i+j+k) : 0   (mean from stats[b])
     PRO_SHIFT,           // x*(-1)^(i+j+k)

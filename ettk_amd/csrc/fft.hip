@@ -209,26 +209,6 @@ __device__ __forceinline__ void pencil_fft(float2* pen, int lane, const float2* 
 
 // ------------------------------------------------------------------ r2c, pass along k (real rows)
 template <int L>
-__device__ __forceinline__ float r2c_load(const R2CArgs& a, long row, int k) {
-    long ij = row % ((long)L * L);
-    int i = (int)(ij / L), j = (int)(ij % L);
-    float sg = ((i + j + k) & 1) ? -1.0f : 1.0f;
-    float x = a.in[row * L + k];
-    if (a.pro == PRO_NONE) return x;
-    switch (a.pro) {
-        case PRO_SQUARE_SHIFT: return x * x * sg;
-        case PRO_SHIFT: return x * sg;
-        case PRO_MASK_SHIFT: return x * a.aux0[ij * L + k] * sg;
-        case PRO_RESLICED: {
-            if (x == -3.402823466e+38f) return 0.0f;  // outside the particle box: -FLT_MAX background
-            long b = row / ((long)L * L);
-            return (x - a.stats[b]) * (a.aux0 ? a.aux0[ij * L + k] : 1.0f) * sg;
-        }
-    }
-    return x;
-}
-
-template <int L>
 __global__ void __launch_bounds__(Shape<L>::THREADS) k_r2c_rows(R2CArgs a, const float2* __restrict__ twg) {
     using S = Shape<L>;
     constexpr int H = L / 2 + 1;
@@ -244,7 +224,7 @@ __global__ void __launch_bounds__(Shape<L>::THREADS) k_r2c_rows(R2CArgs a, const
         float x = 0.0f;
         if (pair < npairs) {
             long row = pair * 2 + r / L;
-            x = r2c_load<L>(a, row, r % L);
+            x = a.in[row * L + r % L];
         }
         float* f = reinterpret_cast<float*>(&lds[q * S::LD + (r % L)]);
         f[r / L] = x;
@@ -616,7 +596,6 @@ __device__ __forceinline__ void r2c_stage_plane(const R2CArgs& a, int pi, const 
             const float sg = ((pi + j + x) & 1) ? -1.0f : 1.0f;
             float r;
             if constexpr (PRO == PRO_NONE) r = v.x;
-            else if constexpr (PRO == PRO_SQUARE_SHIFT) r = v.x * v.x * sg;
             else if constexpr (PRO == PRO_SHIFT) r = v.x * sg;
             else if constexpr (PRO == PRO_MASK_SHIFT) r = v.x * v.y * sg;
             else r = (v.x == -3.402823466e+38f) ? 0.0f : (v.x - mean) * v.y * sg;  // PRO_RESLICED
@@ -638,7 +617,6 @@ __global__ void __launch_bounds__(Plane<L>::THREADS) k_r2c_plane(R2CArgs a, cons
     const float2 twv = twg[threadIdx.x % L];  // stored after the staging loads are in flight
     switch (a.pro) {
         case PRO_NONE: r2c_stage_plane<L, PRO_NONE, false>(a, pi, src, mean, buf); break;
-        case PRO_SQUARE_SHIFT: r2c_stage_plane<L, PRO_SQUARE_SHIFT, false>(a, pi, src, mean, buf); break;
         case PRO_SHIFT: r2c_stage_plane<L, PRO_SHIFT, false>(a, pi, src, mean, buf); break;
         case PRO_MASK_SHIFT: r2c_stage_plane<L, PRO_MASK_SHIFT, true>(a, pi, src, mean, buf); break;
         case PRO_RESLICED:
@@ -1195,7 +1173,8 @@ static void launch_r2c(const FftTables& T, const R2CArgs& a, float2* scratch, hi
         ProfScope ps(T.prof, plane_name<L>(0), vol_r + vol_c, s);
         k_r2c_plane<L><<<(unsigned)((long)a.batch * L), Plane<L>::THREADS, 0, s>>>(a, tw);
     } else {
-        // pass k: real rows -> a.out (half rows)
+        // pass k: real rows -> a.out (half rows); only ettk_fft3 transforms such boxes, without a prologue
+        ETTK_REQUIRE(a.pro == PRO_NONE, ETTK_ERR_UNSUPPORTED, "fft3_r2c: prologues are for n <= 128");
         {
             ProfScope ps(T.prof, prof_name<L>(0), vol_r + vol_c, s);
             k_r2c_rows<L><<<(unsigned)((npairs + S::P - 1) / S::P), S::THREADS, 0, s>>>(a, tw);

@@ -114,7 +114,7 @@ template <int R, bool INV> __device__ __forceinline__ float2 mul_root(float2 z, 
 // DFTs of R points in registers, natural order in and out
 template <int R, bool INV> struct Dft {
     // R = A B: B DFTs of A points over the elements b, b + B, ..., then A DFTs of B points
-    static constexpr int A = R == 6 ? 2 : R == 24 ? 8 : 4, B = R / A;
+    static constexpr int A = R == 24 ? 8 : 4, B = R / A;
     static __device__ __forceinline__ void run(float2* x) {
         float2 y[R];
 #pragma unroll
@@ -133,9 +133,6 @@ template <int R, bool INV> struct Dft {
             for (int q = 0; q < B; q++) x[k + A * q] = y[k * B + q];
         }
     }
-};
-template <bool INV> struct Dft<2, INV> {
-    static __device__ __forceinline__ void run(float2* x) { butterfly<2>(x, INV); }
 };
 template <bool INV> struct Dft<3, INV> {
     static __device__ __forceinline__ void run(float2* x) { butterfly<3>(x, INV); }

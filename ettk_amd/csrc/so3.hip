@@ -28,8 +28,6 @@ static inline bool fused_synthesis(int B) { return B == 8 || B == 16 || B == 32;
 static inline bool mfma_synthesis(int B) { return B == 16 || B == 32; }
 
 // ============================================================== tables (host, FP64)
-static double lfact(int n) { return std::lgamma((double)n + 1.0); }
-
 static void legendre_host(int B, double theta, std::vector<double>& P) {
     P.assign((size_t)B * B, 0.0);
     double x = std::cos(theta), s = std::sin(theta);
