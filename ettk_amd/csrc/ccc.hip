@@ -1,13 +1,11 @@
-// ccc.hip -- kernels of the wedge-constrained FFT cross-correlation (gfx950).
+// ccc.hip -- the reslice, the wedges and the set-up kernels of the wedge-constrained FFT cross-correlation (gfx950).
 //
 // Device side of nbfFourierImageMetric::executeFourierNewHalf (inc/em/nbfFourierImageMetric.h:1078-1323)
 // for a batch of (particle, transform) evaluations:
-//   reslice  -> nbfWedgedSubImage3D::getImage (inc/em/nbfWedgedSubImage3D.h:603-828), VTK tricubic
-//   (the spectral weighting and the transforms around it are in fft.hip)
-//   combine  -> the quadratic expression of FIM.h:1202-1203
-//   dftA/BC  -> the zero-padded (2N)^3 c2r of FIM.h:1209-1214 evaluated only on the search window
-//               (FIM.h:1222-1247) as three separable partial DFTs, followed by the spherical mask and the
-//               first-maximum search of locateMaxima (nbfCorrelationImageMetric.h:304-323)
+//   reslice -> nbfWedgedSubImage3D::getImage (inc/em/nbfWedgedSubImage3D.h:603-828), VTK tricubic
+//   wedge overlap -> nbfCorrelationImageMetric::getWedgeOverlap (nbfCorrelationImageMetric.h:533-566)
+// The transforms, the spectral weighting, the quadratic expression (FIM.h:1202-1203), the upsampled correlation on the
+// search window (FIM.h:1209-1247) and its first maximum (nbfCorrelationImageMetric.h:304-323) are in fft.hip.
 // Per-evaluation sums are written as per-block partials and reduced in a fixed order (deterministic).
 #include "kernels.hpp"
 

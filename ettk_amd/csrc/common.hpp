@@ -336,7 +336,7 @@ void fft_tables_init(FftTables& T, hipStream_t s);
 //   r2c: real n^3 -> half n x n x (n/2+1) complex, forward (e^{-i})
 //   c2r: half -> real, backward (e^{+i}), unnormalised; transforms along i and j first, then the
 //        half-complex transform along k (real part of the k=0 and k=n/2 terms)
-// The r2c load applies an element-wise prologue selected by `pro`.
+// The r2c load applies an element-wise prologue selected by `pro` (n <= 128; larger boxes take PRO_NONE).
 enum Prologue : int {
     PRO_NONE = 0,        // x
     PRO_MASK_SHIFT,      // x*aux0[i,j,k]*(-1)^(i+j+k)

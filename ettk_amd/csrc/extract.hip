@@ -20,8 +20,9 @@ constexpr int kExT = kTriThreads;
 
 // One workgroup per 8x8x8 tile of an output box, interpolated from the LDS-staged box of the tomogram its stencils
 // touch (tricubic.hpp); tiles at the far sides of a box whose size is not a multiple of 8 are partial.  Per-tile
-// (sum, count) of the valid samples.  Bound by the LDS reads of the taps, as the CCC reslice.  The call on 60 boxes of
-// 64^3 takes 201 us; with every tap read from global memory it took 1558 us.
+// (sum, count) of the valid samples (the sum in FP32: two samples per thread, then a tree; the tiles in FP64).  Bound by the
+// LDS reads of the taps, as the CCC reslice.  The call on 60 boxes of 64^3 takes 201 us; with every tap read from global
+// memory it took 1558 us.
 __global__ void __launch_bounds__(kExT, 7) k_extract(const float* __restrict__ tomo, int nx, int ny, int nz,
                                                   const ExtractGeom* __restrict__ geom, int N, float* __restrict__ out,
                                                   float* __restrict__ partials) {

@@ -49,7 +49,7 @@ struct EvalGeom {
 // The CCC steps between the particle's r2c plane passes and the fused plane kernels, on pencils along i
 // (n <= 128): S2 holds the plane-pass output of the resliced particles and receives the
 // filtered particle spectra X2; S3 receives X2 and S1 the filtered reference spectrum X1, both inverse-transformed
-// along i (the inputs of fft3_op_r2c_after_ipass).  Partials: fft3_ccc_ipass_blocks(n) per evaluation.
+// along i (the inputs of fft3_ccc_tail).  Partials: fft3_ccc_ipass_blocks(n) per evaluation.
 struct CccIpassArgs {
     float2* S2;
     float2* S3;

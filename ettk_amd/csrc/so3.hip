@@ -225,9 +225,9 @@ __global__ void __launch_bounds__(64) k_proj_final(const float* __restrict__ R, 
     }
 }
 
-// full-size magnitude volume (rows of M/2 + 2 stored, fft3_pad_magnitude) as ProjRot.h:327-338 leaves it: A(i,j,k) for k <= M/2 is |F| except the i = 0
-// plane (0); for k > M/2: i = 0 -> 0, j = 0 -> the pad constant (the loop never overwrites those voxels of
-// the padded image), otherwise the mirrored value |F|(M-i, M-j, M-k)
+// full-size magnitude volume (rows of M/2 + 2 stored, fft3_pad_magnitude) as ProjRot.h:327-338 leaves it: A(i,j,k) for
+// k <= M/2 is |F| except the i = 0 plane (0); for k > M/2: i = 0 -> 0, j = 0 -> the pad constant (the loop never
+// overwrites those voxels of the padded image), otherwise the mirrored value |F|(M-i, M-j, M-k)
 __device__ __forceinline__ float mag_at(const float* __restrict__ mag, int M, int i, int j, int k, float padc) {
     const int Hm = M / 2 + 2;
     if (i == 0) return 0.f;

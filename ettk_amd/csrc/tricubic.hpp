@@ -10,9 +10,10 @@
 // box and, with the row and plane strides 17 and 300, fall on fewer common LDS banks than those of an 8x8 plane.  A
 // 17^3 box at these strides (20 KB) lets 7 workgroups share a CU.
 //
-// Bound by LDS and VALU together (both 83% busy; the taps' words collide on banks 2.9 times in half a wavefront), so the
-// rest of a tile is kept cheap: the box's bounds and the staging's plane addresses are scalar, tiles away from the
-// volume's border test no sample, the box has a margin instead of a clamp per sample, counts are ballots and sums DPP.
+// Bound by LDS and VALU together (the LDS is busy for 87% of the kernel, 48% of that with bank conflicts, and the SIMDs
+// issue for 89%, at four cycles an instruction), so the rest of a tile is kept cheap: the box's bounds and the staging's
+// plane addresses are scalar, tiles away from the volume's border test no sample, the box has a margin instead of a clamp
+// per sample, counts are ballots and sums DPP.
 // 240 evaluations at 64^3: 605 us, 686 before; extraction of 60 boxes 157 against 176 us.  Layouts that trade bank
 // conflicts for address arithmetic are slower: voxel (x, y, z) on bank (x & 3) + 4 (y & 3) + 16 (z & 1) with the taps
 // visited in a lane's own conflict-free order 675 us (VALU-bound, 1.5 times the instructions), without the z digit 721;
