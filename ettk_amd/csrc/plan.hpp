@@ -95,6 +95,7 @@ struct CccGraph {
 struct ExtractGeom {
     float m[12];    // input index = m[0..2] x + m[3..5] y + m[6..8] z + m[9..11]  (rows x, y, z)
     double md[12];  // the same map in FP64: decides validity for samples within FP32 rounding of the border
+    int steep;      // which form of k_extract cuts it
 };
 struct Timing {
     double ccc_ms = 0, total_ms = 0;
