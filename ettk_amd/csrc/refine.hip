@@ -171,10 +171,9 @@ __device__ __forceinline__ float trilin_box(const float* box, const int lo[3], c
 // 1420 us; split like this the score and gradient of those particles went from 1092 to 690 us and from 2767 to
 // 1334 us.  The 16-byte loads need 4-byte alignment only.
 static constexpr int kMeanU = 8, kMeanV = kT * 4 * kMeanU;
-__global__ void __launch_bounds__(kT) k_vol_sum(const float* __restrict__ vols, long n3, double* __restrict__ part) {
-    __shared__ double sh[kT / 64];
-    const float* v = vols + (size_t)blockIdx.y * n3;
-    const long o0 = (long)blockIdx.x * kMeanV + threadIdx.x * 4;
+// sum of the kMeanV voxels from `first` on over kT threads (t = 0 .. kT - 1), in thread 0; `sh` holds kT / 64 doubles
+__device__ __forceinline__ double mean_part(const float* __restrict__ v, long first, long n3, int t, double* sh) {
+    const long o0 = first + t * 4;
     float4 r[kMeanU];  // all loads in flight; n3 is a multiple of 4 (box sizes are multiples of 8)
 #pragma unroll
     for (int u = 0; u < kMeanU; u++) {
@@ -186,12 +185,32 @@ __global__ void __launch_bounds__(kT) k_vol_sum(const float* __restrict__ vols, 
 #pragma unroll
     for (int u = 0; u < kMeanU; u++) s += ((double)r[u].x + r[u].y) + ((double)r[u].z + r[u].w);
     s = dsum64(s);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    if ((t & 63) == 0) sh[t >> 6] = s;
+    __syncthreads();
+    double sum = 0.0;
+    if (t == 0)
+        for (int w = 0; w < kT / 64; w++) sum += sh[w];
+    return sum;
+}
+__global__ void __launch_bounds__(kT) k_vol_sum(const float* __restrict__ vols, long n3, double* __restrict__ part) {
+    __shared__ double sh[kT / 64];
+    const double t = mean_part(vols + (size_t)blockIdx.y * n3, (long)blockIdx.x * kMeanV, n3, threadIdx.x, sh);
+    if (threadIdx.x == 0) part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = t;
+}
+// Volumes of at most four parts (boxes of 16 and 32): one workgroup holds them all, and the sums, added in the order of
+// k_vol_mean, need no second launch.  Score and gradient of one particle of 32^3: 101 us, 104 with two launches.
+template <int NB>
+__global__ void __launch_bounds__(kT * NB) k_vol_mean_small(const float* __restrict__ vols, long n3, float* __restrict__ mean) {
+    __shared__ double sh[NB][kT / 64];
+    __shared__ double part[NB];
+    const int b = threadIdx.x / kT, t = threadIdx.x % kT;
+    const double sum = mean_part(vols + (size_t)blockIdx.x * n3, (long)b * kMeanV, n3, t, sh[b]);
+    if (t == 0) part[b] = sum;
     __syncthreads();
     if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int w = 0; w < kT / 64; w++) t += sh[w];
-        part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = t;
+        double s = part[0];
+        if constexpr (NB == 4) s = (part[0] + part[2]) + (part[1] + part[3]);
+        mean[blockIdx.x] = (float)(s / (double)n3);
     }
 }
 __global__ void __launch_bounds__(64) k_vol_mean(const double* __restrict__ part, int nb, long n3,
@@ -330,6 +349,12 @@ void launch_vol_mean(const float* vols, int count, int N, double* part, float* m
     ETTK_REQUIRE(N % 4 == 0, ETTK_ERR_ARG, "launch_vol_mean: box size must be a multiple of 4");
     const long n3 = (long)N * N * N;
     const int nb = vol_mean_blocks(N);
+    if (nb <= 4) {
+        if (nb == 1) k_vol_mean_small<1><<<count, kT, 0, s>>>(vols, n3, mean);
+        else k_vol_mean_small<4><<<count, kT * 4, 0, s>>>(vols, n3, mean);
+        ETTK_HIP(hipGetLastError());
+        return;
+    }
     // the particles run along the grid's second axis, at most 65535 per launch
     for (int c0 = 0; c0 < count; c0 += 65535) {
         const int c = std::min(65535, count - c0);
